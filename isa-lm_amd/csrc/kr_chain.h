@@ -16,7 +16,7 @@
 // stayed inside). In bits: a run maps a start s to s + d[s & 1], where d[0]
 // and d[1] come from running it from one even start and the odd start above.
 //
-// The terms are split into chunks (128 terms, at most 128 chunks). For
+// The terms are split into chunks (128 terms, a lane pair each). For
 // each chunk a pair of lanes runs the chain from an even and an odd start in
 // the binade where the prefix before the chunk lies (estimated by fp32
 // partial sums: only its binade matters), checking every SC_BLK terms
@@ -43,14 +43,16 @@
 namespace {
 
 constexpr int SC_LOG_LMIN = 7;                // chunks of 128 terms, doubled while more than SC_MAXC
-constexpr int SC_MAXC = 128;
+constexpr int SC_MAXC = 256;
 constexpr int SC_PAD = 4;                     // floats after each chunk's terms (spreads LDS banks)
 constexpr int SC_BLK = 16;                    // terms between binade checks
 constexpr int SC_MAXNB = 8;                   // blocks per chunk, at most
 constexpr int SC_NSEG = SC_MAXNB / 2;         // runs of unbroken blocks in a chunk, at most
 constexpr int SC_CPW = 32;                    // chunks per wave: one lane pair each
 constexpr int SC_REC = 1 + 3 * SC_NSEG;       // ints of walk record per chunk
-constexpr int SC_MAX_N = SC_MAXC * SC_MAXNB * SC_BLK;
+constexpr int SC_LMAX = SC_MAXNB * SC_BLK;                            // terms of a chunk, at most
+constexpr int SC_MAX_N = 4 * SC_CPW * SC_LMAX;                        // terms 4 waves sum
+constexpr int SC_MAX_N8 = 8 * SC_CPW * SC_LMAX;                       // terms 8 waves or more sum
 
 // log2 of the chunk length for n terms
 __host__ __device__ constexpr int sc_log_len(int n) {
@@ -188,7 +190,8 @@ __device__ __forceinline__ unsigned sc_rest(const float *t, int sh, int c, int m
     return sv;
 }
 
-// The ordered sum s0 + t[0] + ... + t[n-1] (n <= SC_MAX_N) by all NT threads
+// The ordered sum s0 + t[0] + ... + t[n-1] (n <= SC_MAX_N; SC_MAX_N8 from
+// NT = 512 on) by all NT threads
 // of the workgroup; every thread gets the result. Term i sits at
 // t[sc_at(i, sc_log_len(n))] in LDS (16-byte aligned, sc_terms_cap(n)
 // floats: the last chunk's tail is zero-filled here, and s + 0 == s for
@@ -207,7 +210,7 @@ template <int NT, bool REC = false, bool WAVE = false, bool LEAN = false>
 __device__ __forceinline__ float kr_spec_sum(float *t, int n, unsigned char *lds, float s0 = 0.0f,
                                              unsigned *cst = nullptr) {
     constexpr int NW = NT / 64;
-    static_assert(WAVE ? NT == 64 : NW * SC_CPW >= SC_MAXC, "every chunk needs a lane pair");
+    static_assert(WAVE ? NT == 64 : NW * SC_CPW * SC_LMAX >= SC_MAX_N, "every chunk needs a lane pair");
     const int tid = WAVE ? (int)(threadIdx.x & 63) : (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int sh = sc_log_len(n), L = 1 << sh, NB = L / SC_BLK;
     const int C = (n + L - 1) >> sh, NA = (C + SC_CPW - 1) / SC_CPW;   // waves with chunks

@@ -20,7 +20,7 @@ struct krh_sampler_dev {
     unsigned long long *rng;   // xorshift64* state
     int *ring;                 // [2 + R]: n_recent, recent_at, then the ids
     int *first;                // [vocab]: the penalty's first ring slot per id
-    float *probs;              // [vocab]
+    float *probs;              // [vocab]: the softmax's numerators (sm_prob scales them)
     unsigned *keys;            // [2][vocab]: sort keys, two buffers
     int *ids;                  // [2][vocab]
     int *hist;                 // [blocks][256]: digit counts per sort workgroup
@@ -37,7 +37,13 @@ struct krh_sampler {
 namespace {
 
 constexpr int SM_NT = 1024;                                       // threads of the one-workgroup kernels
-constexpr int SM_G = 12288;                                       // terms per ordered-sum group (in LDS)
+// Terms per ordered-sum group (in LDS: 152 of the CU's 160 KB with the sum's
+// scratch; one workgroup runs these kernels). A group costs about 6 us whatever
+// its length, so the fewer the better: with 12,288 terms the 128k vocabulary's
+// softmax took 11 groups and a nucleus of 26k candidates 3 (a top-p draw over
+// 128,256 ids, with the scaling pass gone and the sort's empty workgroups
+// returning at once: 181 -> 125 us).
+constexpr int SM_G = 32768;
 constexpr int SM_RT = 256, SM_ROWS = 4, SM_E = SM_RT * SM_ROWS;   // radix sort: threads, rows, ids per workgroup
 constexpr int SM_HB = 16;                                         // digit counts read at a time
 constexpr int SM_EB = 2048;                                       // ids per elementwise workgroup (256 x 8)
@@ -46,12 +52,12 @@ constexpr int SM_SCR = (sc_lds_bytes(SM_G, SM_NT) + 15) & ~15;
 constexpr int SM_CST = (sc_chunks(SM_G) + 1) * 4;
 constexpr int SM_LDS = SM_TERMS + SM_SCR + SM_CST + 16;
 static_assert(SM_G % SM_NT == 0, "a thread keeps its ids across the softmax's passes");
-static_assert(SM_LDS <= 64 * 1024, "LDS");
+static_assert(SM_LDS <= 160 * 1024 - 1024 && SM_G <= SC_MAX_N8, "LDS");
 
 enum { SM_GREEDY = 0, SM_MULT = 1, SM_TOPK = 2, SM_TOPP = 3 };
 // meta: candidates after the sort's first pass, the coin's bits, whether the
-// id is already decided (NaN probabilities), and that id
-enum { MT_M = 0, MT_COIN = 1, MT_DONE = 2, MT_ID = 3, MT_KIND = 4 };
+// id is already decided (NaN probabilities), that id, and 1 / the softmax's sum
+enum { MT_M = 0, MT_COIN = 1, MT_DONE = 2, MT_ID = 3, MT_KIND = 4, MT_INV = 5 };
 // the softmax's case, from the maxima: numerators expf(p - max), all -inf
 // (uniform 1/n), or a NaN term (every probability NaN)
 enum { SK_EXP = 0, SK_UNIFORM = 1, SK_NAN = 2 };
@@ -77,10 +83,10 @@ __device__ __forceinline__ void sm_take(float &bv, int &bi, float v, int i) {
         bi = i;
     }
 }
-__device__ int sm_argmax(const float *v, int n, float *rv, int *ri) {
+template <class Val> __device__ int sm_argmax(Val v, int n, float *rv, int *ri) {
     float bv = -INFINITY;
     int bi = INT_MAX;
-    for (int i = sm_tid(); i < n; i += SM_NT) sm_take(bv, bi, v[i], i);
+    for (int i = sm_tid(); i < n; i += SM_NT) sm_take(bv, bi, v(i), i);
     for (int o = 32; o >= 1; o >>= 1) sm_take(bv, bi, __shfl_xor(bv, o), __shfl_xor(bi, o));
     if ((sm_tid() & 63) == 0) {
         rv[sm_tid() >> 6] = bv;
@@ -91,7 +97,7 @@ __device__ int sm_argmax(const float *v, int n, float *rv, int *ri) {
     bi = ri[0];
     for (int w = 1; w < SM_NT / 64; w++) sm_take(bv, bi, rv[w], ri[w]);
     __syncthreads();
-    return (bi == INT_MAX || v[0] != v[0]) ? 0 : bi;
+    return (bi == INT_MAX || v(0) != v(0)) ? 0 : bi;
 }
 
 // model/sampler.c:39-48: every distinct id of the ring that is below n, once
@@ -148,6 +154,25 @@ __device__ float sm_coin(unsigned long long *st) {
     return kr_fdiv((float)(hi >> 8), 16777216.0f);
 }
 
+// a probability from its numerator: x * (1 / sum), formed where it is read
+// (k_smp_main alone would pass over the vocabulary once more)
+__device__ __forceinline__ float sm_prob(float x, float inv) { return kr_fmul(x, inv); }
+
+// ng terms from term(g0) into LDS in the ordered sum's layout; each thread's
+// reads SM_FB at a time, all issued before the first store
+constexpr int SM_FB = 16;
+template <class Term>
+__device__ __forceinline__ void sm_fill(float *t, Term term, int g0, int ng, int sh) {
+    for (int i0 = sm_tid(); i0 < ng; i0 += SM_FB * SM_NT) {
+        float v[SM_FB];
+#pragma unroll
+        for (int k = 0; k < SM_FB; k++) v[k] = term(g0 + min(i0 + k * SM_NT, ng - 1));
+#pragma unroll
+        for (int k = 0; k < SM_FB; k++)
+            if (i0 + k * SM_NT < ng) t[sc_at(i0 + k * SM_NT, sh)] = v[k];
+    }
+}
+
 // The first i < m with thr < term(0) + ... + term(i), the sum formed one add
 // at a time from +0 (model/sampler.c:63-70, :113-128, :140-151); -1 when none.
 // val: that partial sum, or the whole sum. SM_G terms at a time go to LDS;
@@ -165,7 +190,7 @@ __device__ int sm_first_above(Term term, int m, float thr, unsigned char *lds, f
     float S = 0.0f;
     for (int g0 = 0; g0 < m; g0 += SM_G) {
         const int ng = min(SM_G, m - g0), sh = sc_log_len(ng), C = sc_chunks(ng), L = 1 << sh;
-        for (int i = tid; i < ng; i += SM_NT) t[sc_at(i, sh)] = term(g0 + i);
+        sm_fill(t, term, g0, ng, sh);
         __syncthreads();
         const float E = kr_spec_sum<SM_NT, true>(t, ng, scr, S, cst);
         if (thr < E) {
@@ -278,7 +303,7 @@ __global__ void __launch_bounds__(256) k_smp_exp(int n, int nblk, Dev d) {
 // draws it leaves the probabilities and the coin for the kernels after it.
 template <int MODE>
 __global__ void __launch_bounds__(SM_NT) k_smp_main(int *tok, int n, Dev d, int *pos, int *log) {
-    extern __shared__ __align__(16) unsigned char sm_lds[];
+    __shared__ __align__(16) unsigned char sm_lds[SM_LDS];
     __shared__ float scoin;
     const int tid = sm_tid();
     {
@@ -288,17 +313,17 @@ __global__ void __launch_bounds__(SM_NT) k_smp_main(int *tok, int n, Dev d, int 
         // keeps no candidate (the argmax of all-NaN: 0), and top-k keeps the
         // first k ids in id order (the last of them)
         const int decided = kind != SK_NAN ? -1 : MODE == SM_MULT ? n - 1 : MODE == SM_TOPK ? d.topk - 1 : 0;
+        float inv = 1.0f;   // uniform: the values are the probabilities (x * 1 is x)
         if (kind == SK_EXP) {
             float *t = (float *)sm_lds;
             float S = 0.0f;
             for (int g0 = 0; g0 < n; g0 += SM_G) {
                 const int ng = min(SM_G, n - g0), sh = sc_log_len(ng);
-                for (int i = tid; i < ng; i += SM_NT) t[sc_at(i, sh)] = p[g0 + i];
+                sm_fill(t, [&](int i) { return p[i]; }, g0, ng, sh);
                 __syncthreads();
                 S = kr_spec_sum<SM_NT>(t, ng, sm_lds + SM_TERMS, S);
             }
-            const float inv = kr_fdiv(1.0f, S);
-            for (int i = tid; i < n; i += SM_NT) p[i] = kr_fmul(p[i], inv);
+            inv = kr_fdiv(1.0f, S);
         }
         if (tid == 0) scoin = sm_coin(d.rng);
         __syncthreads();
@@ -307,7 +332,7 @@ __global__ void __launch_bounds__(SM_NT) k_smp_main(int *tok, int n, Dev d, int 
             int t = decided;
             if (t < 0) {
                 float v;
-                const int j = sm_first_above([&](int i) { return p[i]; }, n, coin, sm_lds, v);
+                const int j = sm_first_above([&](int i) { return sm_prob(p[i], inv); }, n, coin, sm_lds, v);
                 t = j >= 0 ? j : n - 1;
             }
             if (tid == 0) sm_finish(t, tok, pos, log, d);
@@ -316,6 +341,7 @@ __global__ void __launch_bounds__(SM_NT) k_smp_main(int *tok, int n, Dev d, int 
                 d.meta[MT_COIN] = __float_as_int(coin);
                 d.meta[MT_DONE] = decided >= 0;
                 d.meta[MT_ID] = decided;
+                d.meta[MT_INV] = __float_as_int(inv);
             }
         }
     }
@@ -330,14 +356,14 @@ __global__ void __launch_bounds__(SM_NT) k_smp_main(int *tok, int n, Dev d, int 
 // in id order; the passes alternate between the two key buffers and end in
 // the second. Each workgroup takes SM_E ids as SM_ROWS rows of SM_RT.
 template <int P>
-__device__ __forceinline__ void sm_in(const Dev &d, int i, int m, float cutoff, int filt, unsigned &key, int &id,
-                                      bool &keep) {
+__device__ __forceinline__ void sm_in(const Dev &d, int i, int m, float inv, float cutoff, int filt, unsigned &key,
+                                      int &id, bool &keep) {
     keep = i < m;
     key = 0;
     id = 0;
     if (!keep) return;
     if constexpr (P == 0) {
-        const float p = d.probs[i];
+        const float p = sm_prob(d.probs[i], inv);
         keep = !filt || p >= cutoff;
         key = ~__float_as_uint(p);
         id = i;
@@ -353,14 +379,16 @@ __global__ void __launch_bounds__(SM_RT) k_smp_hist(Dev d, int n, float cutoff, 
     __shared__ int cnt[256];
     if (d.meta[MT_DONE]) return;
     const int tid = sm_tid();
+    const int m = P == 0 ? n : d.meta[MT_M];
+    if ((int)blockIdx.x * SM_E >= m) return;   // no ids left for this workgroup: its counts are not read either
+    const float inv = __int_as_float(d.meta[MT_INV]);
     cnt[tid] = 0;
     __syncthreads();
-    const int m = P == 0 ? n : d.meta[MT_M];
     for (int r = 0; r < SM_ROWS; r++) {
         unsigned key;
         int id;
         bool keep;
-        sm_in<P>(d, (int)blockIdx.x * SM_E + r * SM_RT + tid, m, cutoff, filt, key, id, keep);
+        sm_in<P>(d, (int)blockIdx.x * SM_E + r * SM_RT + tid, m, inv, cutoff, filt, key, id, keep);
         if (keep) atomicAdd(&cnt[(key >> (8 * P)) & 255], 1);
     }
     __syncthreads();
@@ -374,8 +402,10 @@ __global__ void __launch_bounds__(SM_RT) k_smp_scatter(Dev d, int n, float cutof
     __shared__ int goff[256];
     __shared__ int wsum[NW];
     if (d.meta[MT_DONE]) return;
-    const int tid = sm_tid(), lane = tid & 63, w = tid >> 6, NB = (int)gridDim.x, b = (int)blockIdx.x;
-    const int m = P == 0 ? n : d.meta[MT_M];
+    const int tid = sm_tid(), lane = tid & 63, w = tid >> 6, b = (int)blockIdx.x;
+    const int m = P == 0 ? n : d.meta[MT_M], NB = (m + SM_E - 1) / SM_E;   // the workgroups that hold ids
+    if (b >= NB) return;
+    const float inv = __int_as_float(d.meta[MT_INV]);
     // digit tid: ids of this digit in earlier workgroups, and in all; the
     // counts are read SM_HB at a time, so their L2 latencies overlap
     int tot = 0, pre = 0;
@@ -405,7 +435,7 @@ __global__ void __launch_bounds__(SM_RT) k_smp_scatter(Dev d, int n, float cutof
     const unsigned long long lt = (1ull << lane) - 1ull;
 #pragma unroll
     for (int r = 0; r < SM_ROWS; r++) {
-        sm_in<P>(d, b * SM_E + r * SM_RT + tid, m, cutoff, filt, key[r], id[r], keep[r]);
+        sm_in<P>(d, b * SM_E + r * SM_RT + tid, m, inv, cutoff, filt, key[r], id[r], keep[r]);
         dg[r] = (int)((key[r] >> (8 * P)) & 255u);
         unsigned long long pm = __ballot(keep[r]);
 #pragma unroll
@@ -448,7 +478,7 @@ __global__ void __launch_bounds__(SM_RT) k_smp_scatter(Dev d, int n, float cutof
 // the probabilities).
 template <int MODE>
 __global__ void __launch_bounds__(SM_NT) k_smp_final(int *tok, int n, Dev d, int *pos, int *log) {
-    extern __shared__ __align__(16) unsigned char sm_lds[];
+    __shared__ __align__(16) unsigned char sm_lds[SM_LDS];
     __shared__ float rv[SM_NT / 64];
     __shared__ int ri[SM_NT / 64];
     int t;
@@ -474,7 +504,8 @@ __global__ void __launch_bounds__(SM_NT) k_smp_final(int *tok, int n, Dev d, int
         } else {
             const int m = d.meta[MT_M];
             if (m == 0) {
-                t = sm_argmax(d.probs, n, rv, ri);
+                const float inv = __int_as_float(d.meta[MT_INV]);
+                t = sm_argmax([&](int i) { return sm_prob(d.probs[i], inv); }, n, rv, ri);
             } else {
                 float cum, c;
                 const int i = sm_first_above(term, m, d.topp, sm_lds, cum);
@@ -609,24 +640,24 @@ extern "C" void krh_sample(krh_sampler *s, int *tok, float *logits, int n, int *
     hipLaunchKernelGGL(k_smp_exp, dim3(nblk), dim3(256), 0, st, n, nblk, d);
     switch (mode) {
     case SM_MULT:
-        hipLaunchKernelGGL(k_smp_main<SM_MULT>, dim3(1), dim3(SM_NT), SM_LDS, st, tok, n, d, pos, log);
+        hipLaunchKernelGGL(k_smp_main<SM_MULT>, dim3(1), dim3(SM_NT), 0, st, tok, n, d, pos, log);
         break;
     default: {
         const int topp = mode == SM_TOPP;
         // model/sampler.c:134, in float as there
         const float cutoff = topp && n > 1 ? (1.0f - d.topp) / (float)(n - 1) : 0.0f;
         if (topp)
-            hipLaunchKernelGGL(k_smp_main<SM_TOPP>, dim3(1), dim3(SM_NT), SM_LDS, st, tok, n, d, pos, log);
+            hipLaunchKernelGGL(k_smp_main<SM_TOPP>, dim3(1), dim3(SM_NT), 0, st, tok, n, d, pos, log);
         else
-            hipLaunchKernelGGL(k_smp_main<SM_TOPK>, dim3(1), dim3(SM_NT), SM_LDS, st, tok, n, d, pos, log);
+            hipLaunchKernelGGL(k_smp_main<SM_TOPK>, dim3(1), dim3(SM_NT), 0, st, tok, n, d, pos, log);
         sort_pass<0>(d, n, cutoff, topp);
         sort_pass<1>(d, n, cutoff, topp);
         sort_pass<2>(d, n, cutoff, topp);
         sort_pass<3>(d, n, cutoff, topp);
         if (topp)
-            hipLaunchKernelGGL(k_smp_final<SM_TOPP>, dim3(1), dim3(SM_NT), SM_LDS, st, tok, n, d, pos, log);
+            hipLaunchKernelGGL(k_smp_final<SM_TOPP>, dim3(1), dim3(SM_NT), 0, st, tok, n, d, pos, log);
         else
-            hipLaunchKernelGGL(k_smp_final<SM_TOPK>, dim3(1), dim3(SM_NT), SM_LDS, st, tok, n, d, pos, log);
+            hipLaunchKernelGGL(k_smp_final<SM_TOPK>, dim3(1), dim3(SM_NT), 0, st, tok, n, d, pos, log);
     }
     }
     kr_check_launch("sample");

@@ -88,9 +88,18 @@ def test_sample_matches_oracle(name, n):
         draws_match(n, opts, kind, 3, seed=7000 + 100 * n + k)
 
 
+@pytest.mark.parametrize("name", ["mult", "topp", "topk_big"])
+@pytest.mark.parametrize("n", [32768, 32769, 66000])
+def test_sample_group_edges(name, n):
+    """vocabularies of exactly one ordered-sum group, one id more, and a ragged third group"""
+    opts = O.sampler_opts(**OPTS[name])
+    for k, kind in enumerate(["normal", "flat", "ties"]):
+        draws_match(n, opts, kind, 3, 900 + k)
+
+
 @pytest.mark.parametrize("name", ["mult", "topp", "topk", "topk_big", "greedy_penalty", "topp_tiny"])
 def test_sample_matches_oracle_llama3_vocab(name):
-    """128256 ids: the softmax's sum and the draws' sums over eleven groups,
+    """128256 ids: the softmax's sum and the draws' sums over several groups,
     the sort over 126 workgroups"""
     opts = O.sampler_opts(**OPTS[name])
     for k, kind in enumerate(["normal", "ties", "tiny", "flat", "nan"]):
