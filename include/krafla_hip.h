@@ -244,11 +244,11 @@ void krh_attention_batch(float *ao, float *att, const float *q, const float *kc,
                          int n_kv_heads, int head_dim, int max_seq, int window, float scale, const int *pos0, int ntok,
                          int last_pos);
 /* The batched attention's choice of kernels (no counterpart in the
- * reference): heads of 64 or 128 dims take the register-blocked score and
- * mix kernels when their rows (token, query head) fill at least min_wg
- * workgroups of 64 rows, and the per-token-block kernels below that
- * (default 512). Tests lower it to run the register-blocked kernels on small
- * shapes; the results are the same bits either way. Process-wide. */
+ * reference): heads of 48, 64, 80, 96, 128 or 256 dims take the
+ * register-blocked score and mix kernels when their grids hold at least
+ * min_wg / 2 workgroups, and the per-token-block kernels below that (default
+ * 512). Tests lower it to run the register-blocked kernels on small shapes;
+ * the results are the same bits either way. Process-wide. */
 void krh_set_attn_rb_min(int min_wg);
 /* h = silu(g) * u per token (k_scalar.c:96-98), quantized to Q8_0 with
  * transposed scales dT[b * ldd + t] */

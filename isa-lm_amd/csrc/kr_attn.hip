@@ -3,6 +3,7 @@
 // kernels/scalar/k_scalar.c:66-77, :111-155), and the F16 / Q8 cache stores
 // (model/transformer.c:191-205). Every float operation is the reference's,
 // in its order.
+#include <algorithm>
 #include "kr_internal.h"
 #include "kr_numerics.h"
 #include "kr_chain.h"
@@ -28,6 +29,17 @@ __device__ __forceinline__ void attn_range(const int *pos_p, int window, int *fi
     *first = window && pos >= window ? pos + 1 - window : 0;
     *n = pos + 1 - *first;
 }
+
+// Where a windowed token's scores start in its row of the scratch: a batched
+// launch (prefill) stores position p's score at index p, so that the tokens
+// of a block, whose windows start one position apart, share position tiles
+// and aligned reads; a decode launch packs the row from its first attended
+// position. Without a window both are position 0. (BATCH is a template
+// argument: reading it from the launch's grid cost the decode kernels 0.7 us
+// of the 41 us an 8B-shape attention block takes.)
+template <bool BATCH> __device__ __forceinline__ int attn_row0(int first) { return BATCH ? first : 0; }
+// the first position token position pos attends
+__device__ __forceinline__ int attn_first(int pos, int window) { return window && pos >= window ? pos + 1 - window : 0; }
 
 // The cache a launch reads (ml_kv_layer, ops/ops.h:16-22, of one layer): K
 // and V rows [max_seq][kv_dim] of floats, halves or int8, and for the Q8
@@ -72,13 +84,13 @@ template <> struct Kv4<KV_Q8> {
 // floats apart so that the 16-byte reads of 8 consecutive lanes cover all
 // banks once; thread (t, j) computes heads j, j + 4, ... of the group for
 // position t, adding the products in index order.
-template <int KT, int TT>
+template <int KT, int TT, bool BATCH>
 __device__ __forceinline__ void attn_scores(float *att, const float *q, const KvView kv, int group, int hd, int kv_dim,
                                             int max_seq, int window, float scale, const int *pos_p) {
     extern __shared__ __align__(16) float at_smem[];
     int first, n;
     attn_range(pos_p, window, &first, &n);
-    att += (size_t)blockIdx.z * gridDim.x * group * max_seq;   // token z: [n_heads][max_seq]
+    att += (size_t)blockIdx.z * gridDim.x * group * max_seq + attn_row0<BATCH>(first);   // token z: [n_heads][max_seq]
     q += (size_t)blockIdx.z * gridDim.x * group * hd;
     const int g = blockIdx.x, t0 = blockIdx.y * TT, tid = threadIdx.x;
     if (t0 >= n) return;
@@ -111,19 +123,19 @@ __device__ __forceinline__ void attn_scores(float *att, const float *q, const Kv
 }
 
 // the F32 cache (its own argument list: the view is built on the device)
-template <int TT>
+template <int TT, bool BATCH = false>
 __global__ void __launch_bounds__(AT_THREADS) k_attn_scores(float *att, const float *q, const float *kc, int group,
                                                             int hd, int kv_dim, int max_seq, int window, float scale,
                                                             const int *pos_p) {
     const KvView kv = { kc, nullptr, nullptr, nullptr, 0 };
-    attn_scores<KV_F32, TT>(att, q, kv, group, hd, kv_dim, max_seq, window, scale, pos_p);
+    attn_scores<KV_F32, TT, BATCH>(att, q, kv, group, hd, kv_dim, max_seq, window, scale, pos_p);
 }
 
-// Batched (prefill) scores over the F32 or F16 cache without a window, a
-// block of AT_TB tokens at a time (F16 rows widened exactly as the K tile is
-// staged). Every token of the block attends from position 0,
-// so one K tile of AT_T positions, staged once in LDS, serves the whole block
-// (the per-token kernel stages it again for every token). The queries of QB
+// Batched (prefill) scores over the F32 or F16 cache, a block of AT_TB tokens
+// at a time (F16 rows widened exactly as the K tile is staged). The block's
+// tiles start at the tile that holds its first token's first attended
+// position; one K tile of AT_T positions, staged once in LDS, serves the
+// whole block (the per-token kernel stages it again for every token). The queries of QB
 // tokens at a time follow in LDS; thread (position t, head j) runs the QB
 // chains of those tokens in one pass over the head's dims, one K read feeding
 // them all (QB independent chains: the LDS latency hides under them). Each
@@ -135,12 +147,13 @@ __global__ void __launch_bounds__(AT_THREADS) k_attn_scores(float *att, const fl
 constexpr int AT_TB = 16;
 template <int HD, int QB, int KT, int TP = AT_T>
 __global__ void __launch_bounds__(AT_THREADS) k_attn_scores_blk(float *att, const float *q, const KvView kv, int group,
-                                                                int hd_arg, int kv_dim, int max_seq, float scale,
-                                                                const int *pos_p, int ntok) {
+                                                                int hd_arg, int kv_dim, int max_seq, int window,
+                                                                float scale, const int *pos_p, int ntok) {
     extern __shared__ __align__(16) float at_smem[];
     const int hd = HD ? HD : hd_arg;
-    const int g = blockIdx.x, t0 = blockIdx.y * TP, z0 = blockIdx.z * AT_TB, tid = threadIdx.x;
+    const int g = blockIdx.x, z0 = blockIdx.z * AT_TB, tid = threadIdx.x;
     const int pos0 = *pos_p, zn = min(AT_TB, ntok - z0);
+    const int t0 = attn_first(pos0 + z0, window) / TP * TP + blockIdx.y * TP;
     const int nlast = pos0 + z0 + zn;   // positions the block's last token attends
     if (t0 >= nlast) return;
     const int nt = min(TP, nlast - t0), ks = hd + 4, h4 = hd / 4, n_heads = gridDim.x * group;
@@ -150,7 +163,7 @@ __global__ void __launch_bounds__(AT_THREADS) k_attn_scores_blk(float *att, cons
         *(float4 *)(kt + r * ks + 4 * c) =
             Kv4<KT>::wide(Kv4<KT>::load(kv.k, (size_t)(t0 + r) * kv_dim + (size_t)g * hd + 4 * c));
     }
-    const int t = tid % TP, p = t0 + t;   // this thread's position (absolute: no window)
+    const int t = tid % TP, p = t0 + t;   // this thread's position
     const size_t qstride = (size_t)group * hd;   // floats between two tokens' queries in LDS
     for (int zb = 0; zb < zn; zb += QB) {
         const int qn = min(QB, zn - zb), gh4 = group * h4;
@@ -184,113 +197,141 @@ __global__ void __launch_bounds__(AT_THREADS) k_attn_scores_blk(float *att, cons
 #pragma unroll
             for (int u = 0; u < QB; u++) {
                 const int z = z0 + zb + u;
-                if (u < qn && p <= pos0 + z)
+                if (u < qn && p <= pos0 + z && p >= attn_first(pos0 + z, window))
                     att[((size_t)z * n_heads + (size_t)g * group + j) * max_seq + p] = kr_fmul(acc[u], scale);
             }
         }
     }
 }
 
-// Batched (prefill) scores without a window for heads of HD = 64 or 128
-// dims, blocked in registers: the rows (token z, query head j) of KV head g,
-// numbered z * group + j, go to workgroups RB_R at a time, each over a chunk
-// of RB_PC tiles of RB_T positions. The workgroup stages its rows' queries
-// in LDS once and each K tile in turn (F16 rows widened exactly), rows HD + 4
-// floats apart; lane (row group rg, position group pg) owns the scores of rows
-// 4 rg .. 4 rg + 3 at positions pg + 16 k (k < 4): per 4 dims it reads 4 query
-// and 4 K 16-byte values, which feed 64 multiplies and 64 adds, each of its
-// 16 sums s = sum_i q_i k_i in index order, then * scale, as in the per-token
-// kernel. A row stores only the positions its token attends. The next tile's
-// loads are in flight while a tile is summed.
+// Batched (prefill) scores for heads of HD dims, blocked in registers: the
+// rows (token z, query head j) of KV head g, numbered z * group + j, go to
+// workgroups RB_R at a time, each over a chunk of pc tiles of RB_T positions
+// (from the tile of its first row's first attended position). The workgroup
+// stages its rows' queries in LDS once and each K tile in turn (F16 rows
+// widened exactly), rows HS + 4 floats apart; lane (row group rg, position
+// group pg) owns the scores of rows 4 rg .. 4 rg + 3 at positions pg + 16 k
+// (k < 4): per 4 dims it reads 4 query and 4 K 16-byte values, which feed 64
+// multiplies and 64 adds, each of its 16 sums s = sum_i q_i k_i in index
+// order, then * scale, as in the per-token kernel. A row stores only the
+// positions its token attends. The next tile's loads are in flight while a
+// tile is summed. HS < HD (256-dim heads, whose tiles would fill the LDS):
+// the queries and K are staged HS dims at a time, the sums carried along.
 constexpr int RB_R = 64, RB_T = 64;   // rows of a register-blocked workgroup; positions of its tiles
-constexpr int RB_PC = 8;             // K tiles per scores workgroup
-// the register-blocked kernels take 64- and 128-dim heads whose rows fill at
-// least 512 workgroups (two a CU): a 511-token prompt over 2 KV heads of 7
-// query heads gives 112, and there the per-token-block kernels measured twice
-// as fast (scores 45.6 against 21.6 us a layer, mix 51.2 against 28.5)
+constexpr int RB_PC = 8;             // K tiles per scores workgroup, at most
+// the register-blocked kernels run when their grids hold at least this many
+// half workgroups (a whole one per CU: rb_fills); smaller grids take the
+// per-token-block kernels. Measured on both sides of the line (us, scores to
+// mix, register-blocked from 128, 256 and 512 workgroups, and never): 8
+// heads of 256 over a 1024 window, 1021 tokens 306, 237, 329, 538; 24 heads of
+// 80, window 300, 1000 tokens 163, 155, 175, 178; 8 heads of 96, window 512,
+// 300 tokens 78, 77, 90, 90; 32 heads of 64, 256 tokens 60, 45, 45, 47.
 static int g_rb_min_wg = 512;
-static bool rb_shape(int hd, int ntok, int group, int n_kv) {
-    return (hd == 64 || hd == 128) && (long)n_kv * ((ntok * group + RB_R - 1) / RB_R) >= g_rb_min_wg;
-}
+static bool rb_fills(long wgs) { return 2 * wgs >= g_rb_min_wg; }
+static bool rb_dims(int hd) { return hd == 48 || hd == 64 || hd == 80 || hd == 96 || hd == 128 || hd == 256; }
 constexpr int RB_NT128 = 512;        // threads of the 128-dim heads' workgroups (4 outputs' rows a lane, LDS for 2
                                      // workgroups a CU: 4 waves a SIMD; 256 threads gave 2 and measured the same)
-template <int HD, int KT, int NT>
+template <int HD, int KT, int NT, bool WIN, int HS = HD>
 __global__ void __launch_bounds__(NT) k_attn_scores_rb(float *att, const float *q, const KvView kv, int group,
-                                                       int kv_dim, int max_seq, float scale, const int *pos_p,
-                                                       int ntok) {
-    constexpr int S = HD + 4;                     // LDS row stride (floats)
+                                                       int kv_dim, int max_seq, int window_arg, float scale,
+                                                       const int *pos_p, int ntok, int pc) {
+    const int window = WIN ? window_arg : 0;
+    constexpr int S = HS + 4;                     // LDS row stride (floats)
+    constexpr int NS = HD / HS;                   // dim slices
     constexpr int NPG = NT / 16, PPL = RB_T / NPG;   // position groups; positions a lane (pg + NPG k)
-    constexpr int NL = RB_T * HD / 4 / NT;        // 4-element K loads a thread stages per tile
-    constexpr int NQL = RB_R * HD / 4 / NT;       // query float4 a thread stages
+    constexpr int NL = RB_T * HS / 4 / NT;        // 4-element K loads a thread stages per tile
+    constexpr int NQL = RB_R * HS / 4 / NT;       // query float4 a thread stages
+    static_assert(NS * HS == HD && NL * NT * 4 == RB_T * HS && NQL * NT * 4 == RB_R * HS, "whole loads");
     __shared__ __align__(16) float qs[RB_R * S];
     __shared__ __align__(16) float ks[RB_T * S];
     const int g = blockIdx.x, tid = threadIdx.x, pg = tid % NPG, rg = tid / NPG;
     const int nrow = ntok * group, R0 = blockIdx.y * RB_R;
     const int pos0 = *pos_p, n_heads = gridDim.x * group;
     const int nlast = pos0 + (min(R0 + RB_R, nrow) - 1) / group + 1;   // positions the block's last row attends
-    const int p0 = blockIdx.z * RB_PC * RB_T;
+    const int p0 = attn_first(pos0 + R0 / group, window) / RB_T * RB_T + blockIdx.z * pc * RB_T;
     if (p0 >= nlast) return;
-    const int ntl = min(RB_PC, (nlast - p0 + RB_T - 1) / RB_T);
-#pragma unroll
-    for (int u = 0; u < NQL; u++) {
-        const int e = tid + NT * u, rr = e / (HD / 4), c4 = e % (HD / 4);
+    const int ntl = min(pc, (nlast - p0 + RB_T - 1) / RB_T);
+    auto q_load = [&](int u, int c0) {
+        const int e = tid + NT * u, rr = e / (HS / 4), c4 = e % (HS / 4);
         const int R = min(R0 + rr, nrow - 1), z = R / group, j = R - z * group;
-        *(float4 *)(qs + rr * S + 4 * c4) = *(const float4 *)(q + ((size_t)z * n_heads + (size_t)g * group + j) * HD + 4 * c4);
-    }
+        return *(const float4 *)(q + ((size_t)z * n_heads + (size_t)g * group + j) * HD + c0 + 4 * c4);
+    };
+    auto q_store = [&](int u, float4 v) {
+        const int e = tid + NT * u, rr = e / (HS / 4), c4 = e % (HS / 4);
+        *(float4 *)(qs + rr * S + 4 * c4) = v;
+    };
     typename Kv4<KT>::T kr[NL];
-    auto load = [&](int t0) {
+    float4 qr[NS > 1 ? NQL : 1];
+    auto load = [&](int t0, int c0) {
 #pragma unroll
         for (int u = 0; u < NL; u++) {
-            const int e = tid + NT * u, p = e / (HD / 4), c4 = e % (HD / 4);
-            kr[u] = Kv4<KT>::load(kv.k, (size_t)min(t0 + p, nlast - 1) * kv_dim + (size_t)g * HD + 4 * c4);
+            const int e = tid + NT * u, p = e / (HS / 4), c4 = e % (HS / 4);
+            kr[u] = Kv4<KT>::load(kv.k, (size_t)min(t0 + p, nlast - 1) * kv_dim + (size_t)g * HD + c0 + 4 * c4);
+        }
+        if constexpr (NS > 1) {
+#pragma unroll
+            for (int u = 0; u < NQL; u++) qr[u] = q_load(u, c0);
         }
     };
-    int zr[4];   // the tokens of the lane's rows (past the last row: -1)
+    if constexpr (NS == 1) {
+#pragma unroll
+        for (int u = 0; u < NQL; u++) q_store(u, q_load(u, 0));
+    }
+    int zr[4], lo[4];   // the tokens of the lane's rows (past the last row: -1) and the first positions they attend
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         const int R = R0 + 4 * rg + r;
         zr[r] = R < nrow ? R / group : -1;
+        lo[r] = attn_first(pos0 + R / group, window);
     }
-    load(p0);
+    load(p0, 0);
     for (int ti = 0; ti < ntl; ti++) {
         const int t0 = p0 + ti * RB_T;
-        __syncthreads();   // the last tile is read
-#pragma unroll
-        for (int u = 0; u < NL; u++) {
-            const int e = tid + NT * u, p = e / (HD / 4), c4 = e % (HD / 4);
-            *(float4 *)(ks + p * S + 4 * c4) = Kv4<KT>::wide(kr[u]);
-        }
-        __syncthreads();
-        if (ti + 1 < ntl) load(t0 + RB_T);
         float acc[4][PPL];
 #pragma unroll
         for (int r = 0; r < 4; r++)
 #pragma unroll
             for (int k = 0; k < PPL; k++) acc[r][k] = 0.0f;
-        const float *qp = qs + 4 * rg * S, *kp = ks + pg * S;
+#pragma unroll 1
+        for (int sl = 0; sl < NS; sl++) {
+            __syncthreads();   // the last tile is read
+#pragma unroll
+            for (int u = 0; u < NL; u++) {
+                const int e = tid + NT * u, p = e / (HS / 4), c4 = e % (HS / 4);
+                *(float4 *)(ks + p * S + 4 * c4) = Kv4<KT>::wide(kr[u]);
+            }
+            if constexpr (NS > 1) {
+#pragma unroll
+                for (int u = 0; u < NQL; u++) q_store(u, qr[u]);
+            }
+            __syncthreads();
+            if (sl + 1 < NS) load(t0, (sl + 1) * HS);
+            else if (ti + 1 < ntl) load(t0 + RB_T, 0);
+            const float *qp = qs + 4 * rg * S, *kp = ks + pg * S;
 #pragma unroll 4
-        for (int i = 0; i < HD; i += 4) {
-            float4 a[4], b[PPL];
+            for (int i = 0; i < HS; i += 4) {
+                float4 a[4], b[PPL];
 #pragma unroll
-            for (int r = 0; r < 4; r++) a[r] = *(const float4 *)(qp + r * S + i);
+                for (int r = 0; r < 4; r++) a[r] = *(const float4 *)(qp + r * S + i);
 #pragma unroll
-            for (int k = 0; k < PPL; k++) b[k] = *(const float4 *)(kp + NPG * k * S + i);
+                for (int k = 0; k < PPL; k++) b[k] = *(const float4 *)(kp + NPG * k * S + i);
 #pragma unroll
-            for (int r = 0; r < 4; r++)
+                for (int r = 0; r < 4; r++)
 #pragma unroll
-                for (int k = 0; k < PPL; k++) acc[r][k] = kr_fadd(acc[r][k], kr_fmul(a[r].x, b[k].x));
+                    for (int k = 0; k < PPL; k++) acc[r][k] = kr_fadd(acc[r][k], kr_fmul(a[r].x, b[k].x));
 #pragma unroll
-            for (int r = 0; r < 4; r++)
+                for (int r = 0; r < 4; r++)
 #pragma unroll
-                for (int k = 0; k < PPL; k++) acc[r][k] = kr_fadd(acc[r][k], kr_fmul(a[r].y, b[k].y));
+                    for (int k = 0; k < PPL; k++) acc[r][k] = kr_fadd(acc[r][k], kr_fmul(a[r].y, b[k].y));
 #pragma unroll
-            for (int r = 0; r < 4; r++)
+                for (int r = 0; r < 4; r++)
 #pragma unroll
-                for (int k = 0; k < PPL; k++) acc[r][k] = kr_fadd(acc[r][k], kr_fmul(a[r].z, b[k].z));
+                    for (int k = 0; k < PPL; k++) acc[r][k] = kr_fadd(acc[r][k], kr_fmul(a[r].z, b[k].z));
 #pragma unroll
-            for (int r = 0; r < 4; r++)
+                for (int r = 0; r < 4; r++)
 #pragma unroll
-                for (int k = 0; k < PPL; k++) acc[r][k] = kr_fadd(acc[r][k], kr_fmul(a[r].w, b[k].w));
+                    for (int k = 0; k < PPL; k++) acc[r][k] = kr_fadd(acc[r][k], kr_fmul(a[r].w, b[k].w));
+            }
         }
 #pragma unroll
         for (int r = 0; r < 4; r++) {
@@ -300,17 +341,17 @@ __global__ void __launch_bounds__(NT) k_attn_scores_rb(float *att, const float *
 #pragma unroll
             for (int k = 0; k < PPL; k++) {
                 const int p = t0 + pg + NPG * k;
-                if (p <= pos0 + zr[r]) dst[p] = kr_fmul(acc[r][k], scale);
+                if (p <= pos0 + zr[r] && p >= lo[r]) dst[p] = kr_fmul(acc[r][k], scale);
             }
         }
     }
 }
 
-template <int KT, int TT>
+template <int KT, int TT, bool BATCH = false>
 __global__ void __launch_bounds__(AT_THREADS) k_attn_scores_kv(float *att, const float *q, const KvView kv, int group,
                                                                int hd, int kv_dim, int max_seq, int window, float scale,
                                                                const int *pos_p) {
-    attn_scores<KT, TT>(att, q, kv, group, hd, kv_dim, max_seq, window, scale, pos_p);
+    attn_scores<KT, TT, BATCH>(att, q, kv, group, hd, kv_dim, max_seq, window, scale, pos_p);
 }
 
 // One query head of hd floats as the Q8 rule does it for the score
@@ -334,13 +375,14 @@ __device__ __forceinline__ void q8_head(const float *x, int hd, int8_t *dst, flo
 // ((float)sum * (dq * scale)) * dk_t. K rows are staged in LDS with a stride
 // of hd + 4 bytes (33 words for hd 128: the lanes of a wave spread over the
 // banks).
+template <bool BATCH = false>
 __global__ void __launch_bounds__(AT_THREADS) k_attn_scores_q8(float *att, const float *q, const KvView kv, int group,
                                                                int hd, int kv_dim, int max_seq, int window, float scale,
                                                                const int *pos_p) {
     extern __shared__ __align__(16) float at_smem[];
     int first, n;
     attn_range(pos_p, window, &first, &n);
-    att += (size_t)blockIdx.z * gridDim.x * group * max_seq;
+    att += (size_t)blockIdx.z * gridDim.x * group * max_seq + attn_row0<BATCH>(first);
     q += (size_t)blockIdx.z * gridDim.x * group * hd;
     const int g = blockIdx.x, t0 = blockIdx.y * AT_T, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     if (t0 >= n) return;
@@ -394,8 +436,8 @@ __global__ void __launch_bounds__(AT_THREADS) k_attn_scores_q8(float *att, const
     }
 }
 
-// Batched (prefill) scores over the Q8 cache without a window, a block of
-// AT_TB tokens at a time: the int8 K tile of AT_T positions and its row
+// Batched (prefill) scores over the Q8 cache, a block of AT_TB tokens at a
+// time: the int8 K tile of AT_T positions and its row
 // scales are staged once for the block; then, QB tokens at a time, the
 // workgroup quantizes those tokens' query heads of its group into LDS
 // (q8_head: the per-token kernel's bits) and thread (position t, head j)
@@ -404,11 +446,13 @@ __global__ void __launch_bounds__(AT_THREADS) k_attn_scores_q8(float *att, const
 template <int QB>
 __global__ void __launch_bounds__(AT_THREADS) k_attn_scores_blk_q8(float *att, const float *q, const KvView kv,
                                                                    int group, int hd, int kv_dim, int max_seq,
-                                                                   float scale, const int *pos_p, int ntok) {
+                                                                   int window, float scale, const int *pos_p,
+                                                                   int ntok) {
     extern __shared__ __align__(16) float at_smem[];
-    const int g = blockIdx.x, t0 = blockIdx.y * AT_T, z0 = blockIdx.z * AT_TB, tid = threadIdx.x;
+    const int g = blockIdx.x, z0 = blockIdx.z * AT_TB, tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     const int pos0 = *pos_p, zn = min(AT_TB, ntok - z0);
+    const int t0 = attn_first(pos0 + z0, window) / AT_T * AT_T + blockIdx.y * AT_T;
     const int nlast = pos0 + z0 + zn;   // positions the block's last token attends
     if (t0 >= nlast) return;
     const int nt = min(AT_T, nlast - t0), ks = hd + 4, n_heads = gridDim.x * group, h4 = hd / 4;
@@ -422,7 +466,7 @@ __global__ void __launch_bounds__(AT_THREADS) k_attn_scores_blk_q8(float *att, c
             *(const int *)((const int8_t *)kv.k + (size_t)(t0 + r) * kv_dim + (size_t)g * hd + 4 * c);
     }
     for (int r = tid; r < nt; r += AT_THREADS) dks[r] = kv.kd[(size_t)(t0 + r) * kv.n_kv + g];
-    const int t = tid % AT_T, p = t0 + t;   // this thread's position (absolute: no window)
+    const int t = tid % AT_T, p = t0 + t;   // this thread's position
     for (int zb = 0; zb < zn; zb += QB) {
         const int qn = min(QB, zn - zb);
         __syncthreads();   // the last queries are read
@@ -449,7 +493,7 @@ __global__ void __launch_bounds__(AT_THREADS) k_attn_scores_blk_q8(float *att, c
 #pragma unroll
             for (int u = 0; u < QB; u++) {
                 const int z = z0 + zb + u;
-                if (u < qn && p <= pos0 + z) {
+                if (u < qn && p <= pos0 + z && p >= attn_first(pos0 + z, window)) {
                     const float c = kr_fmul(qd[u * group + j], scale);
                     att[((size_t)z * n_heads + (size_t)g * group + j) * max_seq + p] = kr_fmul(kr_fmul((float)acc[u], c), dk);
                 }
@@ -469,7 +513,7 @@ __global__ void __launch_bounds__(AT_THREADS) k_attn_scores_blk_q8(float *att, c
 // of up to 4096 scores take 256 (the ordered sum needs 4 waves, and a small
 // workgroup lets 8 rows share a CU's LDS and SIMDs).
 constexpr int SMX_THREADS = 1024, AT_CHUNK = 8192;   // the decode launch
-template <int NT, int CH, bool LEAN = false>
+template <int NT, int CH, bool LEAN = false, bool BATCH = LEAN>
 __global__ void __launch_bounds__(NT) k_attn_softmax(float *att, int max_seq, int window, const int *pos_p) {
     constexpr int SMX_THREADS = NT, AT_CHUNK = CH, AT_V = CH / NT;
     __shared__ __align__(16) float es[sc_terms_cap(AT_CHUNK)];
@@ -478,7 +522,7 @@ __global__ void __launch_bounds__(NT) k_attn_softmax(float *att, int max_seq, in
     __shared__ uint64_t xtab[32];   // expf's table
     int first, n;
     attn_range(pos_p, window, &first, &n);
-    float *a = att + ((size_t)blockIdx.z * gridDim.x + blockIdx.x) * max_seq;
+    float *a = att + ((size_t)blockIdx.z * gridDim.x + blockIdx.x) * max_seq + attn_row0<BATCH>(first);
     const int tid = threadIdx.x;
     if (tid < 32) xtab[tid] = kr_exp2_tab[tid];
     const bool fits = n <= AT_CHUNK;
@@ -563,8 +607,8 @@ __global__ void __launch_bounds__(64 * RW) k_attn_softmax_rows(float *att, int n
     const int r = blockIdx.x * RW + wave;
     if (r >= nrows) return;
     const int z = r / n_heads, pos = *pos_p + z;
-    const int first = window && pos >= window ? pos + 1 - window : 0, n = pos + 1 - first;
-    float *a = att + (size_t)r * max_seq;
+    const int first = attn_first(pos, window), n = pos + 1 - first;
+    float *a = att + (size_t)r * max_seq + first;
     float *es = (float *)(sm_lds + (size_t)wave * (4 * terms_cap + scr_bytes));
     unsigned char *scr = (unsigned char *)(es + terms_cap);
     float v[SV];
@@ -870,7 +914,8 @@ __device__ __forceinline__ void attn_mix_batch(float *ao, const float *att, cons
     const int j = lane / DW, d = lane % DW;
     const size_t vb = (size_t)first * kv_dim + (size_t)g * hd + c0;   // element offset of V row `first`
     const size_t q_dim = (size_t)gridDim.x * group * hd;
-    const float *abase = att + ((size_t)blockIdx.z * gridDim.x * group + (size_t)g * group) * max_seq;
+    const int row0 = attn_row0<true>(first), alim = max_seq - 4 - row0;   // the row's last float4, from its first score
+    const float *abase = att + ((size_t)blockIdx.z * gridDim.x * group + (size_t)g * group) * max_seq + row0;
     ao += blockIdx.z * q_dim;
     const int ntiles = (n + MB_T - 1) / MB_T;
     const int cw = min(DW, hd - c0);   // valid dims of the chunk (a multiple of 4)
@@ -895,7 +940,7 @@ __device__ __forceinline__ void attn_mix_batch(float *ao, const float *att, cons
 #pragma unroll
         for (int k = 0; k < NA; k++) {
             const int e = (k * 64 + lane) * 4, jj = min(e / MB_T, group - 1), r = e % MB_T;
-            const float *src = abase + (size_t)jj * max_seq + min(t0 + r, max_seq - 4);
+            const float *src = abase + (ptrdiff_t)((size_t)jj * max_seq) + min(t0 + r, alim);
             a[k] = make_float4(src[0], src[1], src[2], src[3]);
             if (KT == KV_Q8) {
                 const float *d = kv.vd + (size_t)first * kv.n_kv + g;
@@ -919,8 +964,8 @@ __device__ __forceinline__ void attn_mix_batch(float *ao, const float *att, cons
         for (int k = 0; k < NA; k++) {
             const int e = (k * 64 + lane) * 4, r = e % MB_T;
             // a float4 clamped back from the row's end holds position p at
-            // element p - (max_seq - 4): shift it down to element p - p0
-            const int sh = tile * MB_T + r - min(tile * MB_T + r, max_seq - 4);
+            // element p - alim: shift it down to element p - p0
+            const int sh = tile * MB_T + r - min(tile * MB_T + r, alim);
             const float4 x = a[k];
             float4 y;
             y.x = sh == 0 ? x.x : sh == 1 ? x.y : sh == 2 ? x.z : x.w;
@@ -1011,7 +1056,7 @@ __device__ __forceinline__ void attn_mix_batch(float *ao, const float *att, cons
     if (j < group && d < cw) ao[(size_t)(g * group + j) * hd + c0 + d] = o;
 }
 
-// Batched (prefill) mix without a window, by blocks of MK_W x MK_U tokens: a
+// Batched (prefill) mix by blocks of MK_W x MK_U tokens: a
 // workgroup per (KV head g, DW dims from c0, MK_W MK_U consecutive tokens),
 // MK_U consecutive tokens per wave, lane = (head j of the group, dim d); each
 // lane runs its tokens' chains o += a_t * v_t,d over positions t in order
@@ -1051,8 +1096,8 @@ __device__ __forceinline__ void mk_quad(float (&o)[U], const float (&a)[U], floa
 
 template <int DW, int KT>
 __global__ void __launch_bounds__(64 * MK_W) k_attn_mix_blk(float *ao, const float *att, const KvView kv, int group,
-                                                            int hd, int kv_dim, int max_seq, const int *pos_p,
-                                                            int ntok) {
+                                                            int hd, int kv_dim, int max_seq, int window,
+                                                            const int *pos_p, int ntok) {
     static_assert(DW >= 16, "a 16-lane row must hold one head");
     constexpr int U = MK_U;
     constexpr int QPR = DW / 4;                 // float4 per staged row of DW dims
@@ -1064,12 +1109,15 @@ __global__ void __launch_bounds__(64 * MK_W) k_attn_mix_blk(float *ao, const flo
     const int wave = tid >> 6, lane = tid & 63, j = lane / DW, d = lane % DW;
     const int zw = z0 + wave * U, pos0 = *pos_p;      // the wave's first token
     const int nmax = pos0 + min(z0 + MK_W * U, ntok);   // positions the block's last token attends
-    const int n_heads = gridDim.x * group, cw = min(DW, hd - c0), ntiles = (nmax + MK_T - 1) / MK_T;
-    int n[U];   // positions token zw + u attends (0 past the last token)
+    const int n_heads = gridDim.x * group, cw = min(DW, hd - c0);
+    const int base = attn_first(pos0 + z0, window) / MK_T * MK_T;   // the block's first tile
+    const int ntiles = (nmax - base + MK_T - 1) / MK_T;
+    int n[U], f[U];   // token zw + u attends positions f .. n - 1 (n 0 past the last token)
     const float *arow[U];
 #pragma unroll
     for (int u = 0; u < U; u++) {
         n[u] = zw + u < ntok ? pos0 + zw + u + 1 : 0;
+        f[u] = attn_first(pos0 + zw + u, window);
         arow[u] = att + ((size_t)min(zw + u, ntok - 1) * n_heads + (size_t)g * group + min(j, group - 1)) * max_seq;
     }
     const size_t vbase = (size_t)g * hd + c0;   // element offset of the chunk in a V row
@@ -1081,8 +1129,8 @@ __global__ void __launch_bounds__(64 * MK_W) k_attn_mix_blk(float *ao, const flo
     auto stage_load = [&](int tile) {
 #pragma unroll
         for (int p = 0; p < NP; p++)
-            sv[p] = Kv4<KT>::load(kv.v, vbase + (size_t)min(tile * MK_T + p * RPP + srow, nmax - 1) * kv_dim + scol);
-        if (KT == KV_Q8 && tid < MK_T) sd = kv.vd[(size_t)min(tile * MK_T + tid, nmax - 1) * kv.n_kv + g];
+            sv[p] = Kv4<KT>::load(kv.v, vbase + (size_t)min(base + tile * MK_T + p * RPP + srow, nmax - 1) * kv_dim + scol);
+        if (KT == KV_Q8 && tid < MK_T) sd = kv.vd[(size_t)min(base + tile * MK_T + tid, nmax - 1) * kv.n_kv + g];
     };
     auto stage_store = [&](int buf) {
         float *V = vt[buf];
@@ -1103,7 +1151,7 @@ __global__ void __launch_bounds__(64 * MK_W) k_attn_mix_blk(float *ao, const flo
 #pragma unroll
         for (int u = 0; u < U; u++)
 #pragma unroll
-            for (int b = 0; b < MK_T / 16; b++) a[u][b] = arow[u][min(tile * MK_T + 16 * b + (lane & 15), max_seq - 1)];
+            for (int b = 0; b < MK_T / 16; b++) a[u][b] = arow[u][min(base + tile * MK_T + 16 * b + (lane & 15), max_seq - 1)];
     };
     float o[U];
 #pragma unroll
@@ -1116,7 +1164,7 @@ __global__ void __launch_bounds__(64 * MK_W) k_attn_mix_blk(float *ao, const flo
     if (ntiles > 1) stage_load(1);
     __syncthreads();
     for (int k = 0; k < ntiles; k++) {
-        const int buf = k & 1, t0 = k * MK_T;
+        const int buf = k & 1, t0 = base + k * MK_T;
         if (k + 1 < ntiles) stage_store(buf ^ 1);   // its last reader finished before the last barrier
         a_load(min(k + 2, ntiles - 1), anext2);
         // unconditional (a clamped tile past the end is loaded and never
@@ -1130,7 +1178,7 @@ __global__ void __launch_bounds__(64 * MK_W) k_attn_mix_blk(float *ao, const flo
 #pragma unroll
             for (int u = 0; u < U; u++)
                 aw[b][u] = KT == KV_Q8 ? kr_fmul(acur[u][b], dvs[buf][KT == KV_Q8 ? 16 * b + (lane & 15) : 0]) : acur[u][b];
-        if (t0 + MK_T <= n[0]) {   // a full tile for every token of the wave (tokens past the last are not stored)
+        if (t0 + MK_T <= n[0] && t0 >= f[U - 1]) {   // a full tile for every token of the wave (tokens past the last are not stored)
 #pragma unroll
             for (int b = 0; b < MK_T / 16; b++) {
                 const float4 v0 = *(const float4 *)(V + 16 * b), v1 = *(const float4 *)(V + 16 * b + 4);
@@ -1140,10 +1188,10 @@ __global__ void __launch_bounds__(64 * MK_W) k_attn_mix_blk(float *ao, const flo
                 mk_quad<2>(o, aw[b], v2);
                 mk_quad<3>(o, aw[b], v3);
             }
-        } else {   // the last tiles: each token its live positions
+        } else {   // the first and last tiles: each token its live positions
 #pragma unroll
             for (int u = 0; u < U; u++) {
-                if (t0 >= n[u]) continue;
+                if (t0 >= n[u] || t0 + MK_T <= f[u]) continue;
 #pragma unroll
                 for (int b = 0; b < MK_T / 16; b++) {
                     const float ab = aw[b][u];
@@ -1152,7 +1200,8 @@ __global__ void __launch_bounds__(64 * MK_W) k_attn_mix_blk(float *ao, const flo
                     w[4] = row_bcast<4>(ab); w[5] = row_bcast<5>(ab); w[6] = row_bcast<6>(ab); w[7] = row_bcast<7>(ab);
                     w[8] = row_bcast<8>(ab); w[9] = row_bcast<9>(ab); w[10] = row_bcast<10>(ab); w[11] = row_bcast<11>(ab);
                     w[12] = row_bcast<12>(ab); w[13] = row_bcast<13>(ab); w[14] = row_bcast<14>(ab); w[15] = row_bcast<15>(ab);
-                    for (int i = 0; i < 16 && t0 + 16 * b + i < n[u]; i++) o[u] = kr_fadd(o[u], kr_fmul(w[i], V[16 * b + i]));
+                    for (int i = 0; i < 16 && t0 + 16 * b + i < n[u]; i++)
+                        if (t0 + 16 * b + i >= f[u]) o[u] = kr_fadd(o[u], kr_fmul(w[i], V[16 * b + i]));
                 }
             }
         }
@@ -1173,51 +1222,61 @@ __global__ void __launch_bounds__(64 * MK_W) k_attn_mix_blk(float *ao, const flo
     }
 }
 
-// Batched (prefill) mix without a window for heads of HD = 64 or 128 dims,
-// blocked in registers: the rows (token z, query head j) of KV head g,
-// numbered z * group + j, go to workgroups RB_R at a time (the longest
-// first), and lane (row group rg, dim group dg) of a workgroup owns the
-// 4 x HD / 16 outputs of rows 4 rg .. 4 rg + 3 and dims 64 k + 4 dg + i: one
-// chain o += a_t * v_t,d per output over positions t in order
-// (k_scalar.c:119-122), each product rounded before its add. Per tile of
-// RB_T positions the weights [row][position] (Q8: a_t * dv_t, the per-token
-// kernel's product) and the V rows [position][dim] (F16 widened, Q8 as its
-// int8 values) are staged in LDS; per 4 positions a lane reads its rows' 4
-// weights and, per position, its dims' V values, 16-byte reads that feed
-// every product they take part in (4 x HD / 16 chains a lane, 2 to 4 reads
-// for 64 to 128 multiplies and as many adds: no broadcasts of a weight
-// across lanes). In the tiles past some row's own positions a select leaves
+// Batched (prefill) mix blocked in registers: the rows (token z, query head
+// j) of KV head g, numbered z * group + j, go to workgroups RB_R at a time
+// (the longest first), CW of the head's dims each, and lane (row group rg,
+// dim group dg) of a workgroup owns the 4 x 4 outputs of rows 4 rg ..
+// 4 rg + 3 and dims 4 dg + i: one chain o += a_t * v_t,d per output over
+// positions t in order (k_scalar.c:119-122), each product rounded before its
+// add. Per tile of RB_T positions (from the tile of the first row's first
+// attended position) the weights [row][position] (Q8: a_t * dv_t, the
+// per-token kernel's product) and the V rows [position][dim] (F16 widened, Q8
+// as its int8 values) are staged in LDS; per 4 positions a lane reads its
+// rows' 4 weights and, per position, its dims' V values, 16-byte reads that
+// feed every product they take part in (16 chains a lane, 2 reads for 16
+// multiplies and as many adds: no broadcasts of a weight across lanes). In the
+// tiles past some row's own positions, or before its window, a select leaves
 // those terms out of that row's sums, so no weight or V value there (rows of
 // later tokens, stale rows) reaches them. The next tile's loads are in flight
 // while a tile is summed.
-template <int HD, int KT, int NT>
-__global__ void __launch_bounds__(NT) k_attn_mix_rb(float *ao, const float *att, const KvView kv, int group,
-                                                    int kv_dim, int max_seq, const int *pos_p, int ntok) {
-    constexpr int NDG = NT / 16, DPL = HD / NDG, NQ = DPL / 4;   // dim groups; dims a lane, NQ quads 4 NDG apart
+// WIN: with a window (a launch without one keeps the shorter loop conditions
+// and 4 waves a SIMD: the 1B-shape prompt step ran 1% slower through the
+// windowed form)
+constexpr int rb_cw(int hd) { return hd == 256 ? 128 : hd; }   // dims of a workgroup
+template <int HD, int KT, bool WIN>
+__global__ void __launch_bounds__(4 * rb_cw(HD)) k_attn_mix_rb(float *ao, const float *att, const KvView kv, int group,
+                                                               int kv_dim, int max_seq, int window_arg,
+                                                               const int *pos_p, int ntok) {
+    const int window = WIN ? window_arg : 0;
+    constexpr int CW = rb_cw(HD), hd = HD;
+    constexpr int NT = 4 * CW, NDG = CW / 4;          // threads; dim groups
     constexpr int AS = RB_T + 4;                      // weight row stride (floats)
-    constexpr int NA = RB_R * RB_T / 4 / NT;          // 4-weight loads a thread stages per tile
-    constexpr int NV = RB_T * HD / 4 / NT;            // 4-element V loads a thread stages per tile
+    constexpr int NW4 = RB_R * RB_T / 4;              // a tile's 4-weight loads
+    constexpr int NA = (NW4 + NT - 1) / NT;           // of them a thread's, at most
+    constexpr int NV = RB_T * CW / 4 / NT;            // 4-element V loads a thread stages per tile
     __shared__ __align__(16) float as[RB_R * AS];
-    __shared__ __align__(16) float vs[RB_T * HD];
+    __shared__ __align__(16) float vs[RB_T * CW];
     const int g = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, dg = tid % NDG, rg = tid / NDG;
     const int nrow = ntok * group, R0 = (gridDim.y - 1 - blockIdx.y) * RB_R;
     const int pos0 = *pos_p, n_heads = gridDim.x * group;
     const int nlast = pos0 + (min(R0 + RB_R, nrow) - 1) / group + 1;   // positions the block's last row attends
-    const int ntl = (nlast + RB_T - 1) / RB_T;
-    const int zw = (R0 + 4 * (64 / NDG) * wave) / group;   // the token of the wave's first row
-    const int zlw = (min(R0 + 4 * (64 / NDG) * (wave + 1), nrow) - 1) / group;   // of its last (within the rows)
+    const int base = attn_first(pos0 + R0 / group, window) / RB_T * RB_T;   // the block's first tile
+    const int ntl = (nlast - base + RB_T - 1) / RB_T, c0 = HD == CW ? 0 : blockIdx.z * CW;
+    const int zw = (R0 + 4 * (64 * wave / NDG)) / group;   // the token of the wave's first row
+    const int zlw = (min(R0 + 4 * ((64 * wave + 63) / NDG + 1), nrow) - 1) / group;   // of its last (within the rows)
+    const int fw = attn_first(pos0 + zw, window), flw = attn_first(pos0 + zlw, window);   // the first positions they attend
     typename Kv4<KT>::T vr[NV];
     float4 ar[NA];
     float dv[NA][4];   // Q8: the V row scales of the staged weights' positions
     auto load = [&](int t0) {
 #pragma unroll
         for (int u = 0; u < NV; u++) {
-            const int e = tid + NT * u, p = e / (HD / 4), c4 = e % (HD / 4);
-            vr[u] = Kv4<KT>::load(kv.v, (size_t)min(t0 + p, nlast - 1) * kv_dim + (size_t)g * HD + 4 * c4);
+            const int e = tid + NT * u, p = e / (CW / 4), c4 = e % (CW / 4);
+            vr[u] = Kv4<KT>::load(kv.v, (size_t)min(t0 + p, nlast - 1) * kv_dim + (size_t)g * hd + c0 + 4 * c4);
         }
 #pragma unroll
         for (int u = 0; u < NA; u++) {
-            const int e = tid + NT * u, rr = e / (RB_T / 4), q4 = e % (RB_T / 4);
+            const int e = min(tid + NT * u, NW4 - 1), rr = e / (RB_T / 4), q4 = e % (RB_T / 4);
             const int R = min(R0 + rr, nrow - 1), z = R / group, j = R - z * group;
             ar[u] = *(const float4 *)(att + ((size_t)z * n_heads + (size_t)g * group + j) * max_seq +
                                       min(t0 + 4 * q4, max_seq - 4));
@@ -1227,23 +1286,24 @@ __global__ void __launch_bounds__(NT) k_attn_mix_rb(float *ao, const float *att,
             }
         }
     };
-    float acc[4][DPL];
+    float acc[4][4];
 #pragma unroll
     for (int r = 0; r < 4; r++)
 #pragma unroll
-        for (int c = 0; c < DPL; c++) acc[r][c] = 0.0f;
-    load(0);
+        for (int c = 0; c < 4; c++) acc[r][c] = 0.0f;
+    load(base);
     for (int ti = 0; ti < ntl; ti++) {
-        const int t0 = ti * RB_T;
+        const int t0 = base + ti * RB_T;
         __syncthreads();   // the last tile is read
 #pragma unroll
         for (int u = 0; u < NV; u++) {
             const int e = tid + NT * u;
-            *(float4 *)(vs + 4 * e) = Kv4<KT>::wide(vr[u]);   // [position][dim]: e = p HD / 4 + c4
+            *(float4 *)(vs + 4 * e) = Kv4<KT>::wide(vr[u]);   // [position][dim]: e = p CW / 4 + c4
         }
 #pragma unroll
         for (int u = 0; u < NA; u++) {
             const int e = tid + NT * u, rr = e / (RB_T / 4), q4 = e % (RB_T / 4);
+            if (NW4 % NT && e >= NW4) break;
             float4 a = ar[u];
             if (KT == KV_Q8)
                 a = make_float4(kr_fmul(a.x, dv[u][0]), kr_fmul(a.y, dv[u][1]), kr_fmul(a.z, dv[u][2]),
@@ -1253,47 +1313,46 @@ __global__ void __launch_bounds__(NT) k_attn_mix_rb(float *ao, const float *att,
         __syncthreads();
         if (ti + 1 < ntl) load(t0 + RB_T);
         const float *ap = as + 4 * rg * AS, *vp = vs + 4 * dg;
-        int lim[4];   // in a masked step: position t0 + k counts for row r iff k <= lim[r]
-#pragma unroll
-        for (int r = 0; r < 4; r++) lim[r] = pos0 + (R0 + 4 * rg + r) / group - t0;
-        // positions t .. t + 3 of the tile, every row's terms (UPTO: each
-        // row's up to its own position)
-        auto step = [&](int t, auto upto) {
-            constexpr bool UPTO = decltype(upto)::value;
+        // positions t .. t + 3 of the tile, every row's terms (OWN: each
+        // row's own positions only)
+        auto step = [&](int t, auto own, const int *lo, const int *lim) {
+            constexpr bool OWN = decltype(own)::value;
             float4 a[4];
 #pragma unroll
             for (int r = 0; r < 4; r++) a[r] = *(const float4 *)(ap + r * AS + t);
 #pragma unroll
             for (int k = 0; k < 4; k++) {
-                float4 v[NQ];
-#pragma unroll
-                for (int q = 0; q < NQ; q++) v[q] = *(const float4 *)(vp + (t + k) * HD + 4 * NDG * q);
+                const float4 x = *(const float4 *)(vp + (t + k) * CW);
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
                     const float w = k == 0 ? a[r].x : k == 1 ? a[r].y : k == 2 ? a[r].z : a[r].w;
-                    const bool in = !UPTO || t + k <= lim[r];
-#pragma unroll
-                    for (int q = 0; q < NQ; q++) {
-                        const float4 x = v[q];
-                        float *o = acc[r] + 4 * q;
-                        o[0] = in ? kr_fadd(o[0], kr_fmul(w, x.x)) : o[0];
-                        o[1] = in ? kr_fadd(o[1], kr_fmul(w, x.y)) : o[1];
-                        o[2] = in ? kr_fadd(o[2], kr_fmul(w, x.z)) : o[2];
-                        o[3] = in ? kr_fadd(o[3], kr_fmul(w, x.w)) : o[3];
-                    }
+                    const bool in = !OWN || (t + k <= lim[r] && (!WIN || t + k >= lo[r]));
+                    float *o = acc[r];
+                    o[0] = in ? kr_fadd(o[0], kr_fmul(w, x.x)) : o[0];
+                    o[1] = in ? kr_fadd(o[1], kr_fmul(w, x.y)) : o[1];
+                    o[2] = in ? kr_fadd(o[2], kr_fmul(w, x.z)) : o[2];
+                    o[3] = in ? kr_fadd(o[3], kr_fmul(w, x.w)) : o[3];
                 }
             }
         };
-        if (t0 + RB_T - 1 <= pos0 + zw) {   // every position counts for every row of the wave
+        if (t0 + RB_T - 1 <= pos0 + zw && (!WIN || t0 >= flw)) {   // every position counts for every row of the wave
 #pragma unroll 2
-            for (int t = 0; t < RB_T; t += 4) step(t, std::false_type{});
+            for (int t = 0; t < RB_T; t += 4) step(t, std::false_type{}, nullptr, nullptr);
         } else {
-            // the tile that holds the wave's own positions: whole steps below
-            // its first row's position, masked steps up to its last row's
+            // a tile that holds the wave's own positions or its windows'
+            // starts: whole steps where every row attends, masked steps
+            // where some do, none outside
             const int full = pos0 + zw - t0, any = pos0 + zlw - t0;
-            for (int t = 0; t < RB_T && t <= any; t += 4) {
-                if (t + 3 <= full) step(t, std::false_type{});
-                else step(t, std::true_type{});
+            int lim[4], lo[4];   // in a masked step: position t0 + k counts for row r iff lo[r] <= k <= lim[r]
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int pr = pos0 + (R0 + 4 * rg + r) / group;
+                lim[r] = pr - t0;
+                lo[r] = attn_first(pr, window) - t0;
+            }
+            for (int t = WIN ? max(0, (fw - t0) / 4 * 4) : 0; t < RB_T && t <= any; t += 4) {
+                if (t + 3 <= full && (!WIN || t >= flw - t0)) step(t, std::false_type{}, nullptr, nullptr);
+                else step(t, std::true_type{}, lo, lim);
             }
         }
     }
@@ -1302,10 +1361,8 @@ __global__ void __launch_bounds__(NT) k_attn_mix_rb(float *ao, const float *att,
         const int R = R0 + 4 * rg + r;
         if (R >= nrow) continue;
         const int z = R / group, j = R - z * group;
-        float *dst = ao + (size_t)z * n_heads * HD + (size_t)(g * group + j) * HD + 4 * dg;
-#pragma unroll
-        for (int q = 0; q < NQ; q++)
-            *(float4 *)(dst + 4 * NDG * q) = make_float4(acc[r][4 * q], acc[r][4 * q + 1], acc[r][4 * q + 2], acc[r][4 * q + 3]);
+        *(float4 *)(ao + ((size_t)z * n_heads + (size_t)g * group + j) * hd + c0 + 4 * dg) =
+            make_float4(acc[r][0], acc[r][1], acc[r][2], acc[r][3]);
     }
 }
 
@@ -1365,22 +1422,33 @@ template <int KT, int DW>
 static void launch_mix(const dim3 &grid, int ntok, float *ao, const float *att, const KvView &kv, int group, int hd,
                        int kv_dim, int max_seq, int window, const int *pos) {
     const float *vc = (const float *)kv.v;
-    if (ntok > 1 && window == 0 && rb_shape(hd, ntok, group, grid.x) && max_seq % 4 == 0) {
-        // prefill without a window, 64- or 128-dim heads: register-blocked rows
-        const dim3 rgrid(grid.x, (ntok * group + RB_R - 1) / RB_R, 1);
-        if (hd == 64)
-            hipLaunchKernelGGL((k_attn_mix_rb<64, KT, 256>), rgrid, dim3(256), 0, kr_stream(), ao, att, kv, group,
-                               kv_dim, max_seq, pos, ntok);
-        else
-            hipLaunchKernelGGL((k_attn_mix_rb<128, KT, RB_NT128>), rgrid, dim3(RB_NT128), 0, kr_stream(), ao, att, kv,
-                               group, kv_dim, max_seq, pos, ntok);
+    const dim3 rgrid(grid.x, (ntok * group + RB_R - 1) / RB_R, rb_dims(hd) ? hd / rb_cw(hd) : 1);
+    if (ntok > 1 && rb_dims(hd) && max_seq % 4 == 0 && rb_fills((long)rgrid.x * rgrid.y * rgrid.z)) {
+        // prefill: register-blocked rows
+        auto go = [&](auto dims) {
+            constexpr int HD = decltype(dims)::value;
+            auto run = [&](auto kern) {
+                hipLaunchKernelGGL(kern, rgrid, dim3(4 * rb_cw(HD)), 0, kr_stream(), ao, att, kv, group, kv_dim,
+                                   max_seq, window, pos, ntok);
+            };
+            if (window) run(k_attn_mix_rb<HD, KT, true>);
+            else run(k_attn_mix_rb<HD, KT, false>);
+        };
+        switch (hd) {
+        case 48: go(std::integral_constant<int, 48>{}); break;
+        case 64: go(std::integral_constant<int, 64>{}); break;
+        case 80: go(std::integral_constant<int, 80>{}); break;
+        case 96: go(std::integral_constant<int, 96>{}); break;
+        case 128: go(std::integral_constant<int, 128>{}); break;
+        default: go(std::integral_constant<int, 256>{}); break;
+        }
         return;
     }
     if constexpr (DW >= 16) {
-        if (ntok > 1 && window == 0) {   // prefill without a window: blocks of MK_W tokens share the V tiles
+        if (ntok > 1) {   // prefill: blocks of MK_W tokens share the V tiles
             const dim3 bgrid(grid.x, grid.y, (ntok + MK_W * MK_U - 1) / (MK_W * MK_U));
             hipLaunchKernelGGL((k_attn_mix_blk<DW, KT>), bgrid, dim3(64 * MK_W), 0, kr_stream(), ao, att, kv, group,
-                               hd, kv_dim, max_seq, pos, ntok);
+                               hd, kv_dim, max_seq, window, pos, ntok);
             return;
         }
     }
@@ -1429,6 +1497,13 @@ static void attention(float *ao, float *att, const float *q, const KvView &kv, i
         return;
     }
     const size_t lds = tile_lds(tt);
+    // positions a row attends, and a block of tb tokens from a tile boundary
+    // (tiles of tp positions), at most
+    const int nrow_max = window && window <= max_pos ? window : max_pos + 1;
+    auto span_tiles = [&](int tb, int tp) {
+        const int all = (max_pos + tp) / tp;
+        return window && window <= max_pos ? std::min(all, (window + tb - 1 + tp - 1 + tp - 1) / tp) : all;
+    };
     const dim3 sgrid(n_kv_heads, (max_pos + tt) / tt, ntok);
     if constexpr (KT == KV_Q8) {
         // prefill: the K tile and the quantized queries of QB tokens in LDS
@@ -1437,18 +1512,22 @@ static void attention(float *ao, float *att, const float *q, const KvView &kv, i
                    (size_t)qb * group * head_dim;
         };
         const int qb = qlds(16) <= 64 * 1024 ? 16 : qlds(8) <= 64 * 1024 ? 8 : qlds(4) <= 64 * 1024 ? 4 : 0;
-        if (ntok > 1 && window == 0 && qb) {
-            const dim3 bgrid(n_kv_heads, (max_pos + AT_T) / AT_T, (ntok + AT_TB - 1) / AT_TB);
+        if (ntok > 1 && qb) {
+            const dim3 bgrid(n_kv_heads, span_tiles(AT_TB, AT_T), (ntok + AT_TB - 1) / AT_TB);
             auto go = [&](auto kern) {
                 hipLaunchKernelGGL(kern, bgrid, dim3(AT_THREADS), qlds(qb), kr_stream(), att, q, kv, group, head_dim,
-                                   kv_dim, max_seq, scale, pos, ntok);
+                                   kv_dim, max_seq, window, scale, pos, ntok);
             };
             if (qb == 16) go(k_attn_scores_blk_q8<16>);
             else if (qb == 8) go(k_attn_scores_blk_q8<8>);
             else go(k_attn_scores_blk_q8<4>);
         } else {
-            hipLaunchKernelGGL(k_attn_scores_q8, sgrid, dim3(AT_THREADS), lds, kr_stream(), att, q, kv, group,
-                               head_dim, kv_dim, max_seq, window, scale, pos);
+            auto go = [&](auto kern) {
+                hipLaunchKernelGGL(kern, sgrid, dim3(AT_THREADS), lds, kr_stream(), att, q, kv, group, head_dim,
+                                   kv_dim, max_seq, window, scale, pos);
+            };
+            if (ntok > 1) go(k_attn_scores_q8<true>);
+            else go(k_attn_scores_q8<false>);
         }
     }
     else {
@@ -1458,20 +1537,41 @@ static void attention(float *ao, float *att, const float *q, const KvView &kv, i
         auto ktile = [&](int tp) { return sizeof(float) * (size_t)tp * (head_dim + 4); };
         auto pick_qb = [&](int tp) { return ktile(tp) + 8 * qtok <= 64 * 1024 ? 8 : ktile(tp) + 4 * qtok <= 64 * 1024 ? 4 : 0; };
         const int tp = pick_qb(AT_T) ? AT_T : AT_T / 2, qb = pick_qb(tp);
-        if (ntok > 1 && window == 0 && rb_shape(head_dim, ntok, group, n_kv_heads)) {   // prefill: register-blocked rows
-            const dim3 rgrid(n_kv_heads, (ntok * group + RB_R - 1) / RB_R, (max_pos + RB_PC * RB_T) / (RB_PC * RB_T));
-            if (head_dim == 64)
-                hipLaunchKernelGGL((k_attn_scores_rb<64, KT, 256>), rgrid, dim3(256), 0, kr_stream(), att, q, kv,
-                                   group, kv_dim, max_seq, scale, pos, ntok);
-            else
-                hipLaunchKernelGGL((k_attn_scores_rb<128, KT, RB_NT128>), rgrid, dim3(RB_NT128), 0, kr_stream(), att,
-                                   q, kv, group, kv_dim, max_seq, scale, pos, ntok);
-        } else if (ntok > 1 && window == 0 && qb) {   // prefill: blocks of AT_TB tokens share a K tile
-            const dim3 bgrid(n_kv_heads, (max_pos + tp) / tp, (ntok + AT_TB - 1) / AT_TB);
+        // the register-blocked scores: a workgroup's K tiles are cut until
+        // the grid fills the device
+        const int rtiles = span_tiles((RB_R - 1) / group + 2, RB_T), rblk = n_kv_heads * ((ntok * group + RB_R - 1) / RB_R);
+        int pc = RB_PC;
+        while (pc > 1 && !rb_fills((long)rblk * ((rtiles + pc - 1) / pc) / 2)) pc /= 2;
+        const dim3 rgrid(n_kv_heads, rblk / n_kv_heads, (rtiles + pc - 1) / pc);
+        if (ntok > 1 && rb_dims(head_dim) && rb_fills((long)rblk * rgrid.z)) {   // prefill: register-blocked rows
+            auto go = [&](auto dims, auto threads, auto slice) {
+                constexpr int HD = decltype(dims)::value, NT = decltype(threads)::value, HS = decltype(slice)::value;
+                auto run = [&](auto kern) {
+                    hipLaunchKernelGGL(kern, rgrid, dim3(NT), 0, kr_stream(), att, q, kv, group, kv_dim, max_seq,
+                                       window, scale, pos, ntok, pc);
+                };
+                if (window) run(k_attn_scores_rb<HD, KT, NT, true, HS>);
+                else run(k_attn_scores_rb<HD, KT, NT, false, HS>);
+            };
+            using std::integral_constant;
+            const integral_constant<int, 256> t256{};
+            const integral_constant<int, 64> d64{};
+            switch (head_dim) {
+            case 48: go(integral_constant<int, 48>{}, t256, integral_constant<int, 48>{}); break;
+            case 64: go(d64, t256, d64); break;
+            case 80: go(integral_constant<int, 80>{}, t256, integral_constant<int, 80>{}); break;
+            case 96: go(integral_constant<int, 96>{}, t256, integral_constant<int, 96>{}); break;
+            case 128:
+                go(integral_constant<int, 128>{}, integral_constant<int, RB_NT128>{}, integral_constant<int, 128>{});
+                break;
+            default: go(t256, t256, d64); break;
+            }
+        } else if (ntok > 1 && qb) {   // prefill: blocks of AT_TB tokens share a K tile
+            const dim3 bgrid(n_kv_heads, span_tiles(AT_TB, tp), (ntok + AT_TB - 1) / AT_TB);
             const size_t blds = ktile(tp) + qb * qtok;
             auto go = [&](auto kern) {
                 hipLaunchKernelGGL(kern, bgrid, dim3(AT_THREADS), blds, kr_stream(), att, q, kv, group, head_dim,
-                                   kv_dim, max_seq, scale, pos, ntok);
+                                   kv_dim, max_seq, window, scale, pos, ntok);
             };
             if (tp != AT_T) {
                 if (qb == 8) go(k_attn_scores_blk<0, 8, KT, AT_T / 2>);
@@ -1485,39 +1585,49 @@ static void attention(float *ao, float *att, const float *q, const KvView &kv, i
                 else if (head_dim == 64) go(k_attn_scores_blk<64, 4, KT>);
                 else go(k_attn_scores_blk<0, 4, KT>);
             }
-        } else if (KT != KV_F32) {
-            if (tt == AT_T)
-                hipLaunchKernelGGL((k_attn_scores_kv<KT, AT_T>), sgrid, dim3(AT_THREADS), lds, kr_stream(), att, q, kv,
-                                   group, head_dim, kv_dim, max_seq, window, scale, pos);
-            else
-                hipLaunchKernelGGL((k_attn_scores_kv<KT, AT_TD>), sgrid, dim3(AT_THREADS), lds, kr_stream(), att, q,
-                                   kv, group, head_dim, kv_dim, max_seq, window, scale, pos);
-        } else if (ntok == 1 || tt == AT_TD) {   // decode (or a wide head): tiles of AT_TD positions
-            const dim3 dgrid(n_kv_heads, (max_pos + AT_TD) / AT_TD, ntok);
-            hipLaunchKernelGGL(k_attn_scores<AT_TD>, dgrid, dim3(AT_THREADS), tile_lds(AT_TD), kr_stream(), att, q,
-                               (const float *)kv.k, group, head_dim, kv_dim, max_seq, window, scale, pos);
         } else {
-            hipLaunchKernelGGL(k_attn_scores<AT_T>, sgrid, dim3(AT_THREADS), lds, kr_stream(), att, q,
-                               (const float *)kv.k, group, head_dim, kv_dim, max_seq, window, scale, pos);
+            auto go = [&](auto kern, const dim3 &grid, size_t bytes, auto *k) {
+                hipLaunchKernelGGL(kern, grid, dim3(AT_THREADS), bytes, kr_stream(), att, q, k, group, head_dim,
+                                   kv_dim, max_seq, window, scale, pos);
+            };
+            auto gokv = [&](auto kern) {
+                hipLaunchKernelGGL(kern, sgrid, dim3(AT_THREADS), lds, kr_stream(), att, q, kv, group, head_dim,
+                                   kv_dim, max_seq, window, scale, pos);
+            };
+            const float *k32 = (const float *)kv.k;
+            const dim3 dgrid(n_kv_heads, (max_pos + AT_TD) / AT_TD, ntok);
+            if (KT != KV_F32) {
+                if (tt == AT_T) { if (ntok > 1) gokv(k_attn_scores_kv<KT, AT_T, true>); else gokv(k_attn_scores_kv<KT, AT_T>); }
+                else { if (ntok > 1) gokv(k_attn_scores_kv<KT, AT_TD, true>); else gokv(k_attn_scores_kv<KT, AT_TD>); }
+            } else if (ntok == 1) {   // decode: tiles of AT_TD positions
+                go(k_attn_scores<AT_TD>, dgrid, tile_lds(AT_TD), k32);
+            } else if (tt == AT_TD) {   // a wide head
+                go(k_attn_scores<AT_TD, true>, dgrid, tile_lds(AT_TD), k32);
+            } else {
+                go(k_attn_scores<AT_T, true>, sgrid, lds, k32);
+            }
         }
     }
-    if (cap > 0.0f) krh_softcap_att(att, n_heads, max_seq, window, pos, ntok, cap);   // ops/ops.c:141
-    if (ntok > 1 && max_pos + 1 > SM_WN / 2 && max_pos + 1 <= 4096) {
+    if (cap > 0.0f) kr_softcap_scores(att, n_heads, max_seq, window, pos, ntok, cap);   // ops/ops.c:141
+    if (ntok > 1 && nrow_max > SM_WN / 2 && nrow_max <= 4096) {
         // prefill rows of 2049 to 4096 scores: a 256-thread workgroup each
         // (measured: 1B-shape 4000-token prompt 59.9k -> 61.7k tok/s; rows
         // up to 2048 run faster one wave each), the ordered sum's lean form
         // (90 VGPRs against 111: 5 waves a SIMD; 64.5k -> 65.5k)
         hipLaunchKernelGGL((k_attn_softmax<256, 4096, true>), dim3(n_heads, 1, ntok), dim3(256), 0, kr_stream(), att,
                            max_seq, window, pos);
-    } else if (ntok > 1 && max_pos + 1 <= SM_WN / 2) {   // prefill rows of up to 2048 scores: one wave each
-        const int tcap = sc_terms_cap(max_pos + 1), scr = (sc_lds_bytes(max_pos + 1, 64) + 15) / 16 * 16;
+    } else if (ntok > 1 && nrow_max <= SM_WN / 2) {   // prefill rows of up to 2048 scores: one wave each
+        const int tcap = sc_terms_cap(nrow_max), scr = (sc_lds_bytes(nrow_max, 64) + 15) / 16 * 16;
         const size_t per_wave = 4 * (size_t)tcap + scr;
         const int nrows = n_heads * ntok;
         hipLaunchKernelGGL((k_attn_softmax_rows<4, SM_V / 2>), dim3((nrows + 3) / 4), dim3(256), 4 * per_wave,
                            kr_stream(), att, n_heads, max_seq, window, pos, nrows, tcap, scr);
     } else {
-        hipLaunchKernelGGL((k_attn_softmax<SMX_THREADS, AT_CHUNK>), dim3(n_heads, 1, ntok), dim3(SMX_THREADS), 0, kr_stream(), att, max_seq,
-                           window, pos);
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3(n_heads, 1, ntok), dim3(SMX_THREADS), 0, kr_stream(), att, max_seq, window, pos);
+        };
+        if (ntok > 1) go(k_attn_softmax<SMX_THREADS, AT_CHUNK, false, true>);
+        else go(k_attn_softmax<SMX_THREADS, AT_CHUNK>);
     }
     const int gp = group <= 1 ? 1 : group <= 2 ? 2 : group <= 4 ? 4 : group <= 8 ? 8 : 16;
     const int dw = 64 / gp;

@@ -49,10 +49,11 @@ __global__ void __launch_bounds__(64) k_heads_norm_rope(float *q, float *k, cons
 // cap * tanhf(score / cap) before the softmax. Row (token z, head x) holds
 // max_seq floats; its length follows from the position and the window as
 // the score kernels count it.
-__global__ void k_softcap_att(float *att, int max_seq, int window, const int *pos_p, float cap) {
+// row0: a row's scores start at its first position's index, else at 0
+__global__ void k_softcap_att(float *att, int max_seq, int window, const int *pos_p, float cap, int row0) {
     const int pos = *pos_p + (int)blockIdx.z;
     const int first = window && pos >= window ? pos + 1 - window : 0, n = pos + 1 - first;
-    float *a = att + ((size_t)blockIdx.z * gridDim.x + blockIdx.x) * max_seq;
+    float *a = att + ((size_t)blockIdx.z * gridDim.x + blockIdx.x) * max_seq + (row0 ? first : 0);
     for (int t = (int)threadIdx.x; t < n; t += (int)blockDim.x) a[t] = kr_fmul(cap, kr_tanhf(kr_fdiv(a[t], cap)));
 }
 
@@ -103,7 +104,15 @@ extern "C" void krh_softcap_att(float *att, int n_heads, int max_seq, int window
         return;
     }
     hipLaunchKernelGGL(k_softcap_att, dim3(n_heads, 1, ntok), dim3(256), 0, kr_stream(), att, max_seq, window, pos,
-                       cap);
+                       cap, 0);
+    kr_check_launch("softcap_att");
+}
+
+// the same over the attention launches' own layout: a batch's rows start at
+// their first position's index (kr_attn.hip, attn_row0)
+void kr_softcap_scores(float *att, int n_heads, int max_seq, int window, const int *pos, int ntok, float cap) {
+    hipLaunchKernelGGL(k_softcap_att, dim3(n_heads, 1, ntok), dim3(256), 0, kr_stream(), att, max_seq, window, pos,
+                       cap, ntok > 1);
     kr_check_launch("softcap_att");
 }
 

@@ -13,3 +13,6 @@ void kr_check_launch(const char *what);
 constexpr int KR_MAX_DEVICES = 16;
 // kr_attn.hip: takes this device's address of the attention scratch array
 ml_status kr_attn_setup(int dev);
+// kr_family.hip: soft-caps the attention scratch's scores in place, in the
+// layout the attention launches of ntok tokens use
+void kr_softcap_scores(float *att, int n_heads, int max_seq, int window, const int *pos, int ntok, float cap);

@@ -196,6 +196,61 @@ def kv_batch_case(dev, kv_type, nh, nkv, hd, pos0, T, window):
         assert np.array_equal(bits(got[t]), bits(out)), t
 
 
+# tile edges: windows around a 64-position tile, a first token with and
+# without a whole window behind it, one row and a ragged last row block, every
+# head size of the register-blocked kernels and one only the others take
+@pytest.mark.parametrize("kv_type", [K.ML_F32, K.ML_F16, K.ML_Q8_0])
+@pytest.mark.parametrize("nh,nkv,hd,pos0,T,window", [(4, 2, 48, 130, 67, 64), (3, 1, 64, 300, 65, 63),
+                                                     (8, 2, 80, 0, 70, 33), (4, 4, 96, 190, 33, 65),
+                                                     (6, 2, 128, 64, 2, 1), (4, 2, 256, 200, 37, 128),
+                                                     (2, 1, 256, 40, 90, 0), (6, 2, 96, 3, 80, 0),
+                                                     (4, 2, 32, 100, 50, 40), (8, 1, 64, 400, 112, 200)])
+@pytest.mark.parametrize("choice", [0, 1 << 30])
+def test_attention_batch_blocks(dev, kv_type, nh, nkv, hd, pos0, T, window, choice):
+    """batched attention with the register-blocked kernels for every grid
+    (choice 0) and for none, over a scratch and unattended cache rows of NaN
+    (Q8: scales), against the oracle's per-token attention"""
+    max_seq = 512
+    kvd, qd = nkv * hd, nh * hd
+    Q = f32(RNG.normal(0, 1, (T, qd)))
+    lo, hi = (pos0 + 1 - window if window and pos0 >= window else 0), pos0 + T
+    if kv_type == K.ML_F32:
+        k, v = f32(RNG.normal(0, 1, max_seq * kvd)), f32(RNG.normal(0, 1, max_seq * kvd))
+        kd = vd = None
+        bad, width = (k, v), kvd
+    else:
+        k, v, kd, vd = rand_cache(kv_type, max_seq, kvd, nkv)
+        bad, width = ((k, v), kvd) if kv_type == K.ML_F16 else ((kd, vd), nkv)
+    nan = 0x7E00 if kv_type == K.ML_F16 else np.nan
+    for a in bad:
+        a[:lo * width] = nan
+        a[hi * width:] = nan
+    if kv_type == K.ML_F32:
+        dview = K.MlKvLayer(dev.put(k).ptr, dev.put(v).ptr, None, None, None, None, window, None, None)
+        hview = O.KvLayer(k.ctypes.data, v.ctypes.data, None, None, None, None, window, None, None)
+    else:
+        dview, hview = views(dev, kv_type, k, v, kd, vd, window)
+    scale = float(np.float32(1.0) / np.sqrt(np.float32(hd)))
+    ao, att = dev.zeros(4 * T * qd), dev.put(np.full(T * nh * max_seq, np.nan, np.float32))
+    K.hip.krh_set_attn_rb_min(choice)
+    try:
+        K.hip.krh_attention_kv(ao.ptr, att.ptr, dev.put(Q).ptr, C.byref(dview), nh, nkv, hd, max_seq, scale,
+                               dev.put(np.array([pos0], np.int32)).ptr, T, pos0 + T - 1)
+        ok()
+    finally:
+        K.hip.krh_set_attn_rb_min(512)
+    got = ao.get(np.float32, T * qd).reshape(T, qd)
+    cfg = K.MlConfig(n_heads=nh, n_kv_heads=nkv, head_dim=hd, kv_dim=kvd, q_dim=qd, max_seq=max_seq,
+                     attn_scale=scale)
+    scratch = np.zeros(max_seq, np.float32)
+    for t in range(T):
+        out = np.zeros(qd, np.float32)
+        qt = f32(Q[t])
+        oracle.kro_attention(out.ctypes.data, qt.ctypes.data, C.byref(hview), scratch.ctypes.data, C.byref(cfg),
+                             pos0 + t)
+        assert np.array_equal(bits(got[t]), bits(out)), t
+
+
 KV = {"f16": K.ML_F16, "q8": K.ML_Q8_0}
 
 
