@@ -12,9 +12,9 @@
 // result register r of lane l is C[8 (r / 4) + 4 (l / 32) + r % 4][l % 32].
 // A = the tokens' activations, B = the weight rows, so each lane holds one
 // weight row (one scale per block) and 16 tokens, whose scales come from the
-// transposed activation scales xdT[b][t] through the workgroup's LDS tile. The per-block rescale and the
-// ordered accumulation are 4 unfused VALU operations per output and block,
-// which bound the kernel, not the MFMA.
+// transposed activation scales xdT[b][t] through the workgroup's LDS tile. The
+// per-block rescale and the ordered accumulation are 3 VALU operations per
+// output and block (f32 scales: 4), which bound the kernel, not the MFMA.
 #include "kr_internal.h"
 #include "kr_numerics.h"
 
@@ -45,166 +45,519 @@ struct MmArgs {
     const float *bias[3];
     const float *rope_cos, *rope_sin;
     int head_dim, pos0;
-    int ng;              // row groups per wave (the kernel's NG)
-    int tw;              // waves per workgroup (the kernel's TW): 32 TW tokens a workgroup
+    int ng, rg;          // row groups per wave: NG of k_matmul, or with ng 1 RG of k_matmul_short
     int8_t *hq;          // MM_SWIGLU: h's Q8_0 quants [T][rows] and scales [rows / 32][ldx]
     float *hdT;
 };
 
-constexpr int MM_TT = 128;   // tokens per workgroup
-
-// 16 signed quant bytes of half h (elements 16h .. 16h+15) of a weight block
-template <int QT>
-__device__ __forceinline__ v4i weight_frag(const uint8_t *blk, int h) {
-    if (QT == ML_Q8_0) {
-        const int4 v = *(const int4 *)(blk + 16 * h);
-        return v4i{ v.x, v.y, v.z, v.w };
-    }
-    // byte p of a Q4 block holds element p (low nibble) and p + 16 (high);
-    // nibble n is weight n - 8: (n | 0x80) - 8 never borrows across bytes,
-    // and ^ 0x80 then leaves n - 8 as a signed byte
-    const int4 v = *(const int4 *)blk;
+// the 16 signed quant bytes of elements 16h .. 16h + 15 of a Q4 block: byte p
+// holds element p (low nibble) and p + 16 (high); nibble n is weight n - 8:
+// (n | 0x80) - 8 never borrows across bytes, and ^ 0x80 then leaves n - 8 as
+// a signed byte
+__device__ __forceinline__ v4i q4_frag(const v4i v, int h) {
     const unsigned sh = 4u * (unsigned)h, M = 0x0F0F0F0Fu;
     v4i r;
-    r.x = (int)((((((unsigned)v.x >> sh) & M) | 0x80808080u) - 0x08080808u) ^ 0x80808080u);
-    r.y = (int)((((((unsigned)v.y >> sh) & M) | 0x80808080u) - 0x08080808u) ^ 0x80808080u);
-    r.z = (int)((((((unsigned)v.z >> sh) & M) | 0x80808080u) - 0x08080808u) ^ 0x80808080u);
-    r.w = (int)((((((unsigned)v.w >> sh) & M) | 0x80808080u) - 0x08080808u) ^ 0x80808080u);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        r[i] = (int)((((((unsigned)v[i] >> sh) & M) | 0x80808080u) - 0x08080808u) ^ 0x80808080u);
     return r;
 }
 
-// A wave computes NG row groups x 1 token group of 32 (NG MFMA tiles per
-// block); the workgroup's 4 waves take 4 token groups of the same 32 NG rows.
-// NG = 4 when the grid of 128-row tiles fills the device (long prompts);
-// NG = 1 gives four times the workgroups for short batches (the reference's
-// 128-token prefill steps), whose few 128-row tiles would leave most CUs idle
-// with each tile's VALU work in series.
-
-// Per wave and block: the wave's 32 tokens.
-struct XFrag {
-    v4i xa;              // the wave's 32 tokens
-};
-
-// Per thread and block, for the workgroup's tile: 16 quant bytes of weight
-// row tid / 2 (half tid % 2, Q4 unpacked to n - 8), that row's raw scale, and
-// the scale of the workgroup's token tid % 128.
-struct WReg {
-    v4i w;
-    uint32_t d;
-    float xs;
-};
-
-constexpr int MM_ST = 3;   // LDS ring stages of the weight tile
-constexpr int MM_PD = 8;   // NG = 1: blocks of load lookahead (even: the LDS stage of step k is k % 2)
-
-template <int NG, int TT>
-struct MmLds {
-    v4i w[MM_ST][32 * NG][2];     // [stage][row][half]
-    uint32_t d[MM_ST][32 * NG];   // [stage][row] raw scale bits
-    float xs[MM_ST][TT];          // [stage][token] the tokens' scales
-};
-
-__device__ __forceinline__ void x_load(XFrag &f, const MmArgs &a, int b, int tokl, int lane) {
-    const int t = tokl + (lane & 31);   // readable: the caller pads the activations to ldx rows
-    const int4 v = *(const int4 *)(a.xq + (size_t)t * a.K + (size_t)b * 32 + 16 * (lane >> 5));
-    f.xa = v4i{ v.x, v.y, v.z, v.w };
+// f16 scales: the MFMA's accumulator starts at the bits of the float
+// M = 1.5 * 2^23, so a result register holds the bits of the float M + S
+// exactly (|S| <= 32 * 128 * 127 < 2^22), and fl(S * wd) is one
+// fma(M + S, wd, -M * wd): -M * wd is exact (3 times an 11-bit scale), so the
+// fma's exact value is S * wd and it rounds once, as the product does. (S = 0
+// gives +0 where the product has wd's sign; a sum that starts from +0 cannot
+// tell.) That takes the conversion out: 3 VALU operations an output and block
+// instead of 4. An infinite scale is the one value it does not hold for: the
+// FAST loops collect the scales' largest magnitude, and a workgroup that met
+// an infinity sums its tile again with the conversion. f32 scales (M * wd
+// would round) always convert.
+constexpr int MM_MAGIC = 0x4B400000;      // the bits of M
+constexpr float MM_M = 12582912.0f;
+__device__ __forceinline__ v16i mm_magic() {
+    constexpr int m = MM_MAGIC;
+    return v16i{ m, m, m, m, m, m, m, m, m, m, m, m, m, m, m, m };
 }
 
-// thread tid loads half tid % 2 of tile row (tid / 2) mod 32 NG (for NG < 4
-// the surplus threads repeat a row's load, which keeps every load
-// unconditional; only the first 64 NG store it)
-// (xcol: the scales of this thread's token, tid % TT of the workgroup's,
-// clamped to the last token; threads TT.. repeat thread tid % TT's load,
-// unused; xsb: the stride from block to block). PAIR (NG
-// 4): tile rows 0-63 are rows rowl.. of W, tile rows 64-127 the same rows of
-// W2 (SwiGLU's w1 and w3).
-template <int QT, int D16, int NG, int TT, bool PAIR = false>
-__device__ __forceinline__ void w_load(WReg &R, const MMat &W, const float *xcol, int xsb, int nb, int b, int rowl,
-                                       int tid, const MMat &W2 = MMat{}) {
-    const int tr = (tid >> 1) & (32 * NG - 1);
-    int r = rowl + (PAIR ? tr & 63 : tr);
-    r = r < W.rows ? r : W.rows - 1;   // rows past the end re-read the last row (not stored)
-    const size_t blk = (size_t)r * nb + b;
-    const uint8_t *wq = PAIR && tr >= 64 ? W2.q : W.q;
-    const void *wd = PAIR && tr >= 64 ? W2.d : W.d;
-    R.w = weight_frag<QT>(wq + blk * (QT == ML_Q8_0 ? 32 : 16), tid & 1);
-    R.d = D16 ? (uint32_t)((const uint16_t *)wd)[blk] : ((const uint32_t *)wd)[blk];
-    R.xs = xcol[(size_t)b * xsb];
+constexpr int MM_TT = 128;   // tokens per workgroup
+
+template <int D16> struct MmScale { using T = uint32_t; };
+template <> struct MmScale<1> { using T = uint16_t; };
+
+// The sum of row `row` and token t of matrix mi, stored as the launch asks;
+// lanes 2 i and 2 i + 1 hold neighbouring rows of one token.
+template <int EPI>
+__device__ __forceinline__ void mm_emit(const MmArgs &a, int mi, int rows, int row, int t, float v) {
+    float *Y = mi == 0 ? a.y[0] : (mi == 1 ? a.y[1] : a.y[2]);
+    const int ldy = mi == 0 ? a.ldy[0] : (mi == 1 ? a.ldy[1] : a.ldy[2]);
+    const bool rin = row < rows;
+    if (EPI == MM_QKV) {
+        // bias (model/transformer.c:276-277), then RoPE on q and k
+        // (k_scalar.c:79-94): rows 2i, 2i+1 sit in lanes 2i, 2i+1
+        const float *bias = mi == 0 ? a.bias[0] : (mi == 1 ? a.bias[1] : a.bias[2]);
+        if (bias && rin) v = kr_fadd(v, bias[row]);
+        const float o = __shfl_xor(v, 1);
+        if (mi < 2) {
+            const int hd = a.head_dim, j = row % hd, h2 = hd >> 1;
+            const int pos = a.pos0 + (t < a.T ? t : 0);
+            const float c = a.rope_cos[(size_t)pos * h2 + (j >> 1)];
+            const float sn = a.rope_sin[(size_t)pos * h2 + (j >> 1)];
+            v = (j & 1) == 0 ? kr_fsub(kr_fmul(v, c), kr_fmul(o, sn)) : kr_fadd(kr_fmul(o, sn), kr_fmul(v, c));
+        }
+    }
+    if (rin && t < a.T) {
+        float *p = Y + (size_t)t * ldy + row;
+        if (EPI == MM_ADD) *p = kr_fadd(*p, v);
+        else *p = v;
+    }
 }
 
-template <int NG, int TT>
-__device__ __forceinline__ void w_store(MmLds<NG, TT> &L, int st, const WReg &R, int tid) {
-    if (tid < TT) L.xs[st][tid] = R.xs;
-    if ((tid >> 1) >= 32 * NG) return;
-    L.w[st][tid >> 1][tid & 1] = R.w;
-    if ((tid & 1) == 0) L.d[st][tid >> 1] = R.d;
+// ---- 128- and 64-row tiles: MM_SB blocks a stage ----
+//
+// A stage is MM_SB = 4 blocks: 128 bytes of every weight and token row, so
+// the 8 lanes that load a row's stage use whole cache lines at once. (One
+// block a step, the 32 bytes of 32 rows a load instruction touched cost 4
+// times the lines, and the L1 could not keep them until the next block.) Rows
+// are 144 bytes apart in LDS: the 16-byte fragment reads of 16 consecutive
+// rows then fall on distinct banks. Two stages alternate, one barrier each;
+// the next stage's loads are in flight while a stage is summed.
+constexpr int MM_SB = 4, MM_RC = 2 * MM_SB + 1;   // blocks a stage; 16-byte chunks a staged row (one of padding)
+
+template <int NG, int D16>
+struct MmStage {
+    v4i w[32 * NG][MM_RC];
+    v4i x[MM_TT][MM_RC];
+    float xs[MM_SB][MM_TT];                    // token scales
+    typename MmScale<D16>::T d[32 * NG][MM_SB];   // raw weight scales
+};
+
+// a thread's share of a stage in registers
+template <int QT, int NG>
+struct MmPre {
+    v4i w[QT == ML_Q8_0 ? NG : NG / 2], x[4];
+    uint32_t d[NG / 2];
+    float xs[2];
+};
+
+// wave-uniform bases of the tile's operands at block 0 (w, d: of the first
+// and, for a SwiGLU pair, the second 64 rows' matrix) and this thread's byte
+// offsets from them
+template <int NG>
+struct MmTile {
+    const uint8_t *w[2], *d[2], *xs, *x;
+    uint32_t wo[NG], so[NG / 2], xo, xso, xstep;
+    size_t xsb;
+    int nb;
+};
+
+template <int QT, int D16, int NG, bool PAIR>
+__device__ __forceinline__ MmTile<NG> mm_tile(const MmArgs &a, const MMat &W, const MMat &W2, int nb, int rowl,
+                                              int tok0, int tid) {
+    constexpr int BB = QT == ML_Q8_0 ? 32 : 16, SB = D16 ? 2 : 4;
+    MmTile<NG> t;
+    const size_t blk = (size_t)rowl * nb;
+    t.w[0] = W.q + blk * BB;
+    t.w[1] = (PAIR ? W2.q : W.q) + blk * BB;
+    t.d[0] = (const uint8_t *)W.d + blk * SB;
+    t.d[1] = (const uint8_t *)(PAIR ? W2.d : W.d) + blk * SB;
+    // rows past the end re-read the last row (not stored)
+    auto row = [&](int r) { return (uint32_t)(min(rowl + (PAIR ? r & 63 : r), W.rows - 1) - rowl); };
+#pragma unroll
+    for (int u = 0; u < NG; u++)   // Q8: 8 threads a row; Q4: 4
+        t.wo[u] = QT == ML_Q8_0 ? row((tid >> 3) + 32 * u) * nb * BB : row((tid >> 2) + 64 * (u & (NG / 2 - 1))) * nb * BB;
+#pragma unroll
+    for (int u = 0; u < NG / 2; u++) t.so[u] = row((tid >> 2) + 64 * u) * nb * SB;
+    t.xs = (const uint8_t *)(a.xdT + (size_t)tok0 * a.xst);
+    t.xso = (uint32_t)(min(tok0 + (tid & (MM_TT - 1)), a.T - 1) - tok0) * a.xst * 4;
+    t.xsb = (size_t)a.xsb * 4;
+    t.x = (const uint8_t *)a.xq + (size_t)tok0 * a.K;   // readable: the caller pads to ldx rows
+    t.xo = (uint32_t)(tid >> 3) * a.K;
+    t.xstep = 32u * a.K;
+    t.nb = nb;
+    return t;
 }
 
-// Row group g + 1's MFMA is issued after the whole rescale of group g: an
-// empty asm takes every rescaled value of group g as input and the MFMA's
-// weight operand as in-out, so only one 16-register result set is live.
-// Left to itself the compiler issues all NG MFMAs of a step together and
-// holds NG result sets (64 VGPRs at NG 4: 183 VGPRs, 2 waves per SIMD);
-// with one set the kernel takes 146 VGPRs and runs 3 waves per SIMD, whose
-// interleaving hides the MFMA latency the wave itself now waits out (8B-shape
-// prefill 22.0k -> 23.0k tok/s; an MFMA lookahead of half a group, or 4
-// waves per SIMD, spills). The 16 token scales a lane needs
-// (tokens 8 (r / 4) + 4 (lane / 32) + r % 4 of the wave's 32: the same for
-// the 32 lanes of a half-wave) are four 16-byte LDS broadcast reads of the
-// tile's token scales (16 cross-lane shuffles of one loaded scale per lane
-// cost 3-6% more time). The weight fragments and scales come from the
-// workgroup's LDS tile as well.
-template <int D16, int NG, int TT>
-__device__ __forceinline__ void mm_step(float (&acc)[NG][16], const XFrag &f, const MmLds<NG, TT> &L, int st, int lane,
-                                        int tokw) {
-    const int ln = lane & 31, hf = lane >> 5;
+// the stage at block b0; blocks past the last re-read the last (unused)
+template <int QT, int D16, int NG, bool PAIR>
+__device__ __forceinline__ void mm_load(MmPre<QT, NG> &R, const MmTile<NG> &t, int b0, int tid) {
+    const int left = t.nb - b0;
+    const uint32_t c8 = 16 * min(tid & 7, 2 * left - 1), c4 = min(tid & 3, left - 1);
+    if constexpr (QT == ML_Q8_0) {
+#pragma unroll
+        for (int u = 0; u < NG; u++) R.w[u] = *(const v4i *)(t.w[PAIR && u >= NG / 2] + (size_t)b0 * 32 + (t.wo[u] + c8));
+    } else {
+#pragma unroll
+        for (int u = 0; u < NG / 2; u++) R.w[u] = *(const v4i *)(t.w[PAIR && u] + (size_t)b0 * 16 + (t.wo[u] + 16 * c4));
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) R.x[u] = *(const v4i *)(t.x + (size_t)b0 * 32 + (size_t)u * t.xstep + (t.xo + c8));
+#pragma unroll
+    for (int u = 0; u < NG / 2; u++) {
+        const uint8_t *d = t.d[PAIR && u] + (size_t)b0 * (D16 ? 2 : 4);
+        R.d[u] = D16 ? (uint32_t)*(const uint16_t *)(d + (t.so[u] + 2 * c4)) : *(const uint32_t *)(d + (t.so[u] + 4 * c4));
+    }
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+        R.xs[u] = *(const float *)(t.xs + (size_t)(b0 + min((tid >> 7) + 2 * u, left - 1)) * t.xsb + t.xso);
+}
+
+template <int QT, int D16, int NG>
+__device__ __forceinline__ void mm_put(MmStage<NG, D16> &L, const MmPre<QT, NG> &R, int tid) {
+    if constexpr (QT == ML_Q8_0) {
+#pragma unroll
+        for (int u = 0; u < NG; u++) L.w[(tid >> 3) + 32 * u][tid & 7] = R.w[u];
+    } else {
+#pragma unroll
+        for (int u = 0; u < NG / 2; u++) {
+            L.w[(tid >> 2) + 64 * u][2 * (tid & 3)] = q4_frag(R.w[u], 0);
+            L.w[(tid >> 2) + 64 * u][2 * (tid & 3) + 1] = q4_frag(R.w[u], 1);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) L.x[(tid >> 3) + 32 * u][tid & 7] = R.x[u];
+#pragma unroll
+    for (int u = 0; u < NG / 2; u++) L.d[(tid >> 2) + 64 * u][tid & 3] = (typename MmScale<D16>::T)R.d[u];
+#pragma unroll
+    for (int u = 0; u < 2; u++) L.xs[(tid >> 7) + 2 * u][tid & (MM_TT - 1)] = R.xs[u];
+}
+
+// where a lane reads a block's operands in a stage; stepped from block to
+// block, the row groups at constant offsets
+template <int D16>
+struct MmAt {
+    const v4i *w, *x;
+    const float4 *xs;
+    const typename MmScale<D16>::T *d;
+    __device__ __forceinline__ void next() {
+        w += 2;
+        x += 2;
+        xs += MM_TT / 4;
+        d += 1;
+    }
+};
+
+// the next block of a stage for the wave's 32 tokens
+template <int D16, int NG, bool FAST>
+__device__ __forceinline__ void mm_block(float (&acc)[NG][16], float &mx, const v16i &s0, const MmAt<D16> &p) {
+    const v4i xa = *p.x;
     v4i wb[NG];
     uint32_t wdr[NG];
 #pragma unroll
     for (int g = 0; g < NG; g++) {
-        wb[g] = L.w[st][32 * g + ln][hf];
-        wdr[g] = L.d[st][32 * g + ln];
+        wb[g] = p.w[32 * MM_RC * g];
+        wdr[g] = p.d[32 * MM_SB * g];
     }
     float xd[16];
-    const float4 *xv = (const float4 *)&L.xs[st][tokw + 4 * hf];
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-        const float4 v = xv[2 * q];   // tokens 8 q + 4 hf .. + 3
+        const float4 v = p.xs[2 * q];   // tokens 8 q + 4 hf .. + 3
         xd[4 * q] = v.x;
         xd[4 * q + 1] = v.y;
         xd[4 * q + 2] = v.z;
         xd[4 * q + 3] = v.w;
     }
-    v16i s = __builtin_amdgcn_mfma_i32_32x32x32_i8(f.xa, wb[0], v16i{}, 0, 0, 0);
-    // one row group: the loads around the step stay on their side of its
-    // MFMA (measured 10% faster on the 32-row tiles than a free schedule)
-    if constexpr (NG == 1) __builtin_amdgcn_sched_barrier(0);
+    v16i s = __builtin_amdgcn_mfma_i32_32x32x32_i8(xa, wb[0], s0, 0, 0, 0), sn = s;
 #pragma unroll
     for (int g = 0; g < NG; g++) {
-        const float wd = D16 ? kr_h2f((uint16_t)wdr[g]) : __uint_as_float(wdr[g]);
-#pragma unroll
-        for (int r = 0; r < 16; r++)
-            acc[g][r] = kr_fadd(acc[g][r], kr_fmul(kr_fmul((float)s[r], wd), xd[r]));
-        if (g + 1 < NG) {
-            v4i w = wb[g + 1];
-#pragma unroll
-            for (int r = 0; r < 16; r++) asm volatile("" : "+v"(w) : "v"(acc[g][r]));
-            s = __builtin_amdgcn_mfma_i32_32x32x32_i8(f.xa, w, v16i{}, 0, 0, 0);
+        float wd = D16 ? kr_h2f((uint16_t)wdr[g]) : __uint_as_float(wdr[g]);
+        float c = 0.0f;
+        if constexpr (FAST) {
+            asm volatile("" : "+v"(wd));   // a register: no fma_mix from the half
+            mx = fmaxf(mx, fabsf(wd));
+            c = kr_fmul(-MM_M, wd);
         }
+        __builtin_amdgcn_sched_barrier(0);
+        if (g + 1 < NG) sn = __builtin_amdgcn_mfma_i32_32x32x32_i8(xa, wb[g + 1], s0, 0, 0, 0);
+#pragma unroll
+        for (int h = 0; h < 16; h += 8) {
+            float t[8];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int r = 0; r < 8; r++) t[r] = FAST ? __builtin_fmaf(__int_as_float(s[h + r]), wd, c) : kr_fmul((float)s[h + r], wd);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int r = 0; r < 8; r++) t[r] = kr_fmul(t[r], xd[h + r]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int r = 0; r < 8; r++) acc[g][h + r] = kr_fadd(acc[g][h + r], t[r]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        s = sn;
     }
 }
 
-// Workgroup = TW waves (4, or 1 for short batches) over a 32 NG-row x
-// 32 TW-token tile; wave w takes all the tile's rows (NG row groups) and
-// tokens 32 w .. 32 w + 31. The workgroup's
-// threads load each block's weight tile and its scales once (16 bytes and
-// one scale per thread) into an LDS ring of 3 stages: block b + 1 is stored
-// during step b into the stage step b - 2 read, and the barrier closing each
-// step orders those stores before step b + 1 reads them.
-template <int EPI, int QT, int D16, int NG, int TW = 4>
-__global__ void __launch_bounds__(64 * TW, NG == 1 ? 2 : 3) k_matmul(const MmArgs a) {   // waves per SIMD, at least
-    constexpr int TT = 32 * TW;   // tokens per workgroup
-    __shared__ MmLds<NG, TT> L;
+template <int QT, int D16, int NG, bool PAIR, bool FAST>
+__device__ __forceinline__ float mm_sums(float (&acc)[NG][16], MmStage<NG, D16> *L, const MmTile<NG> &t, int tid) {
+    const int wave = tid >> 6, lane = tid & 63, nb = t.nb;
+    v16i s0 = FAST ? mm_magic() : v16i{};
+    if constexpr (FAST) asm volatile("" : "+v"(s0));
+    float mx = 0.0f;
+#pragma unroll
+    for (int g = 0; g < NG; g++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[g][r] = 0.0f;
+    MmPre<QT, NG> R;
+    mm_load<QT, D16, NG, PAIR>(R, t, 0, tid);
+    mm_put<QT, D16, NG>(L[0], R, tid);
+    __syncthreads();
+    int st = 0;
+    for (int b0 = 0; b0 < nb; b0 += MM_SB) {
+        const bool more = b0 + MM_SB < nb;
+        mm_load<QT, D16, NG, PAIR>(R, t, more ? b0 + MM_SB : b0, tid);   // unconditional: past the end unused
+        __builtin_amdgcn_sched_barrier(0);
+        const int n = min(MM_SB, nb - b0);
+        const int ln = lane & 31, hf = lane >> 5, tk = 32 * wave;
+        MmAt<D16> p = { &L[st].w[ln][hf], &L[st].x[tk + ln][hf], (const float4 *)&L[st].xs[0][tk + 4 * hf],
+                        &L[st].d[ln][0] };
+#pragma unroll 1
+        for (int blk = 0; blk < n; blk++) {
+            mm_block<D16, NG, FAST>(acc, mx, s0, p);
+            p.next();
+        }
+        st ^= 1;
+        mm_put<QT, D16, NG>(L[st], R, tid);
+        __syncthreads();
+    }
+    return mx;
+}
+
+// ---- 16-row tiles: short prompts ----
+//
+// When the grid of 64-row tiles leaves CUs idle, a workgroup takes 16 rows
+// (RG groups of them) x 64 tokens, a wave 16 tokens of all its rows, one
+// v_mfma_i32_16x16x32_i8 per row group and block: a lane holds one weight row
+// and 4 tokens, so the sums' chains are a quarter as long as with the
+// 32 x 32 form and a short batch still has rows / 16 workgroups. A stage is 8
+// blocks (256 bytes of every row: whole cache lines), staged through two LDS
+// buffers and loaded 4 stages ahead (RG 2, whose grids give a CU several workgroups: 2)
+// in a register ring, which keeps 16 KB of weights in flight per workgroup
+// (one workgroup a CU must cover the memory latency by itself).
+constexpr int MS_SB = 8, MS_TT = 64;             // blocks a stage, tokens a workgroup
+constexpr int ms_depth(int rg) { return rg == 1 ? 4 : 2; }   // stages ahead (even)
+constexpr int MS_RC = 2 * MS_SB + 1;             // 16-byte chunks a staged row (one of padding)
+
+template <int RG, int D16>
+struct MsStage {
+    v4i w[16 * RG][MS_RC];
+    v4i x[MS_TT][MS_RC];
+    float xs[MS_SB][MS_TT];
+    __align__(16) typename MmScale<D16>::T d[16 * RG][MS_SB];
+};
+
+template <int QT, int RG>
+struct MsPre {
+    static constexpr int NW = QT == ML_Q8_0 ? RG : (RG + 1) / 2, ND = (RG + 1) / 2;
+    v4i w[NW], x[4];
+    uint32_t d[ND];
+    float xs[2];
+};
+
+template <int QT, int RG>
+struct MsTile {
+    const uint8_t *w, *d, *xs, *x;
+    uint32_t wo[MsPre<QT, RG>::NW], so[MsPre<QT, RG>::ND], xo[4], xso;
+    size_t xsb;
+    int nb;
+};
+
+template <int QT, int D16, int RG>
+__device__ __forceinline__ MsTile<QT, RG> ms_tile(const MmArgs &a, const MMat &W, int nb, int rowl, int tok0, int tid) {
+    constexpr int BB = QT == ML_Q8_0 ? 32 : 16, SB = D16 ? 2 : 4;
+    MsTile<QT, RG> t;
+    const size_t blk = (size_t)rowl * nb;
+    t.w = W.q + blk * BB;
+    t.d = (const uint8_t *)W.d + blk * SB;
+    // rows past the end re-read the last row, tokens past it the last token (not stored)
+    auto row = [&](int r) { return (uint32_t)(min(rowl + (r & (16 * RG - 1)), W.rows - 1) - rowl); };
+#pragma unroll
+    for (int u = 0; u < MsPre<QT, RG>::NW; u++)   // Q8: 16 threads a row; Q4: 8
+        t.wo[u] = row(QT == ML_Q8_0 ? (tid >> 4) + 16 * u : (tid >> 3) + 32 * u) * nb * BB;
+#pragma unroll
+    for (int u = 0; u < MsPre<QT, RG>::ND; u++) t.so[u] = row((tid >> 3) + 32 * u) * nb * SB;
+    t.x = (const uint8_t *)a.xq + (size_t)tok0 * a.K;
+#pragma unroll
+    for (int u = 0; u < 4; u++) t.xo[u] = (uint32_t)(min(tok0 + (tid >> 4) + 16 * u, a.T - 1) - tok0) * a.K;
+    t.xs = (const uint8_t *)(a.xdT + (size_t)tok0 * a.xst);
+    t.xso = (uint32_t)(min(tok0 + (tid & (MS_TT - 1)), a.T - 1) - tok0) * a.xst * 4;
+    t.xsb = (size_t)a.xsb * 4;
+    t.nb = nb;
+    return t;
+}
+
+// the stage at block b0 (one past the last: the last stage again); blocks past the last re-read the last (unused)
+template <int QT, int D16, int RG>
+__device__ __forceinline__ void ms_load(MsPre<QT, RG> &R, const MsTile<QT, RG> &t, int b, int tid) {
+    const int b0 = min(b, (t.nb - 1) / MS_SB * MS_SB), left = t.nb - b0;
+    const uint32_t c16 = 16 * min(tid & 15, 2 * left - 1), c8 = min(tid & 7, left - 1);
+#pragma unroll
+    for (int u = 0; u < MsPre<QT, RG>::NW; u++)
+        R.w[u] = QT == ML_Q8_0 ? *(const v4i *)(t.w + (size_t)b0 * 32 + (t.wo[u] + c16))
+                               : *(const v4i *)(t.w + (size_t)b0 * 16 + (t.wo[u] + 16 * c8));
+#pragma unroll
+    for (int u = 0; u < 4; u++) R.x[u] = *(const v4i *)(t.x + (size_t)b0 * 32 + (t.xo[u] + c16));
+#pragma unroll
+    for (int u = 0; u < MsPre<QT, RG>::ND; u++) {
+        const uint8_t *d = t.d + (size_t)b0 * (D16 ? 2 : 4);
+        R.d[u] = D16 ? (uint32_t)*(const uint16_t *)(d + (t.so[u] + 2 * c8)) : *(const uint32_t *)(d + (t.so[u] + 4 * c8));
+    }
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+        R.xs[u] = *(const float *)(t.xs + (size_t)(b0 + min((tid >> 6) + 4 * u, left - 1)) * t.xsb + t.xso);
+}
+
+template <int QT, int D16, int RG>
+__device__ __forceinline__ void ms_put(MsStage<RG, D16> &L, const MsPre<QT, RG> &R, int tid) {
+#pragma unroll
+    for (int u = 0; u < MsPre<QT, RG>::NW; u++) {
+        if constexpr (QT == ML_Q8_0) {
+            L.w[(tid >> 4) + 16 * u][tid & 15] = R.w[u];
+        } else if ((tid >> 3) + 32 * u < 16 * RG) {   // RG 1: half of the threads
+            L.w[(tid >> 3) + 32 * u][2 * (tid & 7)] = q4_frag(R.w[u], 0);
+            L.w[(tid >> 3) + 32 * u][2 * (tid & 7) + 1] = q4_frag(R.w[u], 1);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) L.x[(tid >> 4) + 16 * u][tid & 15] = R.x[u];
+#pragma unroll
+    for (int u = 0; u < MsPre<QT, RG>::ND; u++)
+        if ((tid >> 3) + 32 * u < 16 * RG) L.d[(tid >> 3) + 32 * u][tid & 7] = (typename MmScale<D16>::T)R.d[u];
+#pragma unroll
+    for (int u = 0; u < 2; u++) L.xs[(tid >> 6) + 4 * u][tid & (MS_TT - 1)] = R.xs[u];
+}
+
+// blocks b0 .. b0 + NB - 1 of a stage for the wave's 16 tokens: every read,
+// then every MFMA, then the rescales, so that one wave a SIMD still overlaps
+// the latencies
+template <int D16, int RG, bool FAST, int NB>
+__device__ __forceinline__ void ms_blocks(float (&acc)[RG][4], float &mx, const v4i &s0, const MsStage<RG, D16> &L,
+                                          int b0, int wave, int lane) {
+    const int ln = lane & 15, q = lane >> 4;
+    const long *xp = (const long *)&L.x[16 * wave + ln][2 * b0] + q;
+    const long *wp = (const long *)&L.w[ln][2 * b0] + q;
+    const float4 *xv = (const float4 *)&L.xs[b0][16 * wave + 4 * q];
+    float4 xd[NB];
+    float wd[NB][RG], c[NB][RG];
+    v4i s[NB][RG];
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        const long xa = xp[4 * b];
+        xd[b] = xv[b * (MS_TT / 4)];
+#pragma unroll
+        for (int g = 0; g < RG; g++) {
+            const uint32_t wdr = L.d[16 * g + ln][b0 + b];
+            wd[b][g] = D16 ? kr_h2f((uint16_t)wdr) : __uint_as_float(wdr);
+            s[b][g] = __builtin_amdgcn_mfma_i32_16x16x32_i8(xa, wp[2 * 16 * MS_RC * g + 4 * b], s0, 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int g = 0; g < RG; g++) {
+            if constexpr (FAST) {
+                asm volatile("" : "+v"(wd[b][g]));   // a register: no fma_mix from the half
+                mx = fmaxf(mx, fabsf(wd[b][g]));
+                c[b][g] = kr_fmul(-MM_M, wd[b][g]);
+            }
+        }
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        const float x4[4] = { xd[b].x, xd[b].y, xd[b].z, xd[b].w };
+#pragma unroll
+        for (int g = 0; g < RG; g++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float t = FAST ? __builtin_fmaf(__int_as_float(s[b][g][r]), wd[b][g], c[b][g])
+                                     : kr_fmul((float)s[b][g][r], wd[b][g]);
+                acc[g][r] = kr_fadd(acc[g][r], kr_fmul(t, x4[r]));
+            }
+    }
+}
+
+template <int D16, int RG, bool FAST>
+__device__ __forceinline__ void ms_stage(float (&acc)[RG][4], float &mx, const v4i &s0, const MsStage<RG, D16> &L,
+                                         int n, int wave, int lane) {
+    constexpr int NB = 4;
+    if (n >= MS_SB) {
+#pragma unroll
+        for (int b = 0; b < MS_SB; b += NB) ms_blocks<D16, RG, FAST, NB>(acc, mx, s0, L, b, wave, lane);
+    } else {
+#pragma unroll 1
+        for (int b = 0; b < n; b++) ms_blocks<D16, RG, FAST, 1>(acc, mx, s0, L, b, wave, lane);
+    }
+}
+
+template <int QT, int D16, int RG, bool FAST>
+__device__ __forceinline__ float ms_sums(float (&acc)[RG][4], MsStage<RG, D16> *L, const MsTile<QT, RG> &t, bool live,
+                                         int tid) {
+    const int wave = tid >> 6, lane = tid & 63, nb = t.nb;
+    constexpr int m = FAST ? MM_MAGIC : 0;
+    v4i s0 = v4i{ m, m, m, m };
+    if constexpr (FAST) asm volatile("" : "+v"(s0));
+    float mx = 0.0f;
+#pragma unroll
+    for (int g = 0; g < RG; g++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) acc[g][r] = 0.0f;
+    constexpr int MS_D = ms_depth(RG);
+    MsPre<QT, RG> R[MS_D];   // stage k sits in R[k % MS_D] until it is put
+#pragma unroll
+    for (int k = 0; k < MS_D; k++) ms_load<QT, D16, RG>(R[k], t, k * MS_SB, tid);
+    ms_put<QT, D16, RG>(L[0], R[0], tid);
+    ms_load<QT, D16, RG>(R[0], t, MS_D * MS_SB, tid);
+    __syncthreads();
+    // step k: stage k is summed from buffer k % 2 while stage k + 1 goes into
+    // the other (its last reader was step k - 1) and stage k + 1 + MS_D is
+    // loaded; every wave reaches every barrier
+    for (int b0 = 0; b0 < nb; b0 += MS_D * MS_SB) {
+#pragma unroll
+        for (int k = 0; k < MS_D; k++) {
+            const int b = b0 + k * MS_SB, k1 = (k + 1) % MS_D;
+            ms_put<QT, D16, RG>(L[(k + 1) & 1], R[k1], tid);
+            ms_load<QT, D16, RG>(R[k1], t, b + (MS_D + 1) * MS_SB, tid);
+            __builtin_amdgcn_sched_barrier(0);
+            if (live) ms_stage<D16, RG, FAST>(acc, mx, s0, L[k & 1], nb - b, wave, lane);
+            __syncthreads();
+        }
+    }
+    return mx;
+}
+
+template <int EPI, int QT, int D16, int RG>
+__global__ void __launch_bounds__(256, 2) k_matmul_short(const MmArgs a) {
+    __shared__ MsStage<RG, D16> L[2];
+    int mi = 0;
+    while (mi + 1 < a.nmat && (int)blockIdx.x >= a.tile0[mi + 1]) mi++;
+    const MMat W = mi == 0 ? a.w[0] : (mi == 1 ? a.w[1] : a.w[2]);
+    const int ntt = (a.T + MS_TT - 1) / MS_TT;
+    const int local = (int)blockIdx.x - a.tile0[mi];
+    const int rt = local / ntt, tt = local - rt * ntt;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int rowl = rt * 16 * RG, tokl = tt * MS_TT + 16 * wave;
+    const MsTile<QT, RG> t = ms_tile<QT, D16, RG>(a, W, a.K / KR_QK, rowl, tt * MS_TT, tid);
+    const bool live = __builtin_amdgcn_readfirstlane(tokl) < a.T;
+    float acc[RG][4];
+    if constexpr (D16) {
+        const float mx = ms_sums<QT, 1, RG, true>(acc, L, t, live, tid);
+        if (__syncthreads_or(mx == __builtin_inff())) ms_sums<QT, 1, RG, false>(acc, L, t, live, tid);
+    } else {
+        ms_sums<QT, 0, RG, false>(acc, L, t, live, tid);
+    }
+#pragma unroll
+    for (int g = 0; g < RG; g++)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            mm_emit<EPI>(a, mi, W.rows, rowl + 16 * g + (lane & 15), tokl + 4 * (lane >> 4) + r, acc[g][r]);
+}
+
+// Workgroup = 4 waves over a 32 NG-row x 128-token tile; wave w takes all the
+// tile's rows (NG row groups) and tokens 32 w .. 32 w + 31, NG 32x32x32 MFMAs a
+// block.
+template <int EPI, int QT, int D16, int NG>
+__global__ void __launch_bounds__(256, 2) k_matmul(const MmArgs a) {
+    constexpr int TT = MM_TT;
+    __shared__ MmStage<NG, D16> L[2];
     int mi = 0;
     while (mi + 1 < a.nmat && (int)blockIdx.x >= a.tile0[mi + 1]) mi++;
     const MMat W = mi == 0 ? a.w[0] : (mi == 1 ? a.w[1] : a.w[2]);
@@ -215,76 +568,14 @@ __global__ void __launch_bounds__(64 * TW, NG == 1 ? 2 : 3) k_matmul(const MmArg
     constexpr bool PAIR = EPI == MM_SWIGLU;   // 64 rows of w1 and the same 64 of w3
     const int rowl = rt * (PAIR ? 64 : 32 * NG), tokl = tt * TT + 32 * wave;
     const int nb = a.K / KR_QK;
-    const float *xcol = a.xdT + (size_t)min(tt * TT + (tid & (TT - 1)), a.T - 1) * a.xst;
-
     float acc[NG][16];
-#pragma unroll
-    for (int g = 0; g < NG; g++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) acc[g][r] = 0.0f;
-
-    // Loads are unconditional (block indices past the end re-read the last
-    // block, unused): a load issued on only one path makes the wait-count
-    // pass drain every in-flight load at the loop head, which would cancel
-    // the prefetch. Only the odd tail's step is conditional; every thread
-    // reaches every barrier.
-    const int bl = nb - 1;
-    if constexpr (NG >= 2) {
-        WReg R;
-        XFrag x0, x1;
-        w_load<QT, D16, NG, TT, PAIR>(R, W, xcol, a.xsb, nb, 0, rowl, tid, a.w[1]);
-        w_store(L, 0, R, tid);
-        w_load<QT, D16, NG, TT, PAIR>(R, W, xcol, a.xsb, nb, 1 < bl ? 1 : bl, rowl, tid, a.w[1]);
-        x_load(x0, a, 0, tokl, lane);
-        x_load(x1, a, 1 < bl ? 1 : bl, tokl, lane);
-        __syncthreads();
-        int st = 0;   // stage of block b
-        for (int b = 0; b < nb; b += 2) {
-            const int s1 = st == MM_ST - 1 ? 0 : st + 1, s2 = s1 == MM_ST - 1 ? 0 : s1 + 1;
-            w_store(L, s1, R, tid);
-            w_load<QT, D16, NG, TT, PAIR>(R, W, xcol, a.xsb, nb, b + 2 < bl ? b + 2 : bl, rowl, tid, a.w[1]);
-            mm_step<D16, NG, TT>(acc, x0, L, st, lane, 32 * wave);
-            x_load(x0, a, b + 2 < bl ? b + 2 : bl, tokl, lane);
-            __syncthreads();
-            w_store(L, s2, R, tid);
-            w_load<QT, D16, NG, TT, PAIR>(R, W, xcol, a.xsb, nb, b + 3 < bl ? b + 3 : bl, rowl, tid, a.w[1]);
-            if (b + 1 < nb) mm_step<D16, NG, TT>(acc, x1, L, s1, lane, 32 * wave);
-            x_load(x1, a, b + 3 < bl ? b + 3 : bl, tokl, lane);
-            __syncthreads();
-            st = s2;
-        }
+    const MmTile<NG> t = mm_tile<QT, D16, NG, PAIR>(a, W, a.w[1], nb, rowl, tt * TT, tid);
+    if constexpr (D16) {
+        // every wave of the workgroup sees the tile's rows: one vote for all
+        const float mx = mm_sums<QT, 1, NG, PAIR, true>(acc, L, t, tid);
+        if (__syncthreads_or(mx == __builtin_inff())) mm_sums<QT, 1, NG, PAIR, false>(acc, L, t, tid);
     } else {
-        // One row group: a block's VALU work is a quarter of NG = 4's, too
-        // little to cover a load's latency, so the weight and token loads
-        // run MM_PD blocks ahead in register rings (R[j], x[j]: the blocks
-        // congruent to j mod MM_PD), and the weight tile passes through a
-        // 2-stage LDS ring. Step t stores block t + 1 (loaded MM_PD steps
-        // earlier) into stage (t + 1) % 2, loads block t + 1 + MM_PD in its
-        // place, runs block t from stage t % 2 and reloads x with block
-        // t + MM_PD; the barrier closing each step orders the stage writes
-        // against the reads of the steps either side.
-        WReg R[MM_PD];
-        XFrag x[MM_PD];
-#pragma unroll
-        for (int j = 0; j < MM_PD; j++) {
-            w_load<QT, D16, NG, TT, PAIR>(R[j], W, xcol, a.xsb, nb, j < bl ? j : bl, rowl, tid, a.w[1]);
-            x_load(x[j], a, j < bl ? j : bl, tokl, lane);
-        }
-        w_store(L, 0, R[0], tid);
-        w_load<QT, D16, NG, TT, PAIR>(R[0], W, xcol, a.xsb, nb, MM_PD < bl ? MM_PD : bl, rowl, tid, a.w[1]);
-        __syncthreads();
-        for (int b0 = 0; b0 < nb; b0 += MM_PD) {
-#pragma unroll
-            for (int k = 0; k < MM_PD; k++) {
-                const int t = b0 + k, k1 = (k + 1) % MM_PD;
-                w_store(L, (k + 1) & 1, R[k1], tid);
-                w_load<QT, D16, NG, TT, PAIR>(R[k1], W, xcol, a.xsb, nb, t + 1 + MM_PD < bl ? t + 1 + MM_PD : bl, rowl,
-                                          tid, a.w[1]);
-                if (t < nb) mm_step<D16, NG, TT>(acc, x[k], L, k & 1, lane, 32 * wave);
-                x_load(x[k], a, t + MM_PD < bl ? t + MM_PD : bl, tokl, lane);
-                __syncthreads();
-            }
-        }
+        mm_sums<QT, 0, NG, PAIR, false>(acc, L, t, tid);
     }
 
     // epilogue: lane = one row (32 g + lane % 32), tokens 8 (r / 4) + 4 (lane / 32) + r % 4
@@ -312,47 +603,22 @@ __global__ void __launch_bounds__(64 * TW, NG == 1 ? 2 : 3) k_matmul(const MmArg
         }
         return;
     }
-    float *Y = mi == 0 ? a.y[0] : (mi == 1 ? a.y[1] : a.y[2]);
-    const int ldy = mi == 0 ? a.ldy[0] : (mi == 1 ? a.ldy[1] : a.ldy[2]);
-    const float *bias = mi == 0 ? a.bias[0] : (mi == 1 ? a.bias[1] : a.bias[2]);
 #pragma unroll
-    for (int g = 0; g < NG; g++) {
-        const int row = rowl + 32 * g + (lane & 31);
-        const bool rin = row < W.rows;
+    for (int g = 0; g < NG; g++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int t = tokl + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-            float v = acc[g][r];
-            if (EPI == MM_QKV) {
-                // bias (model/transformer.c:276-277), then RoPE on q and k
-                // (k_scalar.c:79-94): rows 2i, 2i+1 sit in lanes 2i, 2i+1
-                if (bias && rin) v = kr_fadd(v, bias[row]);
-                const float o = __shfl_xor(v, 1);
-                if (mi < 2) {
-                    const int hd = a.head_dim, j = row % hd, h2 = hd >> 1;
-                    const int pos = a.pos0 + (t < a.T ? t : 0);
-                    const float c = a.rope_cos[(size_t)pos * h2 + (j >> 1)];
-                    const float sn = a.rope_sin[(size_t)pos * h2 + (j >> 1)];
-                    v = (j & 1) == 0 ? kr_fsub(kr_fmul(v, c), kr_fmul(o, sn)) : kr_fadd(kr_fmul(o, sn), kr_fmul(v, c));
-                }
-            }
-            if (rin && t < a.T) {
-                float *p = Y + (size_t)t * ldy + row;
-                if (EPI == MM_ADD) *p = kr_fadd(*p, v);
-                else *p = v;
-            }
-        }
-    }
+        for (int r = 0; r < 16; r++)
+            mm_emit<EPI>(a, mi, W.rows, rowl + 32 * g + (lane & 31), tokl + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3),
+                         acc[g][r]);
 }
 
 template <int EPI>
 void launch_mm(const MmArgs &a, const MMat &W) {
     const int grid = a.tile0[a.nmat];
-    if (a.K % KR_QK || a.T <= 0 || grid <= 0 || a.ldx % MM_TT || a.T > a.ldx || a.xsb <= 0 || a.xst <= 0 || (a.tw != 4 && (a.tw != 1 || a.ng != 1))) {
+    if (a.K % KR_QK || a.T <= 0 || grid <= 0 || a.ldx % MM_TT || a.T > a.ldx || a.xsb <= 0 || a.xst <= 0) {
         kr_fail(ML_E_SHAPE, "matmul shape", hipSuccess);
         return;
     }
-    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * a.tw), 0, kr_stream(), a); };
+    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, kr_stream(), a); };
     if (EPI == MM_SWIGLU && a.ng != 4) {
         kr_fail(ML_E_SHAPE, "matmul: SwiGLU pairs take 128-row tiles", hipSuccess);
         return;
@@ -373,16 +639,16 @@ void launch_mm(const MmArgs &a, const MMat &W) {
             kr_check_launch("matmul");
             return;
         }
-        if (a.tw == 1) {
+        if (a.rg == 2) {
             if (W.type == ML_Q8_0) {
-                if (W.d16) go(k_matmul<EPI, ML_Q8_0, 1, 1, 1>); else go(k_matmul<EPI, ML_Q8_0, 0, 1, 1>);
+                if (W.d16) go(k_matmul_short<EPI, ML_Q8_0, 1, 2>); else go(k_matmul_short<EPI, ML_Q8_0, 0, 2>);
             } else {
-                if (W.d16) go(k_matmul<EPI, ML_Q4_0, 1, 1, 1>); else go(k_matmul<EPI, ML_Q4_0, 0, 1, 1>);
+                if (W.d16) go(k_matmul_short<EPI, ML_Q4_0, 1, 2>); else go(k_matmul_short<EPI, ML_Q4_0, 0, 2>);
             }
         } else if (W.type == ML_Q8_0) {
-            if (W.d16) go(k_matmul<EPI, ML_Q8_0, 1, 1>); else go(k_matmul<EPI, ML_Q8_0, 0, 1>);
+            if (W.d16) go(k_matmul_short<EPI, ML_Q8_0, 1, 1>); else go(k_matmul_short<EPI, ML_Q8_0, 0, 1>);
         } else {
-            if (W.d16) go(k_matmul<EPI, ML_Q4_0, 1, 1>); else go(k_matmul<EPI, ML_Q4_0, 0, 1>);
+            if (W.d16) go(k_matmul_short<EPI, ML_Q4_0, 1, 1>); else go(k_matmul_short<EPI, ML_Q4_0, 0, 1>);
         }
     }
     kr_check_launch("matmul");
@@ -393,37 +659,34 @@ MMat to_mmat(const krh_mat *m) {
     return k;
 }
 
-int row_tiles(int rows, int ng) { return (rows + 32 * ng - 1) / (32 * ng); }
-
-// NG for a launch over these row counts and ntt token tiles: 4 when it has
-// at least two 128-row tiles per CU, else 2 when it has half a 64-row tile
-// per CU (w1 and w3 at the reference's 128-token steps: its 8B prefill
-// through ml_run 5,674 -> 5,844 tok/s), else 1. One 128-row tile per CU
-// leaves each SIMD one wave, which issues a VALU instruction only every 6.5
-// cycles or more: the 1B shape's wo and w2 (256 tiles at 2048 tokens) on
-// 64-row tiles took its 4000-token prefill from 65.4k-65.7k to 67.6k-67.8k
-// tok/s (the threshold was 3/4 of a tile per CU); 64-row tiles up to 3 or 4
-// tiles per CU took the 8B shape's from 21.6k-21.8k to 20.4k-20.5k. Measured (K = 4096, 256
-// CUs): a 128-row tile does 4 times a 32-row tile's work in 1.9 times its
-// time, so from about 200 tiles, where the 32-row grid needs two rounds of
-// resident workgroups, the 128-row grid's one round is the shorter (14336
-// rows at T = 512: 152 against 300 us); below it, 32-row tiles keep more CUs
-// busy (T = 128, 112 tiles: 89 us, where one round of 128-row tiles takes
-// about what it takes at T = 192, 125 us).
-int pick_ng(int rows0, int rows1, int rows2, int ntt) {
-    const int tiles = row_tiles(rows0, 4) + row_tiles(rows1, 4) + row_tiles(rows2, 4);
-    const int cus = krh_device_cus() > 0 ? krh_device_cus() : 256;
-    const int tiles2 = row_tiles(rows0, 2) + row_tiles(rows1, 2) + row_tiles(rows2, 2);
-    return tiles * ntt >= 2L * cus ? 4 : 2L * tiles2 * ntt >= cus ? 2 : 1;
-}
-
-// Waves per workgroup (TW) for an NG 1 launch whose grid of 128-token tiles
-// leaves CUs idle (fewer than two 32-row tiles per CU: the reference's
-// 128-token steps over wq, wk, wv, wo and w2): one wave and 32 tokens a
-// workgroup gives 4 times the workgroups. Else 4.
-int pick_tw(int ng, int grid128) {
-    const int cus = krh_device_cus() > 0 ? krh_device_cus() : 256;
-    return ng == 1 && grid128 < 2 * cus ? 1 : 4;
+// The tiles of a launch over nmat matrices of these rows: NG 4 (128 rows x
+// 128 tokens a workgroup), NG 2 (64 x 128), RG 2 (32 x 64) or RG 1 (16 x 64).
+// Larger tiles load less per sum, smaller ones make more workgroups; the lines,
+// in workgroups per CU, from krh_matmul on 256 CUs (us; Q8, K 4096 and 14336):
+// - NG 4 once NG 2's grid is more than one round of its 2 workgroups a CU:
+//   4096 x 14336, 1100 tokens (2.25 rounds' worth of NG 2): 342 against 381;
+//   14336 x 4096, 511 tokens: 112 against 128; at 2 a CU or less the halves
+//   balance better: 2048 x 2048, 2047 tokens 55 against 43, 14336 x 4096, 256
+//   tokens 92 against 70.
+// - RG 2 below 3 of its workgroups a CU: 4096 x 14336, 300 tokens (2.5 a CU)
+//   167 against NG 2's 187, 14336 x 4096, 64 tokens 38 against 60; above,
+//   14336 x 4096, 128 tokens (3.5) 72 against 60.
+// - RG 1 below 1.25 of RG 2's a CU: 4096 x 14336, 37 tokens 53 against 75 and
+//   128 tokens (1 a CU) 75 against 82; above, 2048 x 2048, 400 tokens 29
+//   against 25.
+void mm_plan(MmArgs &a, int nmat, const int *rows) {
+    const int ntt128 = (a.T + MM_TT - 1) / MM_TT, ntt64 = (a.T + MS_TT - 1) / MS_TT;
+    const long cus = krh_device_cus() > 0 ? krh_device_cus() : 256;
+    long t64 = 0, t32 = 0;   // NG 2's and RG 2's workgroups
+    for (int i = 0; i < nmat; i++) {
+        t64 += (long)(rows[i] + 63) / 64 * ntt128;
+        t32 += (long)(rows[i] + 31) / 32 * ntt64;
+    }
+    a.ng = t64 > 2 * cus ? 4 : t32 >= 3 * cus ? 2 : 1;
+    a.rg = a.ng != 1 ? 0 : 4 * t32 >= 5 * cus ? 2 : 1;
+    const int per = a.rg ? 16 * a.rg : 32 * a.ng;
+    a.tile0[0] = 0;
+    for (int i = 0; i < nmat; i++) a.tile0[i + 1] = a.tile0[i] + (rows[i] + per - 1) / per * (a.rg ? ntt64 : ntt128);
 }
 
 // ---- per-token work of a batched step ----
@@ -493,7 +756,6 @@ extern "C" void krh_matmul_swiglu(int8_t *hq, float *hdT, const krh_mat *w1, con
     a.tile0[0] = 0;
     const int ntt = (T + MM_TT - 1) / MM_TT;
     a.ng = 4;
-    a.tw = 4;
     a.tile0[1] = (w1->rows + 63) / 64 * ntt;
     a.xq = xq;
     a.xdT = xdT;
@@ -513,12 +775,6 @@ static void matmul_one(float *Y, int ldy, const krh_mat *W, const int8_t *xq, co
     MmArgs a = {};
     a.w[0] = to_mmat(W);
     a.nmat = 1;
-    a.tile0[0] = 0;
-    const int ntt128 = (T + MM_TT - 1) / MM_TT;
-    a.ng = pick_ng(W->rows, 0, 0, ntt128);
-    a.tw = pick_tw(a.ng, row_tiles(W->rows, a.ng) * ntt128);
-    const int ntt = (T + 32 * a.tw - 1) / (32 * a.tw);
-    a.tile0[1] = row_tiles(W->rows, a.ng) * ntt;
     a.xq = xq;
     a.xdT = xd;
     a.ldx = ldx;
@@ -528,6 +784,7 @@ static void matmul_one(float *Y, int ldy, const krh_mat *W, const int8_t *xq, co
     a.K = W->cols;
     a.y[0] = Y;
     a.ldy[0] = ldy;
+    mm_plan(a, 1, &W->rows);
     if (accumulate) launch_mm<MM_ADD>(a, a.w[0]);
     else launch_mm<MM_STORE>(a, a.w[0]);
 }
@@ -552,7 +809,6 @@ static void matmul_qkv(float *q, float *kc, float *vc, const krh_mat *wq, const 
         kr_fail(ML_E_SHAPE, "matmul qkv shapes", hipSuccess);
         return;
     }
-    const int ntt128 = (T + MM_TT - 1) / MM_TT;
     MmArgs a = {};
     a.w[0] = to_mmat(wq);
     a.w[1] = to_mmat(wk);
@@ -578,13 +834,8 @@ static void matmul_qkv(float *q, float *kc, float *vc, const krh_mat *wq, const 
     a.rope_sin = rope_sin;
     a.head_dim = head_dim;
     a.pos0 = pos0;
-    a.ng = pick_ng(wq->rows, wk->rows, wv->rows, ntt128);
-    a.tw = pick_tw(a.ng, (row_tiles(wq->rows, a.ng) + 2 * row_tiles(wk->rows, a.ng)) * ntt128);
-    const int ntt = (T + 32 * a.tw - 1) / (32 * a.tw);
-    a.tile0[0] = 0;
-    a.tile0[1] = row_tiles(wq->rows, a.ng) * ntt;
-    a.tile0[2] = a.tile0[1] + row_tiles(wk->rows, a.ng) * ntt;
-    a.tile0[3] = a.tile0[2] + row_tiles(wv->rows, a.ng) * ntt;
+    const int rows[3] = { wq->rows, wk->rows, wv->rows };
+    mm_plan(a, 3, rows);
     if (wv->type == wq->type) {
         a.nmat = 3;
         launch_mm<MM_QKV>(a, a.w[0]);
@@ -595,7 +846,7 @@ static void matmul_qkv(float *q, float *kc, float *vc, const krh_mat *wq, const 
     launch_mm<MM_QKV>(b, b.w[0]);
     MmArgs c = a;   // v alone, as matrix 2 of the same epilogue
     c.tile0[0] = c.tile0[1] = c.tile0[2] = 0;
-    c.tile0[3] = row_tiles(wv->rows, a.ng) * ntt;
+    c.tile0[3] = a.tile0[3] - a.tile0[2];
     c.w[0] = c.w[1] = c.w[2];
     c.nmat = 3;
     launch_mm<MM_QKV>(c, c.w[2]);

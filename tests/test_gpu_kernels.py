@@ -571,6 +571,46 @@ def test_matmul(dev, typ, d16, rows, cols, T):
             assert np.array_equal(bits(got_rows[t]), bits(want)), (t, acc, "rows")
 
 
+# one size for each tile form (16 x 64, 32 x 64, 64 x 128 and 128 x 128 rows x
+# tokens) with ragged rows, tokens and stages (4 or 8 blocks of 32 columns)
+@pytest.mark.parametrize("typ,d16", [(K.ML_Q8_0, 1), (K.ML_Q4_0, 1), (K.ML_Q8_0, 0)])
+@pytest.mark.parametrize("rows,cols,T", [(17, 32, 2), (100, 992, 65), (16, 1056, 64), (10250, 288, 33),
+                                         (10240, 256, 17), (16416, 96, 65), (16416, 128, 128), (16450, 160, 130)])
+@pytest.mark.parametrize("scales", ["plain", "signed", "infinite"])
+def test_matmul_tiles(dev, typ, d16, rows, cols, T, scales):
+    """every tile form's sums equal the matvec's, bit for bit; signed: negative
+    and zero scales (Q4 blocks have them), infinite: a few infinite ones (the
+    f16 form then converts, and 0 * inf is NaN as in the scalar kernel)"""
+    q, d, dh = rand_mat(rows, cols, typ, d16)
+    nb = cols // 32
+    if scales != "plain":
+        at = RNG.integers(0, rows * nb, 40)
+        if scales == "signed":
+            dh[::2] = -dh[::2]
+            dh[at] = 0
+        else:
+            dh[at[:3]] = np.inf
+            dh[at[3:6]] = -np.inf
+        d = dh.astype(np.float32)
+    tk = sorted(set([0, 1, T // 2, T - 1]))
+    ldx = (T + 127) // 128 * 128
+    X = f32(RNG.normal(0, 1, (T, cols)))
+    xq, xd = np.zeros((ldx, cols), np.int8), np.zeros((T, nb), np.float32)
+    for t in range(T):
+        xq[t], xd[t] = O.quantize(X[t])
+    W = dmat(dev, q, d, dh, rows, cols, typ, d16)
+    yb = dev.zeros(4 * T * rows)
+    K.hip.krh_matmul(yb.ptr, rows, C.byref(W), dev.put(xq).ptr, dev.put(transposed_scales(xd, T, nb, ldx)).ptr, ldx,
+                     T, 0)
+    ok()
+    got = yb.get(np.float32, T * rows).reshape(T, rows)
+    for t in tk:
+        want = oracle_matvec(q, d, rows, cols, typ, xq[t], xd[t])
+        nan = np.isnan(want)
+        assert np.array_equal(np.isnan(got[t]), nan), t
+        assert np.array_equal(bits(got[t][~nan]), bits(want[~nan])), t
+
+
 @pytest.mark.parametrize("dim,nh,nkv,hd,typ,vtyp,bias", [(288, 6, 6, 48, K.ML_Q8_0, K.ML_Q8_0, 0),
                                                           (896, 14, 2, 64, K.ML_Q4_0, K.ML_Q8_0, 1),
                                                           (4096, 32, 8, 128, K.ML_Q8_0, K.ML_Q8_0, 0)])
