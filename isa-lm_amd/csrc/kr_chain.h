@@ -154,6 +154,48 @@ __device__ __forceinline__ float sc_blk16(const float *t, int sh, int i0, float 
     return s;
 }
 
+// s + the n terms at t (layout sc_at, sh = SC_LOG_LMIN: rows of 128 with their
+// padding), one add at a time: 32 terms' 16-byte reads are issued ahead of the
+// 32 adds before them, so the chain runs at about the adds' own latency. Every
+// calling lane runs the same chain (one address: the reads broadcast). For a sum of a few hundred
+// terms this is shorter than the speculative form's fixed cost.
+__device__ __forceinline__ float sc_short(const float *t, int n, float s) {
+    constexpr int B = 32;
+    static_assert((1 << SC_LOG_LMIN) % (2 * B) == 0, "a pair of batches stays in its chunk's row");
+    float4 a[B / 4], b[B / 4];
+    auto read = [&](float4 (&v)[B / 4], int i) {
+        const float4 *p = (const float4 *)(t + sc_at(i, SC_LOG_LMIN));
+#pragma unroll
+        for (int k = 0; k < B / 4; k++) v[k] = p[k];
+    };
+    auto add = [&](const float4 (&v)[B / 4]) {
+#pragma unroll
+        for (int k = 0; k < B / 4; k++) {
+            s = kr_fadd(s, v[k].x);
+            s = kr_fadd(s, v[k].y);
+            s = kr_fadd(s, v[k].z);
+            s = kr_fadd(s, v[k].w);
+        }
+    };
+    const int last = n > B ? (n - B) & ~(B - 1) : 0;   // the last whole batch (read again rather than past it)
+    int i = 0;
+    read(a, 0);
+    for (; i + 2 * B <= n; i += 2 * B) {
+        read(b, i + B);
+        __builtin_amdgcn_sched_barrier(0);
+        add(a);
+        read(a, min(i + 2 * B, last));
+        __builtin_amdgcn_sched_barrier(0);
+        add(b);
+    }
+    if (i + B <= n) {
+        add(a);
+        i += B;
+    }
+    for (; i < n; i++) s = kr_fadd(s, t[sc_at(i, SC_LOG_LMIN)]);
+    return s;
+}
+
 // whether the run with even start b and ends e0, e1 maps the true start sv
 // to sv + (its end's offset) inside one binade; end: that value
 __device__ __forceinline__ bool sc_shift(unsigned sv, unsigned b, unsigned e0, unsigned e1, unsigned &end) {
@@ -478,6 +520,24 @@ __device__ __forceinline__ float kr_spec_sum(float *t, int n, unsigned char *lds
     }
     if (WAVE) kr_wave_sync();
     else __syncthreads();
+    return *res;
+}
+
+// The ordered sum by the workgroup's first wave alone (n <= SC_SHORT), as
+// kr_spec_sum otherwise: the same terms, calling rules and bits (+0 start).
+// The line: 288 terms (a 15M model's norms) one by one take the FFN of a token
+// from 10.9 to 9.5 us; 896 terms (the 0.5B shape's) were slower that way (its
+// 31 decoded tokens and prompt 41.2 ms against 40.7).
+constexpr int SC_SHORT = 640;
+template <int NT>
+__device__ __forceinline__ float kr_sum_any(float *t, int n, unsigned char *lds) {
+    if (n > SC_SHORT) return kr_spec_sum<NT>(t, n, lds);
+    float *res = (float *)lds;
+    if (threadIdx.x < 64) {
+        const float s = sc_short(t, n, 0.0f);
+        if (threadIdx.x == 0) *res = s;
+    }
+    __syncthreads();
     return *res;
 }
 

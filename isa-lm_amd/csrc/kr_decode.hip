@@ -533,7 +533,7 @@ __global__ void __launch_bounds__(MV_THREADS, mv_wgs_per_cu(EPI)) k_matvec(const
             for (int d = 0; d < MV_DEPTH - 1; d++) load_item(S[d], I[d]);
             prime_touch();
             __syncthreads();
-            const float ss = kr_spec_sum<MV_THREADS>(sq, K, (unsigned char *)(sq + sc_terms_cap(K)));
+            const float ss = kr_sum_any<MV_THREADS>(sq, K, (unsigned char *)(sq + sc_terms_cap(K)));
             inv = kr_fdiv(1.0f, kr_fsqrt(kr_fadd(kr_fdiv(ss, (float)K), a.eps)));
         }
         if (live) {
@@ -565,7 +565,7 @@ __global__ void __launch_bounds__(MV_THREADS, mv_wgs_per_cu(EPI)) k_matvec(const
                                                   kr_fmul(v.w, v.w));
             }
             __syncthreads();
-            const float ss = kr_spec_sum<MV_THREADS>(sq, K, (unsigned char *)(sq + sc_terms_cap(K)));
+            const float ss = kr_sum_any<MV_THREADS>(sq, K, (unsigned char *)(sq + sc_terms_cap(K)));
             const float inv = kr_fdiv(1.0f, kr_fsqrt(kr_fadd(kr_fdiv(ss, (float)K), a.eps)));
             quantize_to_lds(a.xf, K, xs, xds, a.nw, inv, blockIdx.x == 0 ? a.keep_xb : nullptr);
         } else {

@@ -824,6 +824,13 @@ def test_rmsnorm_matvec(dev, typ, d16, rows, cols):
     assert np.array_equal(bits(yb.get(np.float32, rows)), bits(oracle_matvec(q, d, rows, cols, typ, xq, xd)))
 
 
+# batches of 32 terms, pairs of batches and 128-term rows of the one-wave
+# ordered sum, the last length it takes and the first past it
+@pytest.mark.parametrize("cols", [32, 64, 96, 128, 160, 256, 288, 608, 640, 672])
+def test_rmsnorm_matvec_short_sums(dev, cols):
+    test_rmsnorm_matvec(dev, K.ML_Q8_0, 1, 40, cols)
+
+
 @pytest.mark.parametrize("dim,nh,nkv,hd,typ,vtyp,bias", [(896, 14, 2, 64, K.ML_Q4_0, K.ML_Q8_0, 1),
                                                           (4096, 32, 8, 128, K.ML_Q8_0, K.ML_Q8_0, 0)])
 def test_rmsnorm_qkv_matches_unfused(dev, dim, nh, nkv, hd, typ, vtyp, bias):
