@@ -243,6 +243,11 @@ void krh_matmul_qkv_stage(float *q, float *k, float *v, const krh_mat *wq, const
 void krh_attention_batch(float *ao, float *att, const float *q, const float *kc, const float *vc, int n_heads,
                          int n_kv_heads, int head_dim, int max_seq, int window, float scale, const int *pos0, int ntok,
                          int last_pos);
+/* The rows (positions attended) up to which a decode attention over this
+ * cache type, without soft-capping, is one launch (0: never): a call whose
+ * last position, or window, bounds its row by that takes it. The scratch is
+ * then not written. */
+int krh_attention_short(int head_dim, int kv_type);
 /* The batched attention's choice of kernels (no counterpart in the
  * reference): heads of 48, 64, 80, 96, 128 or 256 dims take the
  * register-blocked score and mix kernels when their grids hold at least

@@ -1380,6 +1380,192 @@ __global__ void __launch_bounds__(64) k_attn_mix_batch_kv(float *ao, const float
     attn_mix_batch<DW, KT>(ao, att, kv, group, hd, kv_dim, max_seq, window, pos_p);
 }
 
+// ---- decode over a short context: one launch ----
+
+// A query head's whole attention in one workgroup, for rows of scores whose K
+// rows fit in LDS together (AS_LDS: 559 positions of 64 dims). The three
+// launches of a longer row spend most of such a token on their gaps, their
+// loads' latencies and the ordered sum's fixed cost: 17.7 us a layer for 14
+// heads of 64 dims at position 530 against the one launch's 9.1. K and V are
+// loaded together up front; V waits in registers while the scores run from
+// K's LDS copy, then its products with the weights take that copy's place.
+//   scores: a thread per position, its ordered dot from LDS;
+//   softmax: max, exponentials, and their ordered sum one add at a time (the
+//     speculative sum's fixed cost is more than these rows' chains);
+//   mix: the products a_t * v_t,d by every thread into [position / 4][dim][4]
+//     order (the 16-byte reads of a wave's dims are contiguous; each thread
+//     stores its 4 dims rotated by its quad's number, which puts the 64
+//     stores of a wave on 64 banks), then one lane per dim adds them in
+//     position order.
+constexpr int AS_NT = 1024, AS_LDS = 152 * 1024;   // threads; bytes of the K copy or the products
+constexpr int AS_NP = 10;   // passes over the rows, at most: 4-element loads a thread holds, of K and of V
+// positions whose K rows (hd + 4 floats) and products fit
+constexpr int as_positions(int hd) {
+    return std::min(std::min((AS_LDS / 4 / (hd + 4)) & ~3, AS_NT), AS_NT / (hd / 4) * AS_NP);
+}
+
+struct AsLds {
+    __align__(16) float kt[AS_LDS / 4];   // K [position][hd + 4], then the products
+    __align__(16) float w[AS_NT + 32];    // exponentials, then weights
+    __align__(16) float qs[256];
+    float red[AS_NT / 64];
+    float sum;
+    uint64_t xtab[32];
+};
+
+// NP: passes of AS_NT / (hd / 4) rows (every load unconditional: the compiler
+// then waits for K without waiting for V)
+template <int KT, int NP>
+__device__ __forceinline__ void attn_short(AsLds &S, float *ao, const float *q, const KvView &kv, int group, int hd,
+                                           int kv_dim, float scale, int first, int n) {
+    float *kt = S.kt, *w = S.w, *qs = S.qs, *red = S.red;
+    const int tid = threadIdx.x, lane = tid & 63, h = blockIdx.x, g = h / group, h4 = hd / 4, ks = hd + 4;
+    const int rows = AS_NT / h4, r0 = tid / h4, c = tid - r0 * h4;   // pass u: row u * rows + r0, dims 4c ..
+    const bool mine = r0 < rows;                                     // the threads past a pass's rows hold none
+    const size_t base = (size_t)first * kv_dim + (size_t)g * hd + 4 * c;
+    typename Kv4<KT>::T kr[NP], vr[NP];
+#pragma unroll
+    for (int u = 0; u < NP; u++) kr[u] = Kv4<KT>::load(kv.k, base + (size_t)min(u * rows + r0, n - 1) * kv_dim);
+#pragma unroll
+    for (int u = 0; u < NP; u++) vr[u] = Kv4<KT>::load(kv.v, base + (size_t)min(u * rows + r0, n - 1) * kv_dim);
+    if (tid < h4) *(float4 *)(qs + 4 * tid) = *(const float4 *)(q + (size_t)h * hd + 4 * tid);
+    if (tid >= AS_NT - 32) S.xtab[tid - (AS_NT - 32)] = kr_exp2_tab[tid - (AS_NT - 32)];
+#pragma unroll
+    for (int u = 0; u < NP; u++)
+        if (mine && u * rows + r0 < n) *(float4 *)(kt + (u * rows + r0) * ks + 4 * c) = Kv4<KT>::wide(kr[u]);
+    __syncthreads();
+    // the score of position tid
+    float x = -INFINITY;
+    if (tid < n) {
+        const float *k = kt + tid * ks;
+        float acc = 0.0f;
+#pragma unroll 4
+        for (int i = 0; i < hd; i += 4) {
+            const float4 a = *(const float4 *)(qs + i), b = *(const float4 *)(k + i);
+            acc = kr_fadd(acc, kr_fmul(a.x, b.x));
+            acc = kr_fadd(acc, kr_fmul(a.y, b.y));
+            acc = kr_fadd(acc, kr_fmul(a.z, b.z));
+            acc = kr_fadd(acc, kr_fmul(a.w, b.w));
+        }
+        x = kr_fmul(acc, scale);
+    }
+    float m = x;
+    for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+    if (lane == 0) red[tid >> 6] = m;
+    __syncthreads();
+    m = red[0];
+    for (int k = 1; k < AS_NT / 64; k++) m = fmaxf(m, red[k]);
+    float e = 0.0f;
+    if (tid < n) {
+        e = kr_expf_tab(kr_fsub(x, m), S.xtab);
+        w[tid] = e;
+    }
+    __syncthreads();
+    if (tid < 64) {   // the ordered sum: every lane the same chain, 32 terms' reads ahead of their adds
+        float s = 0.0f;
+        int t = 0;
+        float4 a[8], b[8];
+        auto read = [&](float4 (&v)[8], int t0) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) v[k] = *(const float4 *)(w + min(t0, AS_NT) + 4 * k);
+        };
+        auto add = [&](const float4 (&v)[8]) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                s = kr_fadd(s, v[k].x);
+                s = kr_fadd(s, v[k].y);
+                s = kr_fadd(s, v[k].z);
+                s = kr_fadd(s, v[k].w);
+            }
+        };
+        read(a, 0);
+        for (; t + 64 <= n; t += 64) {
+            read(b, t + 32);
+            __builtin_amdgcn_sched_barrier(0);
+            add(a);
+            read(a, t + 64);
+            __builtin_amdgcn_sched_barrier(0);
+            add(b);
+        }
+        for (; t < n; t++) s = kr_fadd(s, w[t]);
+        if (tid == 0) S.sum = s;
+    }
+    __syncthreads();
+    // every score -inf: 1 / n (k_scalar.c:66-77)
+    if (tid < n) w[tid] = m == -INFINITY ? kr_fdiv(1.0f, (float)n) : kr_fmul(e, kr_fdiv(1.0f, S.sum));
+    __syncthreads();
+    // products; position r, dims 4c ..: quad r / 4's floats [dim][r % 4]
+    const int rot = (c >> 2) & 3;
+#pragma unroll
+    for (int u = 0; u < NP; u++) {
+        const int r = u * rows + r0;
+        if (mine && r < n) {
+            const float a = w[r];
+            const float4 v = Kv4<KT>::wide(vr[u]);
+            const float p0 = kr_fmul(a, v.x), p1 = kr_fmul(a, v.y), p2 = kr_fmul(a, v.z), p3 = kr_fmul(a, v.w);
+            // slot k: dim 4c + (k + rot) % 4
+            const float a0 = rot & 1 ? p1 : p0, a1 = rot & 1 ? p2 : p1, a2 = rot & 1 ? p3 : p2, a3 = rot & 1 ? p0 : p3;
+            float *d = kt + ((size_t)(r >> 2) * hd + 4 * c) * 4 + (r & 3);
+            d[4 * (rot & 3)] = rot & 2 ? a2 : a0;
+            d[4 * ((1 + rot) & 3)] = rot & 2 ? a3 : a1;
+            d[4 * ((2 + rot) & 3)] = rot & 2 ? a0 : a2;
+            d[4 * ((3 + rot) & 3)] = rot & 2 ? a1 : a3;
+        }
+    }
+    __syncthreads();
+    if (tid < hd) {
+        const float4 *p = (const float4 *)kt + tid;   // quad k at p[k * hd]
+        const int nq = n >> 2;
+        float o = 0.0f;
+        float4 a[8], b[8];
+        auto read = [&](float4 (&v)[8], int k0) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) v[k] = p[min(k0 + k, max(nq - 1, 0)) * hd];
+        };
+        auto add = [&](const float4 (&v)[8]) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                o = kr_fadd(o, v[k].x);
+                o = kr_fadd(o, v[k].y);
+                o = kr_fadd(o, v[k].z);
+                o = kr_fadd(o, v[k].w);
+            }
+        };
+        int k = 0;
+        read(a, 0);
+        for (; k + 16 <= nq; k += 16) {
+            read(b, k + 8);
+            __builtin_amdgcn_sched_barrier(0);
+            add(a);
+            read(a, k + 16);
+            __builtin_amdgcn_sched_barrier(0);
+            add(b);
+        }
+        for (; k < nq; k++) {
+            const float4 v = p[k * hd];
+            o = kr_fadd(o, v.x);
+            o = kr_fadd(o, v.y);
+            o = kr_fadd(o, v.z);
+            o = kr_fadd(o, v.w);
+        }
+        const float *tail = (const float *)(p + nq * hd);   // a partial quad's live positions only
+        for (int i = 0; i < (n & 3); i++) o = kr_fadd(o, tail[i]);
+        ao[(size_t)h * hd + tid] = o;
+    }
+}
+
+template <int KT>
+__global__ void __launch_bounds__(AS_NT) k_attn_short(float *ao, const float *q, const KvView kv, int group, int hd,
+                                                      int kv_dim, int window, float scale, const int *pos_p,
+                                                      int nmax) {
+    __shared__ AsLds S;
+    const int pos = *pos_p, first = attn_first(pos, window), n = min(pos + 1 - first, nmax);
+    const int np = (n + AS_NT / (hd / 4) - 1) / (AS_NT / (hd / 4));
+    if (np <= 2) attn_short<KT, 2>(S, ao, q, kv, group, hd, kv_dim, scale, first, n);
+    else if (np <= 5) attn_short<KT, 5>(S, ao, q, kv, group, hd, kv_dim, scale, first, n);
+    else attn_short<KT, AS_NP>(S, ao, q, kv, group, hd, kv_dim, scale, first, n);
+}
+
 // ---- F16 / Q8 cache rows ----
 
 // store_kv (model/transformer.c:191-205) for the positions *pos0 + t: the
@@ -1484,6 +1670,15 @@ static void attention(float *ao, float *att, const float *q, const KvView &kv, i
         return;
     }
     const int group = n_heads / n_kv_heads, kv_dim = n_kv_heads * head_dim;
+    if constexpr (KT != KV_Q8) {   // decode whose rows, at most this long, run in one launch
+        const int rows = window && window <= max_pos ? window : max_pos + 1;
+        if (ntok == 1 && cap <= 0.0f && head_dim <= 256 && rows <= as_positions(head_dim)) {
+            hipLaunchKernelGGL(k_attn_short<KT>, dim3(n_heads), dim3(AS_NT), 0, kr_stream(), ao, q, kv, group,
+                               head_dim, kv_dim, window, scale, pos, rows);
+            kr_check_launch("attention");
+            return;
+        }
+    }
     // the per-token score kernels' LDS: the group's queries and a K tile of
     // tt positions. F32/F16 tiles of wide heads (Gemma's 256) take AT_TD
     // positions; the int8 Q8 tile fits at AT_T up to heads of 512 and more.
@@ -1696,6 +1891,10 @@ extern "C" void krh_attention_noalloc(float *ao, const float *q, const float *kc
     }
     attention<KV_F32>(ao, g_scratch_ptr[dev], q, f32_view(kc, vc), n_heads, n_kv_heads, head_dim, max_seq, window,
                       scale, pos, 1, max_seq - 1);
+}
+
+extern "C" int krh_attention_short(int head_dim, int kv_type) {
+    return head_dim > 0 && head_dim <= 256 && head_dim % 4 == 0 && kv_type != ML_Q8_0 ? as_positions(head_dim) : 0;
 }
 
 extern "C" void krh_set_attn_rb_min(int min_wg) { g_rb_min_wg = min_wg < 0 ? 0 : min_wg; }

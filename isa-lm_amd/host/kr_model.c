@@ -191,7 +191,11 @@ struct kr_state {
     void *mem;
     float *h_logits;          /* pinned */
     int *h_ints;              /* pinned: tok, pos */
-    krh_graph *g_logits, *g_greedy, *g_prefill, *g_sample;
+    /* a step's graphs by kind: [1] for positions below short_n, whose
+     * attention is one launch (krh_attention_short), [0] for any position */
+    krh_graph *graphs[4][2];
+    int short_n;              /* 0: the two are the same, only [0] is captured */
+    int att_last;             /* the last position the attention being issued has to serve */
     krh_sampler *smp;         /* the device sampler of kr_generate, or NULL: greedy */
     int batch;                /* tokens per batched prefill step; 1: token by token */
     int eager;                /* issue ops directly instead of replaying graphs */
@@ -304,11 +308,12 @@ static void issue_step(kr_state *s, int cls) {
         /* each norm runs inside the launch that consumes it, under that
          * launch's first weight loads */
         if (s->kv_type == ML_F32) {
+            const ml_kv_layer kv = kv_layer(s, l);
             float *kc = (float *)s->kcache + (size_t)l * lkv, *vc = (float *)s->vcache + (size_t)l * lkv;
             krh_rmsnorm_matvec_qkv(s->q, kc, vc, &D->wq, &D->wk, &D->wv, D->bq, D->bk, D->bv, s->x, D->attn_norm,
                                    c->norm_eps, cs, sn, c->head_dim, s->pos);
-            krh_attention(s->ao, NULL, NULL, s->att, s->q, kc, vc, c->n_heads, c->n_kv_heads, c->head_dim,
-                          c->max_seq, L->window, c->attn_scale, s->pos);
+            krh_attention_kv(s->ao, s->att, s->q, &kv, c->n_heads, c->n_kv_heads, c->head_dim, c->max_seq,
+                             c->attn_scale, s->pos, 1, s->att_last);
         } else {
             const ml_kv_layer kv = kv_layer(s, l);
             if (s->kv_type == ML_F16) {   /* the rows rounded to halves in the projection's epilogue */
@@ -316,7 +321,7 @@ static void issue_step(kr_state *s, int cls) {
                 krh_rmsnorm_matvec_qkv_f16(s->q, kh, vh, &D->wq, &D->wk, &D->wv, D->bq, D->bk, D->bv, s->x,
                                            D->attn_norm, c->norm_eps, cs, sn, c->head_dim, s->pos);
                 krh_attention_kv(s->ao, s->att, s->q, &kv, c->n_heads, c->n_kv_heads, c->head_dim, c->max_seq,
-                                 c->attn_scale, s->pos, 1, c->max_seq - 1);
+                                 c->attn_scale, s->pos, 1, s->att_last);
             } else {   /* Q8: the score launch stores row *pos (store_kv) before reading it */
                 krh_rmsnorm_matvec_qkv_stage(s->q, s->kst, s->vst, &D->wq, &D->wk, &D->wv, D->bq, D->bk, D->bv, s->x,
                                              D->attn_norm, c->norm_eps, cs, sn, c->head_dim, s->pos);
@@ -361,7 +366,7 @@ static void issue_family_layer(kr_state *s, int l, const float *cs, const float 
     else
         store_kv(s, l, s->kst, s->vst, 1);
     krh_attention_kv_softcap(s->ao, s->att, s->q, &kv, c->n_heads, c->n_kv_heads, c->head_dim, c->max_seq,
-                             c->attn_scale, s->pos, 1, c->max_seq - 1, c->attn_softcap);
+                             c->attn_scale, s->pos, 1, s->att_last, c->attn_softcap);
     if (D->post_attn_norm) {
         krh_matvec_f(s->yb, &D->wo, s->ao, 0);
         krh_rmsnorm(s->yb, s->yb, D->post_attn_norm, c->dim, c->norm_eps);
@@ -386,7 +391,7 @@ static void issue_family_layer(kr_state *s, int l, const float *cs, const float 
     }
 }
 
-enum { STEP_LOGITS = 0, STEP_GREEDY = 1, STEP_PREFILL = 2, STEP_SAMPLE = 3 };
+enum { STEP_LOGITS = 0, STEP_GREEDY = 1, STEP_PREFILL = 2, STEP_SAMPLE = 3, STEP_KINDS = 4 };
 
 /* The ops of one replayed step: STEP_LOGITS (ml_forward), STEP_GREEDY
  * (ml_forward + the greedy pick, appended to the id log), STEP_PREFILL (the
@@ -400,27 +405,37 @@ static void issue(kr_state *s, int kind) {
     if (kind == STEP_PREFILL) krh_advance(s->pos);
 }
 
-static ml_status capture(kr_state *s, krh_graph **g, int kind) {
-    ml_status st = krh_graph_begin();
-    if (st != ML_OK) return kr_seterr(st, "%s", krh_last_error());
-    issue(s, kind);
-    st = krh_graph_end(g);
-    return st == ML_OK ? ML_OK : kr_seterr(st, "%s", krh_last_error());
+static ml_status capture(kr_state *s, int kind) {
+    for (int i = 0; i < (s->short_n ? 2 : 1); i++) {
+        ml_status st = krh_graph_begin();
+        if (st != ML_OK) return kr_seterr(st, "%s", krh_last_error());
+        s->att_last = i ? s->short_n - 1 : s->m->cfg.max_seq - 1;
+        issue(s, kind);
+        st = krh_graph_end(&s->graphs[kind][i]);
+        if (st != ML_OK) return kr_seterr(st, "%s", krh_last_error());
+    }
+    return ML_OK;
 }
 
-/* Runs a step: replays its graph, or issues its ops one by one when the
- * state is eager (KRAFLA_EAGER=1 in the environment: for profilers that
- * trace kernel dispatches, and for debugging) */
-static ml_status run_step(kr_state *s, int kind) {
+static void free_graphs(kr_state *s, int kind) {
+    for (int i = 0; i < 2; i++) {
+        krh_graph_free(s->graphs[kind][i]);
+        s->graphs[kind][i] = NULL;
+    }
+}
+
+/* Runs a step at position pos (the value of *s->pos when it runs): replays
+ * its graph, or issues its ops one by one when the state is eager
+ * (KRAFLA_EAGER=1 in the environment: for profilers that trace kernel
+ * dispatches, and for debugging) */
+static ml_status run_step(kr_state *s, int kind, int pos) {
+    const int i = pos < s->short_n;
     if (s->eager) {
+        s->att_last = i ? s->short_n - 1 : s->m->cfg.max_seq - 1;
         issue(s, kind);
         return krh_status();
     }
-    const krh_graph *g = kind == STEP_LOGITS   ? s->g_logits
-                         : kind == STEP_GREEDY ? s->g_greedy
-                         : kind == STEP_SAMPLE ? s->g_sample
-                                               : s->g_prefill;
-    return krh_graph_launch(g);
+    return krh_graph_launch(s->graphs[kind][i]);
 }
 
 ml_status kr_state_new(kr_state **out, kr_model *m, int kv_type) {
@@ -490,9 +505,11 @@ ml_status kr_state_new(kr_state **out, kr_model *m, int kv_type) {
     s->batch = c->max_seq < KR_PREFILL_STEP ? c->max_seq : KR_PREFILL_STEP;
     const char *ev = getenv("KRAFLA_EAGER");
     s->eager = ev && ev[0] == '1';
-    if (st == ML_OK && !s->eager) st = capture(s, &s->g_logits, STEP_LOGITS);
-    if (st == ML_OK && !s->eager) st = capture(s, &s->g_greedy, STEP_GREEDY);
-    if (st == ML_OK && !s->eager) st = capture(s, &s->g_prefill, STEP_PREFILL);
+    const int one = krh_attention_short(c->head_dim, kv_type);
+    s->short_n = c->attn_softcap > 0.0f || one >= c->max_seq ? 0 : one;
+    if (st == ML_OK && !s->eager) st = capture(s, STEP_LOGITS);
+    if (st == ML_OK && !s->eager) st = capture(s, STEP_GREEDY);
+    if (st == ML_OK && !s->eager) st = capture(s, STEP_PREFILL);
     if (st != ML_OK) {
         kr_state_free(s);
         return kr_seterr(st, "%s", krh_last_error());
@@ -504,10 +521,7 @@ ml_status kr_state_new(kr_state **out, kr_model *m, int kv_type) {
 void kr_state_free(kr_state *s) {
     if (!s) return;
     krh_free(s->bmem);
-    krh_graph_free(s->g_logits);
-    krh_graph_free(s->g_greedy);
-    krh_graph_free(s->g_prefill);
-    krh_graph_free(s->g_sample);
+    for (int k = 0; k < STEP_KINDS; k++) free_graphs(s, k);
     krh_sampler_free(s->smp);
     krh_free(s->mem);
     krh_host_free(s->h_logits);
@@ -516,14 +530,14 @@ void kr_state_free(kr_state *s) {
 }
 
 ml_status kr_state_set_sampler(kr_state *s, const krh_sampler_opts *o) {
-    krh_graph_free(s->g_sample);
+    free_graphs(s, STEP_SAMPLE);
     krh_sampler_free(s->smp);
-    s->g_sample = NULL;
     s->smp = NULL;
     if (!o) return ML_OK;
     ml_status st = krh_sampler_new(&s->smp, s->m->cfg.vocab, o);
-    if (st == ML_OK && !s->eager) st = capture(s, &s->g_sample, STEP_SAMPLE);
+    if (st == ML_OK && !s->eager) st = capture(s, STEP_SAMPLE);
     if (st != ML_OK) {
+        free_graphs(s, STEP_SAMPLE);
         krh_sampler_free(s->smp);
         s->smp = NULL;
         return kr_seterr(st, "%s", krh_last_error());
@@ -569,7 +583,7 @@ ml_status kr_forward(kr_state *s, int token, int pos, float *logits) {
     const ml_config *c = &s->m->cfg;
     if (pos < 0 || pos >= c->max_seq || token < 0 || token >= c->vocab) return ML_E_SHAPE;
     ml_status st = set_ints(s, token, pos);
-    if (st == ML_OK) st = run_step(s, STEP_LOGITS);
+    if (st == ML_OK) st = run_step(s, STEP_LOGITS, pos);
     if (st == ML_OK && logits) st = krh_copy_d2h(logits, s->logits, sizeof(float) * c->vocab);
     return st == ML_OK ? dev_status() : st;
 }
@@ -785,7 +799,7 @@ ml_status kr_prefill(kr_state *s, const int *tokens, int n, int pos0, float *log
     if (n == 0) return ML_OK;
     ml_status st = krh_copy_h2d(s->prompt + pos0, tokens, sizeof(int) * (size_t)n);
     if (st == ML_OK) st = set_ints(s, 0, pos0);
-    for (int i = 0; st == ML_OK && i < n; i++) st = run_step(s, STEP_PREFILL);
+    for (int i = 0; st == ML_OK && i < n; i++) st = run_step(s, STEP_PREFILL, pos0 + i);
     return st == ML_OK ? dev_status() : st;
 }
 
@@ -820,7 +834,7 @@ int kr_generate(kr_state *s, const int *prompt, int np, int steps, int *out, dou
         if (set_ints(s, token, pos) != ML_OK) return -1;
         const int kind = s->smp ? STEP_SAMPLE : STEP_GREEDY;
         for (; pos < steps; pos++)
-            if (run_step(s, kind) != ML_OK) return -1;
+            if (run_step(s, kind, pos) != ML_OK) return -1;
         if (dev_status() != ML_OK) return -1;
         if (krh_copy_d2h(out + n, s->log + first + 1, sizeof(int) * (size_t)(steps - first)) != ML_OK) return -1;
         n += steps - first;

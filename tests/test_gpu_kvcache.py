@@ -251,6 +251,68 @@ def test_attention_batch_blocks(dev, kv_type, nh, nkv, hd, pos0, T, window, choi
         assert np.array_equal(bits(got[t]), bits(out)), t
 
 
+@pytest.mark.parametrize("kv_type", [K.ML_F32, K.ML_F16])
+@pytest.mark.parametrize("nh,nkv,hd", [(6, 6, 48), (14, 2, 64), (4, 1, 128), (2, 1, 256), (3, 3, 32), (4, 2, 20)])
+def test_attention_short_rows(dev, kv_type, nh, nkv, hd):
+    """the one-launch decode attention at its sums' batch and quad edges, over
+    a window, at its longest row, and the first row past it"""
+    if (nh * hd) % 32:
+        nh, nkv = nh * 2, nkv * 2
+    limit = K.hip.krh_attention_short(hd, kv_type)
+    max_seq = limit + 8
+    kvd, qd = nkv * hd, nh * hd
+    if kv_type == K.ML_F32:
+        k, v = f32(RNG.normal(0, 1, max_seq * kvd)), f32(RNG.normal(0, 1, max_seq * kvd))
+        kp, vp = dev.put(k).ptr, dev.put(v).ptr
+    else:
+        k, v, _, _ = rand_cache(kv_type, max_seq, kvd, nkv)
+    q = f32(RNG.normal(0, 1, qd))
+    qp, ao, att = dev.put(q).ptr, dev.zeros(4 * qd), dev.zeros(4 * nh * max_seq)
+    scale = float(np.float32(1.0) / np.sqrt(np.float32(hd)))
+    cfg = K.MlConfig(n_heads=nh, n_kv_heads=nkv, head_dim=hd, kv_dim=kvd, q_dim=qd, max_seq=max_seq,
+                     attn_scale=scale)
+    scratch = np.zeros(max_seq, np.float32)
+    rows = [1, 2, 3, 4, 5, 31, 32, 33, 63, 64, 65, 97, limit - 1, limit, limit + 1]
+    for n, window in [(n, 0) for n in rows] + [(limit, 7), (limit + 5, 33), (limit + 8, limit)]:
+        if kv_type == K.ML_F32:
+            dview = K.MlKvLayer(kp, vp, None, None, None, None, window, None, None)
+            hview = O.KvLayer(k.ctypes.data, v.ctypes.data, None, None, None, None, window, None, None)
+        else:
+            dview, hview = views(dev, kv_type, k, v, None, None, window)
+        K.hip.krh_attention_kv(ao.ptr, att.ptr, qp, C.byref(dview), nh, nkv, hd, max_seq, scale,
+                               dev.put(np.array([n - 1], np.int32)).ptr, 1, max(n, min(limit, max_seq)) - 1)
+        ok()
+        out = np.zeros(qd, np.float32)
+        oracle.kro_attention(out.ctypes.data, q.ctypes.data, C.byref(hview), scratch.ctypes.data, C.byref(cfg), n - 1)
+        assert np.array_equal(bits(ao.get(np.float32, qd)), bits(out)), (n, window)
+
+
+@pytest.mark.parametrize("kv_type", [K.ML_F32, K.ML_F16, K.ML_Q8_0])
+def test_forward_across_short_limit(kv_type, workdir):
+    """kr_forward's logits on both sides of the position where a step's graph
+    changes (a context too long for the one-launch attention)"""
+    path = os.path.join(workdir, "short_limit.mlb")
+    spec = dict(K.CONFIGS["llama8b_q8"], dim=128, n_layers=2, n_heads=2, n_kv_heads=1, hidden_dim=64, vocab=96,
+                max_seq=640, std=0.1)
+    if not os.path.exists(path):
+        K.gen_mlb(path, **spec)
+    m = K.Model(path)
+    s = K.State(m, kv_type)
+    om = O.OracleModel(path, kv_type)
+    limit = K.hip.krh_attention_short(64, K.ML_F32)
+    assert limit < 640
+    toks = [int(t) for t in np.random.default_rng(8).integers(0, 96, limit + 3)]
+    s.prefill(toks[:limit - 3], 0)
+    om.prefill(toks[:limit - 3], 0)
+    got = np.empty(m.cfg.vocab, np.float32)
+    for pos in range(limit - 3, limit + 3):
+        s.forward(toks[pos], pos, got)
+        assert np.array_equal(bits(got), bits(om.forward(toks[pos], pos))), pos
+    om.close()
+    s.close()
+    m.close()
+
+
 KV = {"f16": K.ML_F16, "q8": K.ML_Q8_0}
 
 
