@@ -142,7 +142,7 @@ struct MmPre {
 };
 
 // wave-uniform bases of the tile's operands at block 0 (w, d: of the first
-// and, for a SwiGLU pair, the second 64 rows' matrix) and this thread's byte
+// and, for a SwiGLU pair, the second half's matrix) and this thread's byte
 // offsets from them
 template <int NG>
 struct MmTile {
@@ -162,8 +162,13 @@ __device__ __forceinline__ MmTile<NG> mm_tile(const MmArgs &a, const MMat &W, co
     t.w[1] = (PAIR ? W2.q : W.q) + blk * BB;
     t.d[0] = (const uint8_t *)W.d + blk * SB;
     t.d[1] = (const uint8_t *)(PAIR ? W2.d : W.d) + blk * SB;
+    if (PAIR && NG == 2 && __builtin_amdgcn_readfirstlane(tid >> 6) >= 2) {
+        // a 64-row pair's second 32 rows in the loads that take 64 rows at once
+        if (QT != ML_Q8_0) t.w[0] = t.w[1];
+        t.d[0] = t.d[1];
+    }
     // rows past the end re-read the last row (not stored)
-    auto row = [&](int r) { return (uint32_t)(min(rowl + (PAIR ? r & 63 : r), W.rows - 1) - rowl); };
+    auto row = [&](int r) { return (uint32_t)(min(rowl + (PAIR ? r & (16 * NG - 1) : r), W.rows - 1) - rowl); };
 #pragma unroll
     for (int u = 0; u < NG; u++)   // Q8: 8 threads a row; Q4: 4
         t.wo[u] = QT == ML_Q8_0 ? row((tid >> 3) + 32 * u) * nb * BB : row((tid >> 2) + 64 * (u & (NG / 2 - 1))) * nb * BB;
@@ -565,8 +570,8 @@ __global__ void __launch_bounds__(256, 2) k_matmul(const MmArgs a) {
     const int local = (int)blockIdx.x - a.tile0[mi];
     const int rt = local / ntt, tt = local - rt * ntt;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    constexpr bool PAIR = EPI == MM_SWIGLU;   // 64 rows of w1 and the same 64 of w3
-    const int rowl = rt * (PAIR ? 64 : 32 * NG), tokl = tt * TT + 32 * wave;
+    constexpr bool PAIR = EPI == MM_SWIGLU;   // 16 NG rows of w1 and the same of w3
+    const int rowl = rt * (PAIR ? 16 : 32) * NG, tokl = tt * TT + 32 * wave;
     const int nb = a.K / KR_QK;
     float acc[NG][16];
     const MmTile<NG> t = mm_tile<QT, D16, NG, PAIR>(a, W, a.w[1], nb, rowl, tt * TT, tid);
@@ -582,15 +587,15 @@ __global__ void __launch_bounds__(256, 2) k_matmul(const MmArgs a) {
     if constexpr (PAIR) {
         // h = silu(w1 x) * (w3 x) (k_scalar.c:96-98), then its Q8_0 in blocks
         // of 32 rows (k_scalar.c:39-57): a block's 32 values are the 32 lanes
-        // of a half-wave (groups 0, 1: w1 rows; 2, 3: the same w3 rows)
+        // of a half-wave (the first NG / 2 groups: w1 rows; the rest: the same w3 rows)
 #pragma unroll
-        for (int g = 0; g < 2; g++) {
+        for (int g = 0; g < NG / 2; g++) {
             const int row = rowl + 32 * g + (lane & 31);
             const bool bin = rowl + 32 * g < W.rows;   // rows % 32 == 0: whole blocks in or out
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const int t = tokl + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                const float h1 = acc[g][r], h3 = acc[g + 2][r];
+                const float h1 = acc[g][r], h3 = acc[g + NG / 2][r];
                 const float v = kr_fmul(kr_fdiv(h1, kr_fadd(1.0f, kr_expf(-h1))), h3);
                 int8_t q;
                 float d;
@@ -619,8 +624,8 @@ void launch_mm(const MmArgs &a, const MMat &W) {
         return;
     }
     auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, kr_stream(), a); };
-    if (EPI == MM_SWIGLU && a.ng != 4) {
-        kr_fail(ML_E_SHAPE, "matmul: SwiGLU pairs take 128-row tiles", hipSuccess);
+    if (EPI == MM_SWIGLU && a.ng == 1) {
+        kr_fail(ML_E_SHAPE, "matmul: SwiGLU pairs take 128- or 64-row tiles", hipSuccess);
         return;
     }
     if (a.ng == 4) {
@@ -629,16 +634,13 @@ void launch_mm(const MmArgs &a, const MMat &W) {
         } else {
             if (W.d16) go(k_matmul<EPI, ML_Q4_0, 1, 4>); else go(k_matmul<EPI, ML_Q4_0, 0, 4>);
         }
-    } else if constexpr (EPI != MM_SWIGLU) {
-        if (a.ng == 2) {
-            if (W.type == ML_Q8_0) {
-                if (W.d16) go(k_matmul<EPI, ML_Q8_0, 1, 2>); else go(k_matmul<EPI, ML_Q8_0, 0, 2>);
-            } else {
-                if (W.d16) go(k_matmul<EPI, ML_Q4_0, 1, 2>); else go(k_matmul<EPI, ML_Q4_0, 0, 2>);
-            }
-            kr_check_launch("matmul");
-            return;
+    } else if (a.ng == 2) {
+        if (W.type == ML_Q8_0) {
+            if (W.d16) go(k_matmul<EPI, ML_Q8_0, 1, 2>); else go(k_matmul<EPI, ML_Q8_0, 0, 2>);
+        } else {
+            if (W.d16) go(k_matmul<EPI, ML_Q4_0, 1, 2>); else go(k_matmul<EPI, ML_Q4_0, 0, 2>);
         }
+    } else if constexpr (EPI != MM_SWIGLU) {
         if (a.rg == 2) {
             if (W.type == ML_Q8_0) {
                 if (W.d16) go(k_matmul_short<EPI, ML_Q8_0, 1, 2>); else go(k_matmul_short<EPI, ML_Q8_0, 0, 2>);
@@ -755,8 +757,10 @@ extern "C" void krh_matmul_swiglu(int8_t *hq, float *hdT, const krh_mat *w1, con
     a.nmat = 1;
     a.tile0[0] = 0;
     const int ntt = (T + MM_TT - 1) / MM_TT;
-    a.ng = 4;
-    a.tile0[1] = (w1->rows + 63) / 64 * ntt;
+    // as mm_plan: 128-row tiles once the 64-row ones are more than a round of two a CU
+    const long t32 = (long)(w1->rows / 32) * ntt, cus = krh_device_cus() > 0 ? krh_device_cus() : 256;
+    a.ng = t32 > 2 * cus ? 4 : 2;
+    a.tile0[1] = (w1->rows + 16 * a.ng - 1) / (16 * a.ng) * ntt;
     a.xq = xq;
     a.xdT = xdT;
     a.ldx = ldx;
