@@ -42,8 +42,11 @@ constexpr int SM_NT = 1024;                                       // threads of 
 // its length, so the fewer the better: with 12,288 terms the 128k vocabulary's
 // softmax took 11 groups and a nucleus of 26k candidates 3 (a top-p draw over
 // 128,256 ids, with the scaling pass gone and the sort's empty workgroups
-// returning at once: 181 -> 125 us).
+// returning at once: 181 -> 125 us; 116 with the draw's second sum gone).
 constexpr int SM_G = 32768;
+// and per group of the sorted draws, whose answer lies early: two more
+// searches of the first group cost no sum of their own
+constexpr int SM_GF = 16384;
 constexpr int SM_RT = 256, SM_ROWS = 4, SM_E = SM_RT * SM_ROWS;   // radix sort: threads, rows, ids per workgroup
 constexpr int SM_HB = 16;                                         // digit counts read at a time
 constexpr int SM_EB = 2048;                                       // ids per elementwise workgroup (256 x 8)
@@ -173,63 +176,88 @@ __device__ __forceinline__ void sm_fill(float *t, Term term, int g0, int ng, int
     }
 }
 
+// The group of terms an ordered-prefix search summed last: terms g0 ..
+// g0 + ng - 1 are in LDS, S and E the sums before and after them, the chunk
+// starts recorded.
+struct SmGroup {
+    int g0, ng;
+    float S, E;
+};
+
+// The first term of the group whose partial sum passes thr (thr < E), and that
+// partial sum: the first chunk whose end passes thr holds it, and one lane
+// runs that chunk's chain from its recorded start. All SM_NT threads call it.
+__device__ int sm_find(const SmGroup &G, float thr, unsigned char *lds, float &val) {
+    const float *t = (const float *)lds;
+    const unsigned *cst = (const unsigned *)(lds + SM_TERMS + SM_SCR);
+    int *res = (int *)(lds + SM_TERMS + SM_SCR + SM_CST);
+    const int tid = sm_tid(), lane = tid & 63, sh = sc_log_len(G.ng), C = sc_chunks(G.ng), L = 1 << sh;
+    if (tid < 64) {
+        int c = -1;
+        if (cst[C] == 0) {
+            for (int c0 = 0; c0 < C && c < 0; c0 += 64) {
+                const int cc = c0 + lane;
+                const float end = cc + 1 < C ? __uint_as_float(cst[min(cc + 1, C - 1)]) : G.E;
+                const unsigned long long b = __ballot(cc < C && thr < end);
+                if (b) c = c0 + __builtin_ctzll(b);
+            }
+        }
+        if (lane == 0) {
+            // c < 0: the sum went through the sequential loop; so does the search
+            float s = c >= 0 ? __uint_as_float(cst[c]) : G.S;
+            const int i0 = c >= 0 ? c * L : 0, i1 = c >= 0 ? min(i0 + L, G.ng) : G.ng;
+            int f = G.ng - 1;
+            for (int i = i0; i < i1; i++) {
+                s = kr_fadd(s, t[sc_at(i, sh)]);
+                if (thr < s) {
+                    f = i;
+                    break;
+                }
+            }
+            res[0] = G.g0 + f;
+            res[1] = __float_as_int(s);
+        }
+    }
+    __syncthreads();
+    val = __int_as_float(res[1]);
+    const int r = res[0];
+    __syncthreads();
+    return r;
+}
+
 // The first i < m with thr < term(0) + ... + term(i), the sum formed one add
 // at a time from +0 (model/sampler.c:63-70, :113-128, :140-151); -1 when none.
-// val: that partial sum, or the whole sum. SM_G terms at a time go to LDS;
-// the group whose end passes thr is searched from the chunk starts its
-// ordered sum recorded: the first chunk whose end passes thr holds the
-// answer, and one lane runs that chunk's chain from its true start. All
-// SM_NT threads call it.
-template <class Term>
-__device__ int sm_first_above(Term term, int m, float thr, unsigned char *lds, float &val) {
+// val: that partial sum, or the whole sum. GT terms at a time go to LDS; the
+// group whose end passes thr is searched (sm_find), and grp describes the
+// last group summed. All SM_NT threads call it.
+template <int GT, class Term>
+__device__ int sm_first_above(Term term, int m, float thr, unsigned char *lds, float &val, SmGroup &grp) {
+    static_assert(GT <= SM_G, "the group fits the LDS layout");
     float *t = (float *)lds;
     unsigned char *scr = lds + SM_TERMS;
     unsigned *cst = (unsigned *)(scr + SM_SCR);
-    int *res = (int *)(lds + SM_TERMS + SM_SCR + SM_CST);
-    const int tid = sm_tid(), lane = tid & 63;
     float S = 0.0f;
-    for (int g0 = 0; g0 < m; g0 += SM_G) {
-        const int ng = min(SM_G, m - g0), sh = sc_log_len(ng), C = sc_chunks(ng), L = 1 << sh;
+    for (int g0 = 0; g0 < m; g0 += GT) {
+        const int ng = min(GT, m - g0), sh = sc_log_len(ng);
         sm_fill(t, term, g0, ng, sh);
         __syncthreads();
         const float E = kr_spec_sum<SM_NT, true>(t, ng, scr, S, cst);
-        if (thr < E) {
-            if (tid < 64) {
-                int c = -1;
-                if (cst[C] == 0) {
-                    for (int c0 = 0; c0 < C && c < 0; c0 += 64) {
-                        const int cc = c0 + lane;
-                        const float end = cc + 1 < C ? __uint_as_float(cst[min(cc + 1, C - 1)]) : E;
-                        const unsigned long long b = __ballot(cc < C && thr < end);
-                        if (b) c = c0 + __builtin_ctzll(b);
-                    }
-                }
-                if (lane == 0) {
-                    // c < 0: the sum went through the sequential loop; so does the search
-                    float s = c >= 0 ? __uint_as_float(cst[c]) : S;
-                    const int i0 = c >= 0 ? c * L : 0, i1 = c >= 0 ? min(i0 + L, ng) : ng;
-                    int f = ng - 1;
-                    for (int i = i0; i < i1; i++) {
-                        s = kr_fadd(s, t[sc_at(i, sh)]);
-                        if (thr < s) {
-                            f = i;
-                            break;
-                        }
-                    }
-                    res[0] = g0 + f;
-                    res[1] = __float_as_int(s);
-                }
-            }
-            __syncthreads();
-            val = __int_as_float(res[1]);
-            const int r = res[0];
-            __syncthreads();
-            return r;
-        }
+        grp = { g0, ng, S, E };
+        if (thr < E) return sm_find(grp, thr, lds, val);
         S = E;
     }
     val = S;
     return -1;
+}
+
+// The same search again over the first m terms, whose sum is whole, with
+// another threshold: from the recorded sums when the last search's group was
+// the first one (every partial sum up to m is in it), else anew.
+template <int GT, class Term>
+__device__ int sm_again(Term term, int m, float whole, float thr, unsigned char *lds, float &val, SmGroup &grp) {
+    if (grp.g0 != 0) return sm_first_above<GT>(term, m, thr, lds, val, grp);
+    val = whole;
+    return thr < whole ? sm_find(grp, thr, lds, val) : -1;
 }
 
 // The penalty alone (one workgroup), ahead of the kernels that read the logits.
@@ -332,7 +360,8 @@ __global__ void __launch_bounds__(SM_NT) k_smp_main(int *tok, int n, Dev d, int 
             int t = decided;
             if (t < 0) {
                 float v;
-                const int j = sm_first_above([&](int i) { return sm_prob(p[i], inv); }, n, coin, sm_lds, v);
+                SmGroup grp;
+                const int j = sm_first_above<SM_G>([&](int i) { return sm_prob(p[i], inv); }, n, coin, sm_lds, v, grp);
                 t = j >= 0 ? j : n - 1;
             }
             if (tid == 0) sm_finish(t, tok, pos, log, d);
@@ -489,17 +518,18 @@ __global__ void __launch_bounds__(SM_NT) k_smp_final(int *tok, int n, Dev d, int
         const unsigned *keys = d.keys + d.vocab;
         const int *ids = d.ids + d.vocab;
         auto term = [&](int i) { return __uint_as_float(~keys[i]); };
+        SmGroup grp;
         if constexpr (MODE == SM_TOPK) {
             const int k = d.topk;
             float total, cum, c;
-            sm_first_above(term, k, INFINITY, sm_lds, total);
+            sm_first_above<SM_GF>(term, k, INFINITY, sm_lds, total, grp);
             int last = k - 1;
             if (d.topp > 0.0f && d.topp < 1.0f) {
-                const int i = sm_first_above(term, k, kr_fmul(d.topp, total), sm_lds, cum);
+                const int i = sm_again<SM_GF>(term, k, total, kr_fmul(d.topp, total), sm_lds, cum, grp);
                 if (i >= 0) last = i;
                 total = cum;
             }
-            const int j = sm_first_above(term, last + 1, kr_fmul(coin, total), sm_lds, c);
+            const int j = sm_again<SM_GF>(term, last + 1, total, kr_fmul(coin, total), sm_lds, c, grp);
             t = ids[j >= 0 ? j : last];
         } else {
             const int m = d.meta[MT_M];
@@ -508,9 +538,9 @@ __global__ void __launch_bounds__(SM_NT) k_smp_final(int *tok, int n, Dev d, int
                 t = sm_argmax([&](int i) { return sm_prob(d.probs[i], inv); }, n, rv, ri);
             } else {
                 float cum, c;
-                const int i = sm_first_above(term, m, d.topp, sm_lds, cum);
+                const int i = sm_first_above<SM_GF>(term, m, d.topp, sm_lds, cum, grp);
                 const int last = i >= 0 ? i : m - 1;
-                const int j = sm_first_above(term, last + 1, kr_fmul(coin, cum), sm_lds, c);
+                const int j = sm_again<SM_GF>(term, last + 1, cum, kr_fmul(coin, cum), sm_lds, c, grp);
                 t = ids[j >= 0 ? j : last];
             }
         }
