@@ -228,6 +228,9 @@ constexpr int RB_PC = 8;             // K tiles per scores workgroup, at most
 // 300 tokens 78, 77, 90, 90; 32 heads of 64, 256 tokens 60, 45, 45, 47.
 static int g_rb_min_wg = 512;
 static bool rb_fills(long wgs) { return 2 * wgs >= g_rb_min_wg; }
+// heads with a form of their own for launches without a window (the others run
+// the windowed form with none)
+constexpr bool rb_plain(int hd) { return hd == 64 || hd == 128; }
 static bool rb_dims(int hd) { return hd == 48 || hd == 64 || hd == 80 || hd == 96 || hd == 128 || hd == 256; }
 constexpr int RB_NT128 = 512;        // threads of the 128-dim heads' workgroups (4 outputs' rows a lane, LDS for 2
                                      // workgroups a CU: 4 waves a SIMD; 256 threads gave 2 and measured the same)
@@ -1600,6 +1603,16 @@ __global__ void __launch_bounds__(64) k_store_kv(const KvOut o, const float *k, 
     if (lane == 0) (which ? o.vd : o.kd)[(size_t)(*pos0 + t) * o.n_kv + h] = zero ? 0.0f : kr_fdiv(m, 127.0f);
 }
 
+// The decode kernels first and together in the code object: a token's three
+// attention launches then run from one stretch of it.
+template __global__ void k_attn_scores<AT_TD, false>(float *, const float *, const float *, int, int, int, int, int, float,
+                                                     const int *);
+template __global__ void k_attn_softmax<SMX_THREADS, AT_CHUNK, false, false>(float *, int, int, const int *);
+template __global__ void k_attn_mix<16>(float *, const float *, const float *, int, int, int, int, int, const int *);
+template __global__ void k_attn_mix<8>(float *, const float *, const float *, int, int, int, int, int, const int *);
+template __global__ void k_attn_mix<32>(float *, const float *, const float *, int, int, int, int, int, const int *);
+template __global__ void k_attn_mix<64>(float *, const float *, const float *, int, int, int, int, int, const int *);
+
 }   // namespace
 
 // ---- C ABI ----
@@ -1617,8 +1630,10 @@ static void launch_mix(const dim3 &grid, int ntok, float *ao, const float *att, 
                 hipLaunchKernelGGL(kern, rgrid, dim3(4 * rb_cw(HD)), 0, kr_stream(), ao, att, kv, group, kv_dim,
                                    max_seq, window, pos, ntok);
             };
-            if (window) run(k_attn_mix_rb<HD, KT, true>);
-            else run(k_attn_mix_rb<HD, KT, false>);
+            if constexpr (rb_plain(HD)) {
+                if (!window) return run(k_attn_mix_rb<HD, KT, false>);
+            }
+            run(k_attn_mix_rb<HD, KT, true>);
         };
         switch (hd) {
         case 48: go(std::integral_constant<int, 48>{}); break;
@@ -1745,8 +1760,10 @@ static void attention(float *ao, float *att, const float *q, const KvView &kv, i
                     hipLaunchKernelGGL(kern, rgrid, dim3(NT), 0, kr_stream(), att, q, kv, group, kv_dim, max_seq,
                                        window, scale, pos, ntok, pc);
                 };
-                if (window) run(k_attn_scores_rb<HD, KT, NT, true, HS>);
-                else run(k_attn_scores_rb<HD, KT, NT, false, HS>);
+                if constexpr (rb_plain(HD)) {
+                    if (!window) return run(k_attn_scores_rb<HD, KT, NT, false, HS>);
+                }
+                run(k_attn_scores_rb<HD, KT, NT, true, HS>);
             };
             using std::integral_constant;
             const integral_constant<int, 256> t256{};

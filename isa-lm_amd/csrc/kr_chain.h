@@ -523,15 +523,13 @@ __device__ __forceinline__ float kr_spec_sum(float *t, int n, unsigned char *lds
     return *res;
 }
 
-// The ordered sum by the workgroup's first wave alone (n <= SC_SHORT), as
-// kr_spec_sum otherwise: the same terms, calling rules and bits (+0 start).
-// The line: 288 terms (a 15M model's norms) one by one take the FFN of a token
-// from 10.9 to 9.5 us; 896 terms (the 0.5B shape's) were slower that way (its
-// 31 decoded tokens and prompt 41.2 ms against 40.7).
+// The ordered sum by the workgroup's first wave alone, as kr_spec_sum
+// otherwise: the same terms, calling rules and bits (+0 start). Kernels take
+// it for n <= SC_SHORT. The line: 288 terms (a 15M model's norms) one by one
+// take the FFN of a token from 10.8 to 9.45 us; 896 terms (the 0.5B shape's)
+// were slower that way (its prompt and 32 decoded tokens 41.2 ms against 40.7).
 constexpr int SC_SHORT = 640;
-template <int NT>
-__device__ __forceinline__ float kr_sum_any(float *t, int n, unsigned char *lds) {
-    if (n > SC_SHORT) return kr_spec_sum<NT>(t, n, lds);
+__device__ __forceinline__ float kr_short_sum(const float *t, int n, unsigned char *lds) {
     float *res = (float *)lds;
     if (threadIdx.x < 64) {
         const float s = sc_short(t, n, 0.0f);

@@ -16,3 +16,6 @@ ml_status kr_attn_setup(int dev);
 // kr_family.hip: soft-caps the attention scratch's scores in place, in the
 // layout the attention launches of ntok tokens use
 void kr_softcap_scores(float *att, int n_heads, int max_seq, int window, const int *pos, int ntok, float cap);
+// kr_matvec_short.hip: launches a normalizing matvec whose sum is short; args
+// is the caller's MvArgs (kr_matvec.h)
+void kr_matvec_short(int epi, bool mixed, int type, int d16, const void *args, size_t bytes, int grid, size_t lds);
