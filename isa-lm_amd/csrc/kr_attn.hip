@@ -1826,8 +1826,11 @@ static void attention(float *ao, float *att, const float *q, const KvView &kv, i
         // (measured: 1B-shape 4000-token prompt 59.9k -> 61.7k tok/s; rows
         // up to 2048 run faster one wave each), the ordered sum's lean form
         // (90 VGPRs against 111: 5 waves a SIMD; 64.5k -> 65.5k)
-        hipLaunchKernelGGL((k_attn_softmax<256, 4096, true>), dim3(n_heads, 1, ntok), dim3(256), 0, kr_stream(), att,
-                           max_seq, window, pos);
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3(n_heads, 1, ntok), dim3(256), 0, kr_stream(), att, max_seq, window, pos);
+        };
+        if (window) go(k_attn_softmax<256, 4096, true, true>);
+        else go(k_attn_softmax<256, 4096, true, false>);
     } else if (ntok > 1 && nrow_max <= SM_WN / 2) {   // prefill rows of up to 2048 scores: one wave each
         const int tcap = sc_terms_cap(nrow_max), scr = (sc_lds_bytes(nrow_max, 64) + 15) / 16 * 16;
         const size_t per_wave = 4 * (size_t)tcap + scr;
