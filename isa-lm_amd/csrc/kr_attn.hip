@@ -1388,8 +1388,9 @@ __global__ void __launch_bounds__(64) k_attn_mix_batch_kv(float *ao, const float
 // A query head's whole attention in one workgroup, for rows of scores whose K
 // rows fit in LDS together (AS_LDS: 559 positions of 64 dims). The three
 // launches of a longer row spend most of such a token on their gaps, their
-// loads' latencies and the ordered sum's fixed cost: 17.7 us a layer for 14
-// heads of 64 dims at position 530 against the one launch's 9.1. K and V are
+// loads' latencies and the ordered sum's fixed cost: for 6 heads of 48 dims at
+// positions up to 136 they took 14.7 us a layer and two gaps, this launch 6.7;
+// for 14 heads of 64 dims at 530 positions 17.7 and the gaps against 14.4. K and V are
 // loaded together up front; V waits in registers while the scores run from
 // K's LDS copy, then its products with the weights take that copy's place.
 //   scores: a thread per position, its ordered dot from LDS;
