@@ -1386,7 +1386,7 @@ __global__ void __launch_bounds__(64) k_attn_mix_batch_kv(float *ao, const float
 // ---- decode over a short context: one launch ----
 
 // A query head's whole attention in one workgroup, for rows of scores whose K
-// rows fit in LDS together (AS_LDS: 559 positions of 64 dims). The three
+// rows fit in LDS together (AS_LDS: 572 positions of 64 dims). The three
 // launches of a longer row spend most of such a token on their gaps, their
 // loads' latencies and the ordered sum's fixed cost: for 6 heads of 48 dims at
 // positions up to 136 they took 14.7 us a layer and two gaps, this launch 6.7;
