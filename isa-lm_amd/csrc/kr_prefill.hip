@@ -86,20 +86,33 @@ constexpr int MM_TT = 128;   // tokens per workgroup
 template <int D16> struct MmScale { using T = uint32_t; };
 template <> struct MmScale<1> { using T = uint16_t; };
 
-// The sum of row `row` and token t of matrix mi, stored as the launch asks;
-// lanes 2 i and 2 i + 1 hold neighbouring rows of one token.
+// Where matrix mi's sums go, read once before the epilogue (read in mm_emit,
+// the compiler selected the argument's address and each of a lane's 16 to 64
+// sums waited for its own scalar loads: 1 us of a 14336 x 64 product's 6.3
+// with 100 tokens)
+struct MmOut {
+    float *y;
+    const float *bias;
+    int mi, rows, ldy;
+};
+__device__ __forceinline__ MmOut mm_out(const MmArgs &a, int mi, int rows) {
+    MmOut o = { a.y[0], a.bias[0], mi, rows, a.ldy[0] };
+    if (mi == 1) o = { a.y[1], a.bias[1], mi, rows, a.ldy[1] };
+    if (mi == 2) o = { a.y[2], a.bias[2], mi, rows, a.ldy[2] };
+    return o;
+}
+
+// The sum of row `row` and token t, stored as the launch asks; lanes 2 i and
+// 2 i + 1 hold neighbouring rows of one token.
 template <int EPI>
-__device__ __forceinline__ void mm_emit(const MmArgs &a, int mi, int rows, int row, int t, float v) {
-    float *Y = mi == 0 ? a.y[0] : (mi == 1 ? a.y[1] : a.y[2]);
-    const int ldy = mi == 0 ? a.ldy[0] : (mi == 1 ? a.ldy[1] : a.ldy[2]);
-    const bool rin = row < rows;
+__device__ __forceinline__ void mm_emit(const MmArgs &a, const MmOut &out, int row, int t, float v) {
+    const bool rin = row < out.rows;
     if (EPI == MM_QKV) {
         // bias (model/transformer.c:276-277), then RoPE on q and k
         // (k_scalar.c:79-94): rows 2i, 2i+1 sit in lanes 2i, 2i+1
-        const float *bias = mi == 0 ? a.bias[0] : (mi == 1 ? a.bias[1] : a.bias[2]);
-        if (bias && rin) v = kr_fadd(v, bias[row]);
+        if (out.bias && rin) v = kr_fadd(v, out.bias[row]);
         const float o = __shfl_xor(v, 1);
-        if (mi < 2) {
+        if (out.mi < 2) {
             const int hd = a.head_dim, j = row % hd, h2 = hd >> 1;
             const int pos = a.pos0 + (t < a.T ? t : 0);
             const float c = a.rope_cos[(size_t)pos * h2 + (j >> 1)];
@@ -108,7 +121,7 @@ __device__ __forceinline__ void mm_emit(const MmArgs &a, int mi, int rows, int r
         }
     }
     if (rin && t < a.T) {
-        float *p = Y + (size_t)t * ldy + row;
+        float *p = out.y + (size_t)t * out.ldy + row;
         if (EPI == MM_ADD) *p = kr_fadd(*p, v);
         else *p = v;
     }
@@ -549,11 +562,12 @@ __global__ void __launch_bounds__(256, 2) k_matmul_short(const MmArgs a) {
     } else {
         ms_sums<QT, 0, RG, false>(acc, L, t, live, tid);
     }
+    const MmOut out = mm_out(a, mi, W.rows);
 #pragma unroll
     for (int g = 0; g < RG; g++)
 #pragma unroll
         for (int r = 0; r < 4; r++)
-            mm_emit<EPI>(a, mi, W.rows, rowl + 16 * g + (lane & 15), tokl + 4 * (lane >> 4) + r, acc[g][r]);
+            mm_emit<EPI>(a, out, rowl + 16 * g + (lane & 15), tokl + 4 * (lane >> 4) + r, acc[g][r]);
 }
 
 // Workgroup = 4 waves over a 32 NG-row x 128-token tile; wave w takes all the
@@ -608,11 +622,12 @@ __global__ void __launch_bounds__(256, 2) k_matmul(const MmArgs a) {
         }
         return;
     }
+    const MmOut out = mm_out(a, mi, W.rows);
 #pragma unroll
     for (int g = 0; g < NG; g++)
 #pragma unroll
         for (int r = 0; r < 16; r++)
-            mm_emit<EPI>(a, mi, W.rows, rowl + 32 * g + (lane & 31), tokl + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3),
+            mm_emit<EPI>(a, out, rowl + 32 * g + (lane & 31), tokl + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3),
                          acc[g][r]);
 }
 
