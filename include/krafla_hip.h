@@ -217,6 +217,10 @@ void krh_matmul(float *Y, int ldy, const krh_mat *W, const int8_t *xq, const flo
  * place, no transpose launch); xd is read for T rows only. */
 void krh_matmul_rows(float *Y, int ldy, const krh_mat *W, const int8_t *xq, const float *xd, int ldx, int T,
                      int accumulate);
+/* The tiles krh_matmul takes for a matrix of these sizes and ntok tokens, or
+ * krh_matmul_swiglu for a pair of them (no counterpart in the reference): 0 to 5
+ * (kr_prefill.hip's MmForm), -1 for no size. */
+int krh_matmul_form(int rows, int cols, int ntok, int swiglu);
 /* The FFN's products and activation of a prompt step in one launch
  * (model/transformer.c:410-413: the w1 and w3 ml_matmul calls, then
  * TOK_DOWN_IN's act_mul and quantize_row_t, :353-355): per

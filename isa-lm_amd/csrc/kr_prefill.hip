@@ -15,6 +15,7 @@
 // transposed activation scales xdT[b][t] through the workgroup's LDS tile. The
 // per-block rescale and the ordered accumulation are 3 VALU operations per
 // output and block (f32 scales: 4), which bound the kernel, not the MFMA.
+#include <algorithm>
 #include "kr_internal.h"
 #include "kr_numerics.h"
 
@@ -45,7 +46,7 @@ struct MmArgs {
     const float *bias[3];
     const float *rope_cos, *rope_sin;
     int head_dim, pos0;
-    int ng, rg;          // row groups per wave: NG of k_matmul, or with ng 1 RG of k_matmul_short
+    int form;            // MmForm
     int8_t *hq;          // MM_SWIGLU: h's Q8_0 quants [T][rows] and scales [rows / 32][ldx]
     float *hdT;
 };
@@ -82,6 +83,16 @@ __device__ __forceinline__ v16i mm_magic() {
 }
 
 constexpr int MM_TT = 128;   // tokens per workgroup
+
+// The kernels of a launch, by the rows x tokens of a workgroup. 16 x 64 and
+// 32 x 64: k_matmul_short;
+// 64 x 128 and 128 x 128: k_matmul, or k_matmul_ring for short reductions.
+// A SwiGLU pair takes half a tile's rows from each matrix.
+enum MmForm { MF_16, MF_32, MF_64, MF_128, MF_RING_64, MF_RING_128, MF_FORMS };
+__host__ __device__ constexpr int mf_rows(int f) {
+    return f == MF_16 ? 16 : f == MF_32 ? 32 : f == MF_64 || f == MF_RING_64 ? 64 : 128;
+}
+__host__ __device__ constexpr int mf_tokens(int f) { return f <= MF_32 ? 64 : MM_TT; }
 
 template <int D16> struct MmScale { using T = uint32_t; };
 template <> struct MmScale<1> { using T = uint16_t; };
@@ -124,6 +135,44 @@ __device__ __forceinline__ void mm_emit(const MmArgs &a, const MmOut &out, int r
         float *p = out.y + (size_t)t * out.ldy + row;
         if (EPI == MM_ADD) *p = kr_fadd(*p, v);
         else *p = v;
+    }
+}
+
+// The sums of a wave over 32 x 32 tiles: lane = one row (32 g + lane % 32),
+// tokens 8 (r / 4) + 4 (lane / 32) + r % 4 of the wave's 32
+template <int EPI, int NG>
+__device__ __forceinline__ void mm_finish(const MmArgs &a, int mi, int rows, int rowl, int tokl,
+                                          const float (&acc)[NG][16], int lane) {
+    if constexpr (EPI == MM_SWIGLU) {
+        // h = silu(w1 x) * (w3 x) (k_scalar.c:96-98), then its Q8_0 in blocks
+        // of 32 rows (k_scalar.c:39-57): a block's 32 values are the 32 lanes
+        // of a half-wave (the first NG / 2 groups: w1 rows; the rest: the same w3 rows)
+#pragma unroll
+        for (int g = 0; g < NG / 2; g++) {
+            const int row = rowl + 32 * g + (lane & 31);
+            const bool bin = rowl + 32 * g < rows;   // rows % 32 == 0: whole blocks in or out
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int t = tokl + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+                const float h1 = acc[g][r], h3 = acc[g + NG / 2][r];
+                const float v = kr_fmul(kr_fdiv(h1, kr_fadd(1.0f, kr_expf(-h1))), h3);
+                int8_t q;
+                float d;
+                kr_quant_block32(v, &q, &d);
+                if (bin && t < a.T) {
+                    a.hq[(size_t)t * rows + row] = q;
+                    if ((lane & 31) == 0) a.hdT[(size_t)(row >> 5) * a.ldx + t] = d;
+                }
+            }
+        }
+    } else {
+        const MmOut out = mm_out(a, mi, rows);
+#pragma unroll
+        for (int g = 0; g < NG; g++)
+#pragma unroll
+            for (int r = 0; r < 16; r++)
+                mm_emit<EPI>(a, out, rowl + 32 * g + (lane & 31), tokl + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3),
+                             acc[g][r]);
     }
 }
 
@@ -349,11 +398,11 @@ __device__ __forceinline__ float mm_sums(float (&acc)[NG][16], MmStage<NG, D16> 
 // and 4 tokens, so the sums' chains are a quarter as long as with the
 // 32 x 32 form and a short batch still has rows / 16 workgroups. A stage is 8
 // blocks (256 bytes of every row: whole cache lines), staged through two LDS
-// buffers and loaded 4 stages ahead (RG 2, whose grids give a CU several workgroups: 2)
-// in a register ring, which keeps 16 KB of weights in flight per workgroup
-// (one workgroup a CU must cover the memory latency by itself).
+// buffers and loaded 2 stages ahead in a register ring. (4 stages ahead took all
+// 256 VGPRs, spilled, and were 3 to 6% slower from 2048 to 4096 columns, 1% at
+// 14336.)
 constexpr int MS_SB = 8, MS_TT = 64;             // blocks a stage, tokens a workgroup
-constexpr int ms_depth(int rg) { return rg == 1 ? 4 : 2; }   // stages ahead (even)
+constexpr int MS_D = 2;                          // stages ahead (even)
 constexpr int MS_RC = 2 * MS_SB + 1;             // 16-byte chunks a staged row (one of padding)
 
 template <int RG, int D16>
@@ -518,7 +567,6 @@ __device__ __forceinline__ float ms_sums(float (&acc)[RG][4], MsStage<RG, D16> *
     for (int g = 0; g < RG; g++)
 #pragma unroll
         for (int r = 0; r < 4; r++) acc[g][r] = 0.0f;
-    constexpr int MS_D = ms_depth(RG);
     MsPre<QT, RG> R[MS_D];   // stage k sits in R[k % MS_D] until it is put
 #pragma unroll
     for (int k = 0; k < MS_D; k++) ms_load<QT, D16, RG>(R[k], t, k * MS_SB, tid);
@@ -597,38 +645,167 @@ __global__ void __launch_bounds__(256, 2) k_matmul(const MmArgs a) {
         mm_sums<QT, 0, NG, PAIR, false>(acc, L, t, tid);
     }
 
-    // epilogue: lane = one row (32 g + lane % 32), tokens 8 (r / 4) + 4 (lane / 32) + r % 4
-    if constexpr (PAIR) {
-        // h = silu(w1 x) * (w3 x) (k_scalar.c:96-98), then its Q8_0 in blocks
-        // of 32 rows (k_scalar.c:39-57): a block's 32 values are the 32 lanes
-        // of a half-wave (the first NG / 2 groups: w1 rows; the rest: the same w3 rows)
+    mm_finish<EPI, NG>(a, mi, W.rows, rowl, tokl, acc, lane);
+}
+
+// ---- 128- and 64-row tiles of a short reduction: one block a stage ----
+//
+// A reduction of few blocks never fills k_matmul's pipeline: its stages of 4
+// blocks cost the first one's whole latency, and their 80 KB leave a CU two
+// workgroups to overlap it (and the stores of the sums) with. Here a stage is one
+// block in an LDS ring of 3: 12 KB and 146 VGPRs, 3 waves a SIMD. On the other
+// side of the line its 32 bytes a row and load cost 4 times the cache lines.
+// 128-row tiles, 14336 rows and 700 tokens: 288 columns 21.8 us against
+// k_matmul's 26.5, 896 columns 47.0 against 48.0, 2048 columns 101 against 97.
+struct MrX {
+    v4i xa;              // the wave's 32 tokens
+};
+
+// Per thread and block, for the workgroup's tile: 16 quant bytes of weight
+// row tid / 2 (half tid % 2, Q4 unpacked to n - 8), that row's raw scale, and
+// the scale of the workgroup's token tid % 128.
+struct MrW {
+    v4i w;
+    uint32_t d;
+    float xs;
+};
+
+constexpr int MR_ST = 3;   // LDS ring stages of the weight tile
+
+template <int NG>
+struct MrLds {
+    v4i w[MR_ST][32 * NG][2];     // [stage][row][half]
+    uint32_t d[MR_ST][32 * NG];   // [stage][row] raw scale bits
+    float xs[MR_ST][MM_TT];       // [stage][token] the tokens' scales
+};
+
+__device__ __forceinline__ void mr_load_x(MrX &f, const MmArgs &a, int b, int tokl, int lane) {
+    const int t = tokl + (lane & 31);   // readable: the caller pads the activations to ldx rows
+    f.xa = *(const v4i *)(a.xq + (size_t)t * a.K + (size_t)b * 32 + 16 * (lane >> 5));
+}
+
+// thread tid loads half tid % 2 of tile row (tid / 2) mod 32 NG (NG 2: the
+// second half of the threads repeats a row's load, which keeps every load
+// unconditional, and does not store it); xcol: the scales of this thread's token,
+// clamped to the last. PAIR: the tile's first half are rows rowl.. of W,
+// the second the same rows of W2 (SwiGLU's w1 and w3).
+template <int QT, int D16, int NG, bool PAIR>
+__device__ __forceinline__ void mr_load(MrW &R, const MMat &W, const MMat &W2, const float *xcol, int xsb, int nb,
+                                        int b, int rowl, int tid) {
+    const int tr = (tid >> 1) & (32 * NG - 1);
+    const int r = min(rowl + (PAIR ? tr & (16 * NG - 1) : tr), W.rows - 1);   // rows past the end re-read the last (not stored)
+    const size_t blk = (size_t)r * nb + b;
+    const bool second = PAIR && tr >= 16 * NG;
+    const uint8_t *wq = (second ? W2.q : W.q) + blk * (QT == ML_Q8_0 ? 32 : 16);
+    const void *wd = second ? W2.d : W.d;
+    R.w = QT == ML_Q8_0 ? *(const v4i *)(wq + 16 * (tid & 1)) : q4_frag(*(const v4i *)wq, tid & 1);
+    R.d = D16 ? (uint32_t)((const uint16_t *)wd)[blk] : ((const uint32_t *)wd)[blk];
+    R.xs = xcol[(size_t)b * xsb];
+}
+
+template <int NG>
+__device__ __forceinline__ void mr_put(MrLds<NG> &L, int st, const MrW &R, int tid) {
+    if (tid < MM_TT) L.xs[st][tid] = R.xs;
+    if ((tid >> 1) >= 32 * NG) return;
+    L.w[st][tid >> 1][tid & 1] = R.w;
+    if ((tid & 1) == 0) L.d[st][tid >> 1] = R.d;
+}
+
+// Row group g + 1's MFMA is issued after the whole rescale of group g: an
+// empty asm takes every rescaled value of group g as input and the MFMA's
+// weight operand as in-out, so only one 16-register result set is live (left
+// to itself the compiler holds NG of them: 183 VGPRs, 2 waves a SIMD).
+template <int D16, int NG>
+__device__ __forceinline__ void mr_step(float (&acc)[NG][16], const MrX &f, const MrLds<NG> &L, int st, int lane,
+                                        int tokw) {
+    const int ln = lane & 31, hf = lane >> 5;
+    v4i wb[NG];
+    uint32_t wdr[NG];
 #pragma unroll
-        for (int g = 0; g < NG / 2; g++) {
-            const int row = rowl + 32 * g + (lane & 31);
-            const bool bin = rowl + 32 * g < W.rows;   // rows % 32 == 0: whole blocks in or out
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int t = tokl + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                const float h1 = acc[g][r], h3 = acc[g + NG / 2][r];
-                const float v = kr_fmul(kr_fdiv(h1, kr_fadd(1.0f, kr_expf(-h1))), h3);
-                int8_t q;
-                float d;
-                kr_quant_block32(v, &q, &d);
-                if (bin && t < a.T) {
-                    a.hq[(size_t)t * W.rows + row] = q;
-                    if ((lane & 31) == 0) a.hdT[(size_t)(row >> 5) * a.ldx + t] = d;
-                }
-            }
-        }
-        return;
+    for (int g = 0; g < NG; g++) {
+        wb[g] = L.w[st][32 * g + ln][hf];
+        wdr[g] = L.d[st][32 * g + ln];
     }
-    const MmOut out = mm_out(a, mi, W.rows);
+    float xd[16];
+    const float4 *xv = (const float4 *)&L.xs[st][tokw + 4 * hf];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const float4 v = xv[2 * q];   // tokens 8 q + 4 hf .. + 3
+        xd[4 * q] = v.x;
+        xd[4 * q + 1] = v.y;
+        xd[4 * q + 2] = v.z;
+        xd[4 * q + 3] = v.w;
+    }
+    v16i s = __builtin_amdgcn_mfma_i32_32x32x32_i8(f.xa, wb[0], v16i{}, 0, 0, 0);
+#pragma unroll
+    for (int g = 0; g < NG; g++) {
+        const float wd = D16 ? kr_h2f((uint16_t)wdr[g]) : __uint_as_float(wdr[g]);
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+            acc[g][r] = kr_fadd(acc[g][r], kr_fmul(kr_fmul((float)s[r], wd), xd[r]));
+        if (g + 1 < NG) {
+            v4i w = wb[g + 1];
+#pragma unroll
+            for (int r = 0; r < 16; r++) asm volatile("" : "+v"(w) : "v"(acc[g][r]));
+            s = __builtin_amdgcn_mfma_i32_32x32x32_i8(f.xa, w, v16i{}, 0, 0, 0);
+        }
+    }
+}
+
+// The workgroup's threads load each block's weight tile and its scales once
+// (16 bytes and one scale per thread) into the LDS ring: block b + 1 is stored
+// during step b into the stage step b - 2 read, and the barrier closing each
+// step orders those stores before step b + 1 reads them.
+template <int EPI, int QT, int D16, int NG>
+__global__ void __launch_bounds__(256, 3) k_matmul_ring(const MmArgs a) {
+    __shared__ MrLds<NG> L;
+    int mi = 0;
+    while (mi + 1 < a.nmat && (int)blockIdx.x >= a.tile0[mi + 1]) mi++;
+    const MMat W = mi == 0 ? a.w[0] : (mi == 1 ? a.w[1] : a.w[2]);
+    const int ntt = (a.T + MM_TT - 1) / MM_TT;
+    const int local = (int)blockIdx.x - a.tile0[mi];
+    const int rt = local / ntt, tt = local - rt * ntt;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    constexpr bool PAIR = EPI == MM_SWIGLU;   // 16 NG rows of w1 and the same of w3
+    const int rowl = rt * (PAIR ? 16 : 32) * NG, tokl = tt * MM_TT + 32 * wave;
+    const int nb = a.K / KR_QK;
+    const float *xcol = a.xdT + (size_t)min(tt * MM_TT + (tid & (MM_TT - 1)), a.T - 1) * a.xst;
+    float acc[NG][16];
 #pragma unroll
     for (int g = 0; g < NG; g++)
 #pragma unroll
-        for (int r = 0; r < 16; r++)
-            mm_emit<EPI>(a, out, rowl + 32 * g + (lane & 31), tokl + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3),
-                         acc[g][r]);
+        for (int r = 0; r < 16; r++) acc[g][r] = 0.0f;
+    // Loads are unconditional (block indices past the end re-read the last
+    // block, unused): a load issued on only one path makes the wait-count
+    // pass drain every in-flight load at the loop head, which would cancel
+    // the prefetch. Only the odd tail's step is conditional; every thread
+    // reaches every barrier.
+    const int bl = nb - 1;
+    MrW R;
+    MrX x0, x1;
+    auto load = [&](int b) { mr_load<QT, D16, NG, PAIR>(R, W, a.w[1], xcol, a.xsb, nb, min(b, bl), rowl, tid); };
+    load(0);
+    mr_put(L, 0, R, tid);
+    load(1);
+    mr_load_x(x0, a, 0, tokl, lane);
+    mr_load_x(x1, a, min(1, bl), tokl, lane);
+    __syncthreads();
+    int st = 0;   // stage of block b
+    for (int b = 0; b < nb; b += 2) {
+        const int s1 = st == MR_ST - 1 ? 0 : st + 1, s2 = s1 == MR_ST - 1 ? 0 : s1 + 1;
+        mr_put(L, s1, R, tid);
+        load(b + 2);
+        mr_step<D16, NG>(acc, x0, L, st, lane, 32 * wave);
+        mr_load_x(x0, a, min(b + 2, bl), tokl, lane);
+        __syncthreads();
+        mr_put(L, s2, R, tid);
+        load(b + 3);
+        if (b + 1 < nb) mr_step<D16, NG>(acc, x1, L, s1, lane, 32 * wave);
+        mr_load_x(x1, a, min(b + 3, bl), tokl, lane);
+        __syncthreads();
+        st = s2;
+    }
+    mm_finish<EPI, NG>(a, mi, W.rows, rowl, tokl, acc, lane);
 }
 
 template <int EPI>
@@ -638,35 +815,25 @@ void launch_mm(const MmArgs &a, const MMat &W) {
         kr_fail(ML_E_SHAPE, "matmul shape", hipSuccess);
         return;
     }
-    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, kr_stream(), a); };
-    if (EPI == MM_SWIGLU && a.ng == 1) {
-        kr_fail(ML_E_SHAPE, "matmul: SwiGLU pairs take 128- or 64-row tiles", hipSuccess);
-        return;
-    }
-    if (a.ng == 4) {
-        if (W.type == ML_Q8_0) {
-            if (W.d16) go(k_matmul<EPI, ML_Q8_0, 1, 4>); else go(k_matmul<EPI, ML_Q8_0, 0, 4>);
-        } else {
-            if (W.d16) go(k_matmul<EPI, ML_Q4_0, 1, 4>); else go(k_matmul<EPI, ML_Q4_0, 0, 4>);
+    auto run = [&](auto qt, auto d16) {
+        constexpr int QT = decltype(qt)::value, D16 = decltype(d16)::value;
+        auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, kr_stream(), a); };
+        if constexpr (EPI != MM_SWIGLU) {
+            if (a.form == MF_16) return go(k_matmul_short<EPI, QT, D16, 1>);
+            if (a.form == MF_32) return go(k_matmul_short<EPI, QT, D16, 2>);
         }
-    } else if (a.ng == 2) {
-        if (W.type == ML_Q8_0) {
-            if (W.d16) go(k_matmul<EPI, ML_Q8_0, 1, 2>); else go(k_matmul<EPI, ML_Q8_0, 0, 2>);
-        } else {
-            if (W.d16) go(k_matmul<EPI, ML_Q4_0, 1, 2>); else go(k_matmul<EPI, ML_Q4_0, 0, 2>);
-        }
-    } else if constexpr (EPI != MM_SWIGLU) {
-        if (a.rg == 2) {
-            if (W.type == ML_Q8_0) {
-                if (W.d16) go(k_matmul_short<EPI, ML_Q8_0, 1, 2>); else go(k_matmul_short<EPI, ML_Q8_0, 0, 2>);
-            } else {
-                if (W.d16) go(k_matmul_short<EPI, ML_Q4_0, 1, 2>); else go(k_matmul_short<EPI, ML_Q4_0, 0, 2>);
-            }
-        } else if (W.type == ML_Q8_0) {
-            if (W.d16) go(k_matmul_short<EPI, ML_Q8_0, 1, 1>); else go(k_matmul_short<EPI, ML_Q8_0, 0, 1>);
-        } else {
-            if (W.d16) go(k_matmul_short<EPI, ML_Q4_0, 1, 1>); else go(k_matmul_short<EPI, ML_Q4_0, 0, 1>);
-        }
+        if (a.form == MF_64) return go(k_matmul<EPI, QT, D16, 2>);
+        if (a.form == MF_128) return go(k_matmul<EPI, QT, D16, 4>);
+        if (a.form == MF_RING_64) return go(k_matmul_ring<EPI, QT, D16, 2>);
+        go(k_matmul_ring<EPI, QT, D16, 4>);
+    };
+    using std::integral_constant;
+    if (W.type == ML_Q8_0) {
+        if (W.d16) run(integral_constant<int, ML_Q8_0>{}, integral_constant<int, 1>{});
+        else run(integral_constant<int, ML_Q8_0>{}, integral_constant<int, 0>{});
+    } else {
+        if (W.d16) run(integral_constant<int, ML_Q4_0>{}, integral_constant<int, 1>{});
+        else run(integral_constant<int, ML_Q4_0>{}, integral_constant<int, 0>{});
     }
     kr_check_launch("matmul");
 }
@@ -676,34 +843,59 @@ MMat to_mmat(const krh_mat *m) {
     return k;
 }
 
-// The tiles of a launch over nmat matrices of these rows: NG 4 (128 rows x
-// 128 tokens a workgroup), NG 2 (64 x 128), RG 2 (32 x 64) or RG 1 (16 x 64).
-// Larger tiles load less per sum, smaller ones make more workgroups; the lines,
-// in workgroups per CU, from krh_matmul on 256 CUs (us; Q8, K 4096 and 14336):
-// - NG 4 once NG 2's grid is more than one round of its 2 workgroups a CU:
-//   4096 x 14336, 1100 tokens (2.25 rounds' worth of NG 2): 342 against 381;
-//   14336 x 4096, 511 tokens: 112 against 128; at 2 a CU or less the halves
-//   balance better: 2048 x 2048, 2047 tokens 55 against 43, 14336 x 4096, 256
-//   tokens 92 against 70.
-// - RG 2 below 3 of its workgroups a CU: 4096 x 14336, 300 tokens (2.5 a CU)
-//   167 against NG 2's 187, 14336 x 4096, 64 tokens 38 against 60; above,
-//   14336 x 4096, 128 tokens (3.5) 72 against 60.
-// - RG 1 below 1.25 of RG 2's a CU: 4096 x 14336, 37 tokens 53 against 75 and
-//   128 tokens (1 a CU) 75 against 82; above, 2048 x 2048, 400 tokens 29
-//   against 25.
-void mm_plan(MmArgs &a, int nmat, const int *rows) {
-    const int ntt128 = (a.T + MM_TT - 1) / MM_TT, ntt64 = (a.T + MS_TT - 1) / MS_TT;
-    const long cus = krh_device_cus() > 0 ? krh_device_cus() : 256;
-    long t64 = 0, t32 = 0;   // NG 2's and RG 2's workgroups
-    for (int i = 0; i < nmat; i++) {
-        t64 += (long)(rows[i] + 63) / 64 * ntt128;
-        t32 += (long)(rows[i] + 31) / 32 * ntt64;
+// The form of a launch: the one with the least estimated time on this device,
+//   rounds * (fixed + K / 32 * alone) + (n - rounds) * K / 32 * shared + n * tile   (us),
+// n the workgroups of the fullest CU, which holds `resident` of them at a time:
+// the first of a round takes `alone` a block of 32 columns, each of the others
+// adds `shared`, and each stores its tile. Larger tiles load less per sum, smaller
+// ones make more workgroups. The constants are fitted to the choice, over krh_matmul
+// and krh_matmul_swiglu with every form timed at 11 heights from 288 to 14336
+// rows, 7 reductions from 288 to 14336 columns and 19 batches from 2 to 2047
+// tokens (Q8 and Q4, f16 and f32 scales): over those 3914 sizes it costs 0.2%
+// more than the best form of each. Some of its lines (us, the call alone):
+// 16-row tiles 13.3 and 32-row ones 10.6 (896 x 896, 700 tokens), 7.0 and 8.6 (64
+// tokens); 64-row tiles 63 and 128-row ones 86 (14336 x 4096, 256 tokens), 122
+// and 106 (511 tokens); SwiGLU 14336 x 288, 300 tokens: rings 35, k_matmul 47;
+// 4864 x 2048, 511 tokens: 76 and 69.
+struct MmCost {
+    int resident;
+    float fixed, alone, shared, tile;
+};
+constexpr MmCost MF_COST[MF_FORMS] = {
+    { 3, 3.3f, 0.076f, 0.089f, 0.38f }, { 2, 4.0f, 0.18f, 0.06f, 0.026f }, { 2, 3.3f, 0.49f, 0.025f, 1.1f },
+    { 2, 6.2f, 0.7f, 0.13f, 1.5f }, { 4, 6.3f, 0.53f, 0.2f, 0.15f }, { 3, 2.6f, 1.2f, 0.32f, 0.79f },
+};
+constexpr MmCost MF_PAIR_COST[MF_FORMS] = {
+    {}, {}, { 2, 19.0f, 0.3f, 0.097f, 0.13f }, { 2, 29.0f, 0.47f, 0.21f, 2.0f },
+    { 4, 14.0f, 0.62f, 0.23f, 0.56f }, { 3, 30.0f, 0.51f, 0.48f, 1.6f },
+};
+
+int mm_form(int nmat, const int *rows, int K, int T, bool pair) {
+    const int cus = krh_device_cus() > 0 ? krh_device_cus() : 256;
+    const float nb = (float)(K / KR_QK);
+    int best = MF_64;
+    float least = INFINITY;
+    for (int f = pair ? MF_64 : MF_16; f < MF_FORMS; f++) {
+        const int per = mf_rows(f) / (pair ? 2 : 1);
+        long wgs = 0;
+        for (int i = 0; i < nmat; i++) wgs += (long)((rows[i] + per - 1) / per) * ((T + mf_tokens(f) - 1) / mf_tokens(f));
+        const MmCost &c = (pair ? MF_PAIR_COST : MF_COST)[f];
+        const long nl = (wgs + cus - 1) / cus;
+        const float n = (float)nl, rounds = (float)((nl + c.resident - 1) / c.resident);
+        const float t = rounds * (c.fixed + nb * c.alone) + (n - rounds) * nb * c.shared + n * c.tile;
+        if (t < least) {
+            least = t;
+            best = f;
+        }
     }
-    a.ng = t64 > 2 * cus ? 4 : t32 >= 3 * cus ? 2 : 1;
-    a.rg = a.ng != 1 ? 0 : 4 * t32 >= 5 * cus ? 2 : 1;
-    const int per = a.rg ? 16 * a.rg : 32 * a.ng;
+    return best;
+}
+
+void mm_plan(MmArgs &a, int nmat, const int *rows, bool pair = false) {
+    a.form = mm_form(nmat, rows, a.K, a.T, pair);
+    const int per = mf_rows(a.form) / (pair ? 2 : 1), ntt = (a.T + mf_tokens(a.form) - 1) / mf_tokens(a.form);
     a.tile0[0] = 0;
-    for (int i = 0; i < nmat; i++) a.tile0[i + 1] = a.tile0[i] + (rows[i] + per - 1) / per * (a.rg ? ntt64 : ntt128);
+    for (int i = 0; i < nmat; i++) a.tile0[i + 1] = a.tile0[i] + (rows[i] + per - 1) / per * ntt;
 }
 
 // ---- per-token work of a batched step ----
@@ -758,6 +950,10 @@ __global__ void k_embed_batch(float *x, const MMat e, const int *tok, float scal
 
 // ---- C ABI ----
 
+extern "C" int krh_matmul_form(int rows, int cols, int ntok, int swiglu) {
+    return rows > 0 && cols > 0 && ntok > 0 ? mm_form(1, &rows, cols, ntok, swiglu != 0) : -1;
+}
+
 extern "C" void krh_matmul_swiglu(int8_t *hq, float *hdT, const krh_mat *w1, const krh_mat *w3, const int8_t *xq,
                                   const float *xdT, int ldx, int T) {
     if (!hq || !hdT || w1->rows != w3->rows || w1->cols != w3->cols || w1->type != w3->type || w1->d16 != w3->d16 ||
@@ -770,12 +966,6 @@ extern "C" void krh_matmul_swiglu(int8_t *hq, float *hdT, const krh_mat *w1, con
     a.w[0] = to_mmat(w1);
     a.w[1] = to_mmat(w3);
     a.nmat = 1;
-    a.tile0[0] = 0;
-    const int ntt = (T + MM_TT - 1) / MM_TT;
-    // as mm_plan: 128-row tiles once the 64-row ones are more than a round of two a CU
-    const long t32 = (long)(w1->rows / 32) * ntt, cus = krh_device_cus() > 0 ? krh_device_cus() : 256;
-    a.ng = t32 > 2 * cus ? 4 : 2;
-    a.tile0[1] = (w1->rows + 16 * a.ng - 1) / (16 * a.ng) * ntt;
     a.xq = xq;
     a.xdT = xdT;
     a.ldx = ldx;
@@ -785,6 +975,7 @@ extern "C" void krh_matmul_swiglu(int8_t *hq, float *hdT, const krh_mat *w1, con
     a.K = w1->cols;
     a.hq = hq;
     a.hdT = hdT;
+    mm_plan(a, 1, &w1->rows, true);
     launch_mm<MM_SWIGLU>(a, a.w[0]);
 }
 

@@ -179,6 +179,7 @@ for name, res, args in [
     ("krh_quantize_q8_t", None, [_P, _P, C.c_int, _P, C.c_int, C.c_int]),
     ("krh_matmul", None, [_P, C.c_int, C.POINTER(KrhMat), _P, _P, C.c_int, C.c_int, C.c_int]),
     ("krh_matmul_rows", None, [_P, C.c_int, C.POINTER(KrhMat), _P, _P, C.c_int, C.c_int, C.c_int]),
+    ("krh_matmul_form", C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int]),
     ("krh_matmul_swiglu", None, [_P, _P, C.POINTER(KrhMat), C.POINTER(KrhMat), _P, _P, C.c_int, C.c_int]),
     ("krh_matmul_qkv", None, [_P, _P, _P, C.POINTER(KrhMat), C.POINTER(KrhMat), C.POINTER(KrhMat), _P, _P, _P,
                               _P, _P, C.c_int, C.c_int, _P, _P, C.c_int, C.c_int]),

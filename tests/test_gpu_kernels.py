@@ -10,6 +10,7 @@ import pytest
 import krafla as K
 import oracle_lib as O
 from oracle_lib import oracle
+from matmul_sizes import MATMUL_TILES, SWIGLU_TILES
 
 pytestmark = pytest.mark.gpu
 RNG = np.random.default_rng(42)
@@ -571,11 +572,11 @@ def test_matmul(dev, typ, d16, rows, cols, T):
             assert np.array_equal(bits(got_rows[t]), bits(want)), (t, acc, "rows")
 
 
-# one size for each tile form (16 x 64, 32 x 64, 64 x 128 and 128 x 128 rows x
-# tokens) with ragged rows, tokens and stages (4 or 8 blocks of 32 columns)
+# ragged rows, tokens and stages (1, 4 or 8 blocks of 32 columns) of every tile
+# form (16 x 64, 32 x 64, 64 x 128 and 128 x 128 rows x tokens, the last two for
+# long and short reductions: test_matmul_forms.py)
 @pytest.mark.parametrize("typ,d16", [(K.ML_Q8_0, 1), (K.ML_Q4_0, 1), (K.ML_Q8_0, 0)])
-@pytest.mark.parametrize("rows,cols,T", [(17, 32, 2), (100, 992, 65), (16, 1056, 64), (10250, 288, 33),
-                                         (10240, 256, 17), (16416, 96, 65), (16416, 128, 128), (16450, 160, 130)])
+@pytest.mark.parametrize("rows,cols,T", MATMUL_TILES)
 @pytest.mark.parametrize("scales", ["plain", "signed", "infinite"])
 def test_matmul_tiles(dev, typ, d16, rows, cols, T, scales):
     """every tile form's sums equal the matvec's, bit for bit; signed: negative
@@ -760,7 +761,7 @@ def test_silu_quant(dev):
 
 @pytest.mark.parametrize("typ,d16", [(K.ML_Q8_0, 1), (K.ML_Q4_0, 1), (K.ML_Q8_0, 0)])
 @pytest.mark.parametrize("rows,cols,T", [(14336, 4096, 300), (4864, 896, 511), (768, 288, 37), (96, 64, 5),
-                                         (8192, 2048, 129)])
+                                         (8192, 2048, 129)] + SWIGLU_TILES)
 def test_matmul_swiglu_matches_separate(dev, typ, d16, rows, cols, T):
     """krh_matmul_swiglu (w1 and w3 tiles in one launch, SiLU and the Q8_0 of
     h in its epilogue) gives the bits of two krh_matmul calls and
