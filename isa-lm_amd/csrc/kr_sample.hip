@@ -37,9 +37,10 @@ struct krh_sampler {
 namespace {
 
 constexpr int SM_NT = 1024;                                       // threads of the one-workgroup kernels
-// Terms per ordered-sum group (in LDS: 152 of the CU's 160 KB with the sum's
-// scratch; one workgroup runs these kernels). A group costs about 6 us whatever
-// its length, so the fewer the better: with 12,288 terms the 128k vocabulary's
+// Terms per ordered-sum group (in LDS: 146 of the CU's 160 KB with the sum's
+// scratch; one workgroup runs these kernels). Most of a group's time does not
+// depend on its length, so the fewer the better (k_smp_main over 128,256 ids
+// 83 us in 11 groups of 12,288, 36 in 4): with 12,288 terms that vocabulary's
 // softmax took 11 groups and a nucleus of 26k candidates 3 (a top-p draw over
 // 128,256 ids, with the scaling pass gone and the sort's empty workgroups
 // returning at once: 181 -> 125 us; 116 with the draw's second sum gone).
@@ -162,18 +163,26 @@ __device__ float sm_coin(unsigned long long *st) {
 __device__ __forceinline__ float sm_prob(float x, float inv) { return kr_fmul(x, inv); }
 
 // ng terms from term(g0) into LDS in the ordered sum's layout; each thread's
-// reads SM_FB at a time, all issued before the first store
-constexpr int SM_FB = 16;
-template <class Term>
-__device__ __forceinline__ void sm_fill(float *t, Term term, int g0, int ng, int sh) {
-    for (int i0 = sm_tid(); i0 < ng; i0 += SM_FB * SM_NT) {
-        float v[SM_FB];
+// reads FB at a time, all issued before the first store
+template <int FB, class Term>
+__device__ __forceinline__ void sm_fill_n(float *t, Term term, int g0, int ng, int sh) {
+    for (int i0 = sm_tid(); i0 < ng; i0 += FB * SM_NT) {
+        float v[FB];
 #pragma unroll
-        for (int k = 0; k < SM_FB; k++) v[k] = term(g0 + min(i0 + k * SM_NT, ng - 1));
+        for (int k = 0; k < FB; k++) v[k] = term(g0 + min(i0 + k * SM_NT, ng - 1));
 #pragma unroll
-        for (int k = 0; k < SM_FB; k++)
+        for (int k = 0; k < FB; k++)
             if (i0 + k * SM_NT < ng) t[sc_at(i0 + k * SM_NT, sh)] = v[k];
     }
+}
+
+// 16 reads a thread, most of them repeats where the group is shorter than 16
+// ids a thread: from 4 ids a thread down, 4 (a draw over 600 ids 16.3 -> 14.7
+// us in k_smp_main, 1500 ids 16.9 -> 14.8; 8000 ids take the 16: 19.2 and 19.0)
+template <class Term>
+__device__ __forceinline__ void sm_fill(float *t, Term term, int g0, int ng, int sh) {
+    if (ng <= 4 * SM_NT) sm_fill_n<4>(t, term, g0, ng, sh);
+    else sm_fill_n<16>(t, term, g0, ng, sh);
 }
 
 // The group of terms an ordered-prefix search summed last: terms g0 ..

@@ -89,9 +89,10 @@ def test_sample_matches_oracle(name, n):
 
 
 @pytest.mark.parametrize("name", ["mult", "topp", "topk_big"])
-@pytest.mark.parametrize("n", [32768, 32769, 66000])
+@pytest.mark.parametrize("n", [4096, 4097, 32768, 32769, 66000])
 def test_sample_group_edges(name, n):
-    """vocabularies of exactly one ordered-sum group, one id more, and a ragged third group"""
+    """vocabularies of exactly one ordered-sum group, one id more, and a ragged
+    third group; 4 ids a thread and one id more (the group's fill)"""
     opts = O.sampler_opts(**OPTS[name])
     for k, kind in enumerate(["normal", "flat", "ties"]):
         draws_match(n, opts, kind, 3, 900 + k)
