@@ -253,12 +253,19 @@ void krh_attention_batch(float *ao, float *att, const float *q, const float *kc,
  * then not written. */
 int krh_attention_short(int head_dim, int kv_type);
 /* The batched attention's choice of kernels (no counterpart in the
- * reference): heads of 48, 64, 80, 96, 128 or 256 dims take the
- * register-blocked score and mix kernels when their grids hold at least
- * min_wg / 2 workgroups, and the per-token-block kernels below that (default
- * 512). Tests lower it to run the register-blocked kernels on small shapes;
- * the results are the same bits either way. Process-wide. */
+ * reference): by default (512) each stage takes the kernels with the least
+ * estimated time. Any other value decides between the register-blocked score
+ * and mix kernels (heads of 48, 64, 80, 96, 128 or 256 dims) and the token-block
+ * ones by the grids alone:
+ * from min_wg / 2 workgroups the former run. Tests set it to run either
+ * on small shapes; the results are the same bits whatever runs. Process-wide. */
 void krh_set_attn_rb_min(int min_wg);
+/* That choice for ntok > 1 tokens, the last at last_pos: scores + 4 softmax +
+ * 16 mix, scores and mix 0 (a token a workgroup), 1 (token blocks) or 2
+ * (register-blocked rows), softmax 0, 1 (a row 1024 or 256 threads) or 2 (a
+ * wave); -1 for no such batch. */
+int krh_attention_plan(int kv_type, int n_heads, int n_kv_heads, int head_dim, int max_seq, int window, int ntok,
+                       int last_pos);
 /* h = silu(g) * u per token (k_scalar.c:96-98), quantized to Q8_0 with
  * transposed scales dT[b * ldd + t] */
 void krh_silu_quant(int8_t *q, float *dT, int ldd, const float *g, const float *u, int n, int ntok);

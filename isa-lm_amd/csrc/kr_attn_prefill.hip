@@ -3,6 +3,7 @@
 // comment; every float operation is the reference's, in its order). A code
 // object of its own: with these kernels in the decode kernels' object, a decode
 // launch of the 8B shape's attention took 0.6 us longer.
+#include <cmath>
 #include "kr_attn.h"
 
 namespace {
@@ -101,15 +102,6 @@ __global__ void __launch_bounds__(AT_THREADS) k_attn_scores_blk(float *att, cons
 // the queries and K are staged HS dims at a time, the sums carried along.
 constexpr int RB_R = 64, RB_T = 64;   // rows of a register-blocked workgroup; positions of its tiles
 constexpr int RB_PC = 8;             // K tiles per scores workgroup, at most
-// the register-blocked kernels run when their grids hold at least this many
-// half workgroups (a whole one per CU: rb_fills); smaller grids take the
-// per-token-block kernels. Measured on both sides of the line (us, scores to
-// mix, register-blocked from 128, 256 and 512 workgroups, and never): 8
-// heads of 256 over a 1024 window, 1021 tokens 306, 237, 329, 538; 24 heads of
-// 80, window 300, 1000 tokens 163, 155, 175, 178; 8 heads of 96, window 512,
-// 300 tokens 78, 77, 90, 90; 32 heads of 64, 256 tokens 60, 45, 45, 47.
-static int g_rb_min_wg = 512;
-static bool rb_fills(long wgs) { return 2 * wgs >= g_rb_min_wg; }
 static bool rb_dims(int hd) { return hd == 48 || hd == 64 || hd == 80 || hd == 96 || hd == 128 || hd == 256; }
 constexpr int RB_NT128 = 512;        // threads of the 128-dim heads' workgroups (4 outputs' rows a lane, LDS for 2
                                      // workgroups a CU: 4 waves a SIMD; 256 threads gave 2 and measured the same)
@@ -904,18 +896,157 @@ struct AttnShape {
     int mix_row_blocks() const { return n_kv * row_blocks() * (hd / rb_cw(hd)); }
 };
 
+// The choice: for each stage the kernels with the least estimated time. The
+// constants (us, on the 256 CUs of an MI355X) are fitted to the choice: every
+// form of the three stages was timed for 21 head counts and sizes (1 to 32 heads
+// over 1 to 16 KV heads of 32 to 256 dims), three cache types, prompts of 2 to 2000
+// tokens at positions 0, 500 and 2000, without a window and with ones of 96 to
+// 1024 positions: 5040 launches. The choice's three stages together cost 0.6%
+// more than the best form of each, and 24 of the 5040 take over 4% longer than with
+// the token blocks and register-blocked rows chosen by the grid's size alone
+// and windows one token a workgroup; on average 25% less. Windowed batches of few
+// tokens lose most in large blocks: 4 heads of 64, 101 tokens over a window of
+// 70: 12.7 us one token a workgroup, 43 in blocks.
+struct ApScores {      // one token a workgroup; token blocks
+    float lat, lat_hd, tile_math, tile_stage, wide, tile, grid, blk_lat, blk_lat_hd, blk_step, blk_tile, blk_tile_step,
+        q8_step;
+};
+constexpr ApScores AP_SC = { 6.0f, 0.014f, 3.4e-05f, 2e-05f, 1.4f, 5e-07f, 3.1e-06f, 5.8f, 0.00044f, 0.089f, 0.01f, 0.00015f, 0.0f };
+constexpr ApScores AP_SC_Q8 = { 4.6f, 0.022f, 1.5e-05f, 0.0f, 1.0f, 0.00079f, 0.0004f, 6.0f, 0.02f, 0.095f, 0.0025f, 0.00021f, 0.014f };
+struct ApRows {        // register-blocked rows of hd dims: workgroups a CU holds, scores, mix
+    int hd, resident;
+    float fixed, tile, shared, mix_tile;
+};
+constexpr ApRows AP_ROW[] = {
+    { 48, 4, 6.3f, 3.2f, 1.3f, 0.011f },
+    { 64, 4, 4.5f, 8.4f, 1.1f, 0.0092f },
+    { 80, 3, 5.9f, 11.0f, 2.4f, 0.036f },
+    { 96, 3, 6.6f, 13.0f, 4.0f, 0.022f },
+    { 128, 2, 4.0f, 10.0f, 3.8f, 0.028f },
+    { 256, 4, 2.0f, 41.0f, 16.0f, 0.03f },
+};
+
+// what a launch does, for the estimates
+struct ApWork {
+    double pairs;          // (token, position) pairs attended
+    float n, navg;         // positions a token attends, at most and on average
+    bool cut;              // a token attends less than its prefix
+    bool full;             // every token a whole window
+    int tb;                // tokens of a block of RB_R rows, at most
+};
+
+ApWork ap_work(const AttnShape &s) {
+    ApWork w;
+    const double T = s.ntok, p0 = s.max_pos + 1 - s.ntok;
+    w.cut = s.cut();
+    w.full = w.cut && p0 >= s.window;
+    if (!w.cut) w.pairs = T * p0 + T * (T + 1) / 2;
+    else if (w.full) w.pairs = T * s.window;
+    else {
+        const double k = s.window - p0;   // tokens below the window's length
+        w.pairs = k * p0 + k * (k + 1) / 2 + (T - k) * s.window;
+    }
+    w.n = (float)s.nmax();
+    w.navg = (float)(w.pairs / T);
+    w.tb = std::min(s.ntok, (RB_R - 1) / s.group() + 1);
+    return w;
+}
+
+const ApRows *ap_rows(int hd) {
+    for (const ApRows &r : AP_ROW)
+        if (r.hd == hd) return &r;
+    return nullptr;
+}
+
+// the scores: one token a workgroup and tile, or blocks of AT_TB tokens a tile
+float est_scores_token(const AttnShape &s, const ApWork &w) {
+    const bool q8 = s.kt == KV_Q8;
+    const ApScores &c = q8 ? AP_SC_Q8 : AP_SC;
+    const float g4 = (float)((s.group() + 3) / 4), hd = (float)s.hd, kvt = (float)s.n_kv * s.ntok;
+    const bool wide = !q8 && attn_tile<KV_F32>(s.group(), s.hd) == AT_TD;
+    const float tp = wide ? AT_TD : AT_T;
+    const float tiles = w.full ? kvt * ((s.window + 63) / 64) : (float)s.n_kv * (float)(w.pairs / 64 + 0.5 * s.ntok);
+    const float x = (float)s.n_kv * hd * (float)(w.pairs / 64);
+    const float thr = (x * (c.tile_math * g4 + c.tile_stage) + c.tile * tiles) * (wide ? c.wide : 1.0f) +
+                      c.grid * kvt * std::ceil(w.n / tp);
+    return std::max(c.lat + c.lat_hd * hd * g4, thr);
+}
+float est_scores_block(const AttnShape &s, const ApWork &w) {
+    const bool q8 = s.kt == KV_Q8;
+    const ApScores &c = q8 ? AP_SC_Q8 : AP_SC;
+    const float hd = (float)s.hd;
+    const int zn = std::min(s.ntok, AT_TB), qb = q8 ? AT_TB : s.qb();
+    const float step = q8 ? (float)(zn * s.group()) * (1.0f + c.q8_step * hd)
+                          : hd * (float)((zn + qb - 1) / qb) * (float)((s.group() + 3) / 4);
+    const float tiles = (float)s.n_kv * ((s.ntok + AT_TB - 1) / AT_TB) * ((w.navg + 15) / s.tp() + 1);
+    return std::max(c.blk_lat + c.blk_lat_hd * hd + c.blk_step * step, tiles * (c.blk_tile + c.blk_tile_step * step));
+}
+// register-blocked scores, pc tiles a workgroup
+float est_scores_rows(const AttnShape &s, const ApWork &w, const ApRows &c, int pc) {
+    const float nt = std::floor((w.n + w.tb - 1 + 63) / 64), tiles = (w.navg + w.tb - 1) / 64 + 1;
+    const float pe = std::min((float)pc, nt), blocks = (float)s.n_kv * s.row_blocks();
+    const float n = std::max(1.0f, blocks * std::min(std::ceil(nt / pc), tiles / pc + 0.5f) / 256);
+    const float rounds = std::max(1.0f, n / c.resident);
+    return rounds * (c.fixed + c.tile * pe) + (n - rounds) * c.shared * pe;
+}
+
+// the mix: a wave a token and DW dims, token blocks, register-blocked rows
+float est_mix_token(const AttnShape &s, const ApWork &w) {
+    const bool q8 = s.kt == KV_Q8;
+    const int dw = s.dw(), k = dw == 64 ? 0 : dw == 32 ? 1 : 2;
+    constexpr float per[2][3] = { { 6.7e-05f, 2e-05f, 1.2e-05f }, { 6.7e-05f, 2.1e-05f, 1.8e-05f } };
+    const float lat = 1.8f + (q8 ? 0.19f : 0.0f) + (k == 0 ? 0.018f : 0.0098f) * w.n;
+    return std::max(lat, per[q8][k] * (float)s.n_kv * ((s.hd + dw - 1) / dw) * (float)w.pairs);
+}
+float est_mix_block(const AttnShape &s, const ApWork &w) {
+    const int dw = s.dw();
+    const float lat = 2.0f + (w.cut ? 17.0f : 0.0f) + (dw == 64 ? 2.1f : 1.7f) * w.n / 64;
+    const float wgs = (float)s.n_kv * ((s.hd + dw - 1) / dw) * ((s.ntok + MK_W * MK_U - 1) / (MK_W * MK_U));
+    return std::max(lat, (dw == 64 ? 0.0039f : 0.0021f) * wgs * ((w.navg + 7) / 64 + 1 + (w.cut ? 2.7f : 0.0f)));
+}
+float est_mix_rows(const AttnShape &s, const ApWork &w, const ApRows &c) {
+    const float lat = 1.6f + 6.6f * ((w.n + w.tb - 1) / 64 + (w.cut ? 0.35f : 0.0f));
+    return std::max(lat, c.mix_tile * (float)s.mix_row_blocks() * ((w.navg + w.tb - 1) / 64 + 1)) * (s.kt == KV_Q8 ? 1.1f : 1.0f);
+}
+
+// krh_set_attn_rb_min: at other values than its default the grids alone decide
+// between register-blocked rows and token blocks
+constexpr int RB_MIN_WG = 512;
+int g_rb_min_wg = RB_MIN_WG;
+bool rb_fills(long wgs) { return 2 * wgs >= g_rb_min_wg; }
+
 AttnPlan attn_plan(const AttnShape &s) {
-    AttnPlan p = { s.scores_block() ? AP_BLOCK : AP_TOKEN, RB_PC, AP_SMX_1024, s.mix_block() ? AP_BLOCK : AP_TOKEN };
-    // the register-blocked scores: a workgroup's K tiles are cut until the
-    // grid fills the device
-    const long blocks = (long)s.n_kv * s.row_blocks();
-    auto chunks = [&] { return (s.row_tiles() + p.pc - 1) / p.pc; };
-    while (p.pc > 1 && !rb_fills(blocks * chunks() / 2)) p.pc /= 2;
-    if (s.scores_rows() && rb_fills(blocks * chunks())) p.scores = AP_ROWS;
-    if (s.mix_rows() && rb_fills(s.mix_row_blocks())) p.mix = AP_ROWS;
-    // rows of 2049 to 4096 scores: a 256-thread workgroup each (measured:
-    // 1B-shape 4000-token prompt 59.9k -> 61.7k tok/s); up to 2048, a wave each
-    if (s.nmax() <= SM_WN / 2) p.softmax = AP_SMX_WAVE;
+    AttnPlan p = { AP_TOKEN, RB_PC, AP_SMX_1024, AP_TOKEN };
+    if (g_rb_min_wg != RB_MIN_WG) {
+        if (s.scores_block()) p.scores = AP_BLOCK;
+        if (s.mix_block()) p.mix = AP_BLOCK;
+        // a scores workgroup's K tiles are cut until the grid fills the device
+        const long blocks = (long)s.n_kv * s.row_blocks();
+        auto chunks = [&] { return (s.row_tiles() + p.pc - 1) / p.pc; };
+        while (p.pc > 1 && !rb_fills(blocks * chunks() / 2)) p.pc /= 2;
+        if (s.scores_rows() && rb_fills(blocks * chunks())) p.scores = AP_ROWS;
+        if (s.mix_rows() && rb_fills(s.mix_row_blocks())) p.mix = AP_ROWS;
+    } else {
+        const ApWork w = ap_work(s);
+        const ApRows *rows = ap_rows(s.hd);
+        float t = est_scores_token(s, w);
+        auto take = [&](float e, int &choice, int form) {
+            if (e >= t) return false;
+            t = e;
+            choice = form;
+            return true;
+        };
+        if (s.scores_block()) take(est_scores_block(s, w), p.scores, AP_BLOCK);
+        for (int pc = 1; s.scores_rows() && pc <= RB_PC; pc *= 2)
+            if (take(est_scores_rows(s, w, *rows, pc), p.scores, AP_ROWS)) p.pc = pc;
+        t = est_mix_token(s, w);
+        if (s.mix_block()) take(est_mix_block(s, w), p.mix, AP_BLOCK);
+        if (s.mix_rows()) take(est_mix_rows(s, w, *rows), p.mix, AP_ROWS);
+    }
+    // a wave a row only for rows of up to 2048 scores that fill the device:
+    // 1024 rows of 1000 scores take 9.9 us a wave each and 7.6 at 256 threads each,
+    // 2048 rows 11.4 and 12.2; rows past 4096 scores take 1024 threads
+    if (s.nmax() <= SM_WN / 2 && (long)s.ntok * s.n_heads > 1024) p.softmax = AP_SMX_WAVE;
     else if (s.nmax() <= 4096) p.softmax = AP_SMX_256;
     return p;
 }
@@ -981,7 +1112,7 @@ void launch_scores(const AttnShape &s, const AttnPlan &p, float *att, const floa
     // a workgroup for each token and tile of the positions it attends
     const int tt = attn_tile<KT>(group, s.hd);
     const size_t lds = attn_tile_lds<KT>(group, s.hd, tt);
-    const dim3 grid(s.n_kv, (s.max_pos + 1 + tt - 1) / tt, s.ntok);
+    const dim3 grid(s.n_kv, (s.nmax() + tt - 1) / tt, s.ntok);
     auto go = [&](auto kern, auto k) {
         hipLaunchKernelGGL(kern, grid, dim3(AT_THREADS), lds, kr_stream(), att, q, k, group, s.hd, kv_dim, s.max_seq,
                            s.window, scale, pos);
@@ -1080,6 +1211,16 @@ void kr_attn_prefill(int kt, float *ao, float *att, const float *q, const KvView
     if (kt == KV_F32) run(ic<KV_F32>{});
     else if (kt == KV_F16) run(ic<KV_F16>{});
     else run(ic<KV_Q8>{});
+}
+
+extern "C" int krh_attention_plan(int kv_type, int n_heads, int n_kv_heads, int head_dim, int max_seq, int window,
+                                  int ntok, int last_pos) {
+    const int kt = kv_type == ML_F32 ? KV_F32 : kv_type == ML_F16 ? KV_F16 : KV_Q8;
+    if (n_kv_heads <= 0 || n_heads <= 0 || n_heads % n_kv_heads || n_heads / n_kv_heads > 16 || head_dim <= 0 ||
+        head_dim % 4 || head_dim > 1024 || ntok <= 1 || last_pos < ntok - 1 || last_pos >= max_seq)
+        return -1;
+    const AttnPlan p = attn_plan({ kt, n_heads, n_kv_heads, head_dim, max_seq, window, ntok, last_pos });
+    return p.scores + 4 * p.softmax + 16 * p.mix;
 }
 
 extern "C" void krh_set_attn_rb_min(int min_wg) { g_rb_min_wg = min_wg < 0 ? 0 : min_wg; }

@@ -188,6 +188,7 @@ for name, res, args in [
     ("krh_attention_batch", None, [_P, _P, _P, _P, _P, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_float,
                                    _P, C.c_int, C.c_int]),
     ("krh_set_attn_rb_min", None, [C.c_int]),
+    ("krh_attention_plan", C.c_int, [C.c_int] * 8),
     ("krh_attention_short", C.c_int, [C.c_int, C.c_int]),
     ("krh_silu_quant", None, [_P, _P, C.c_int, _P, _P, C.c_int, C.c_int]),
     ("krh_embed_batch", None, [_P, C.POINTER(KrhMat), _P, C.c_int, C.c_float]),

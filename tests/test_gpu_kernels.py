@@ -659,10 +659,8 @@ def test_matmul_qkv_matches_decode(dev, dim, nh, nkv, hd, typ, vtyp, bias):
                                                      (32, 8, 64, 5, 100, 0), (8, 4, 64, 450, 62, 0)])
 @pytest.mark.parametrize("rb", [False, True])
 def test_attention_batch_matches_decode(dev, nh, nkv, hd, pos0, T, window, rb):
-    """rb: the register-blocked kernels forced on (64- and 128-dim heads; at
-    these sizes the launch would take the per-token-block kernels)"""
-    if rb and hd not in (64, 128):
-        pytest.skip("the register-blocked kernels take 64- and 128-dim heads")
+    """rb: the register-blocked kernels forced on (at these sizes the launch
+    would take others)"""
     with rb_forced(rb):
         attention_batch_case(dev, nh, nkv, hd, pos0, T, window)
 

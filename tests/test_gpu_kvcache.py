@@ -11,6 +11,7 @@ import pytest
 
 import krafla as K
 import oracle_lib as O
+from attn_sizes import BATCH_BLOCKS
 from oracle_lib import oracle
 from test_gpu_kernels import Dev, bits, f32, ok
 from test_gpu_model import SMALL
@@ -153,10 +154,8 @@ def test_attention_kv(dev, kv_type, nh, nkv, hd, pos, window):
 @pytest.mark.parametrize("rb", [False, True])
 def test_attention_kv_batch(dev, kv_type, nh, nkv, hd, pos0, T, window, rb):
     """batched attention over F16 and Q8 caches against the oracle's per-token
-    attention; rb: the register-blocked kernels forced on (64- and 128-dim
-    heads; at these sizes the launch would take the per-token-block kernels)"""
-    if rb and hd not in (64, 128):
-        pytest.skip("the register-blocked kernels take 64- and 128-dim heads")
+    attention; rb: the register-blocked kernels forced on (at these sizes the
+    launch would take others)"""
     if rb:
         K.hip.krh_set_attn_rb_min(0)
     try:
@@ -196,20 +195,19 @@ def kv_batch_case(dev, kv_type, nh, nkv, hd, pos0, T, window):
         assert np.array_equal(bits(got[t]), bits(out)), t
 
 
-# tile edges: windows around a 64-position tile, a first token with and
-# without a whole window behind it, one row and a ragged last row block, every
-# head size of the register-blocked kernels and one only the others take
+# every form (test_attention_plan.py) at its tiles' edges: windows around a
+# 64-position tile, a first token with and without a whole window behind it,
+# one row and a ragged last row block, every head size of the register-blocked
+# kernels and ones only the others take; cap: scores soft-capped between the two
 @pytest.mark.parametrize("kv_type", [K.ML_F32, K.ML_F16, K.ML_Q8_0])
-@pytest.mark.parametrize("nh,nkv,hd,pos0,T,window", [(4, 2, 48, 130, 67, 64), (3, 1, 64, 300, 65, 63),
-                                                     (8, 2, 80, 0, 70, 33), (4, 4, 96, 190, 33, 65),
-                                                     (6, 2, 128, 64, 2, 1), (4, 2, 256, 200, 37, 128),
-                                                     (2, 1, 256, 40, 90, 0), (6, 2, 96, 3, 80, 0),
-                                                     (4, 2, 32, 100, 50, 40), (8, 1, 64, 400, 112, 200)])
-@pytest.mark.parametrize("choice", [0, 1 << 30])
-def test_attention_batch_blocks(dev, kv_type, nh, nkv, hd, pos0, T, window, choice):
+@pytest.mark.parametrize("nh,nkv,hd,pos0,T,window", BATCH_BLOCKS)
+@pytest.mark.parametrize("choice", [0, 1 << 30, 512])
+@pytest.mark.parametrize("cap", [0.0, 1.5])
+def test_attention_batch_blocks(dev, kv_type, nh, nkv, hd, pos0, T, window, choice, cap):
     """batched attention with the register-blocked kernels for every grid
-    (choice 0) and for none, over a scratch and unattended cache rows of NaN
-    (Q8: scales), against the oracle's per-token attention"""
+    (choice 0), with the token blocks (1 << 30) and by estimate (512), over a
+    scratch and unattended cache rows of NaN (Q8: scales), against the oracle's
+    per-token attention"""
     max_seq = 512
     kvd, qd = nkv * hd, nh * hd
     Q = f32(RNG.normal(0, 1, (T, qd)))
@@ -234,14 +232,18 @@ def test_attention_batch_blocks(dev, kv_type, nh, nkv, hd, pos0, T, window, choi
     ao, att = dev.zeros(4 * T * qd), dev.put(np.full(T * nh * max_seq, np.nan, np.float32))
     K.hip.krh_set_attn_rb_min(choice)
     try:
-        K.hip.krh_attention_kv(ao.ptr, att.ptr, dev.put(Q).ptr, C.byref(dview), nh, nkv, hd, max_seq, scale,
-                               dev.put(np.array([pos0], np.int32)).ptr, T, pos0 + T - 1)
+        args = (ao.ptr, att.ptr, dev.put(Q).ptr, C.byref(dview), nh, nkv, hd, max_seq, scale,
+                dev.put(np.array([pos0], np.int32)).ptr, T, pos0 + T - 1)
+        if cap > 0:
+            K.hip.krh_attention_kv_softcap(*args, cap)
+        else:
+            K.hip.krh_attention_kv(*args)
         ok()
     finally:
         K.hip.krh_set_attn_rb_min(512)
     got = ao.get(np.float32, T * qd).reshape(T, qd)
     cfg = K.MlConfig(n_heads=nh, n_kv_heads=nkv, head_dim=hd, kv_dim=kvd, q_dim=qd, max_seq=max_seq,
-                     attn_scale=scale)
+                     attn_scale=scale, attn_softcap=cap)
     scratch = np.zeros(max_seq, np.float32)
     for t in range(T):
         out = np.zeros(qd, np.float32)
