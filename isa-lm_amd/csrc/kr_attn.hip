@@ -250,8 +250,11 @@ __global__ void __launch_bounds__(64 * (1 + MX_P)) k_attn_mix_kv(float *ao, cons
 // rows fit in LDS together (AS_LDS: 572 positions of 64 dims). The three
 // launches of a longer row spend most of such a token on their gaps, their
 // loads' latencies and the ordered sum's fixed cost: for 6 heads of 48 dims at
-// positions up to 136 they took 14.7 us a layer and two gaps, this launch 6.7;
-// for 14 heads of 64 dims at 530 positions 17.7 and the gaps against 14.4. K and V are
+// positions up to 136 they took 14.7 us a layer and two gaps, this launch 6.7.
+// It stays the faster up to the longest rows that fit (us a call, three
+// launches and this one, F32): 64 dims, 572 positions, 14 or 32 heads 14.4 and
+// 14.0; 48 dims, 710 positions 16.8 and 13.7; 128 dims, 292 positions, 32 heads
+// 13.3 and 12.0; 256 dims, 140 positions 14.6 and 11.3. K and V are
 // loaded together up front; V waits in registers while the scores run from
 // K's LDS copy, then its products with the weights take that copy's place.
 //   scores: a thread per position, its ordered dot from LDS;
@@ -326,17 +329,20 @@ __device__ __forceinline__ void attn_short(AsLds &S, float *ao, const float *q, 
         w[tid] = e;
     }
     __syncthreads();
-    if (tid < 64) {   // the ordered sum: every lane the same chain, 32 terms' reads ahead of their adds
+    if (tid < 64) {   // the ordered sum: every lane the same chain, 4 B terms' reads ahead of their adds
+        // B: half as many where 10 passes of floats wait in registers (with all 8
+        // the kernel spilled 27 of them)
+        constexpr int B = KT == KV_F32 && NP > 5 ? 4 : 8;
         float s = 0.0f;
         int t = 0;
-        float4 a[8], b[8];
-        auto read = [&](float4 (&v)[8], int t0) {
+        float4 a[B], b[B];
+        auto read = [&](float4 (&v)[B], int t0) {
 #pragma unroll
-            for (int k = 0; k < 8; k++) v[k] = *(const float4 *)(w + min(t0, AS_NT) + 4 * k);
+            for (int k = 0; k < B; k++) v[k] = *(const float4 *)(w + min(t0, AS_NT) + 4 * k);
         };
-        auto add = [&](const float4 (&v)[8]) {
+        auto add = [&](const float4 (&v)[B]) {
 #pragma unroll
-            for (int k = 0; k < 8; k++) {
+            for (int k = 0; k < B; k++) {
                 s = kr_fadd(s, v[k].x);
                 s = kr_fadd(s, v[k].y);
                 s = kr_fadd(s, v[k].z);
@@ -344,11 +350,11 @@ __device__ __forceinline__ void attn_short(AsLds &S, float *ao, const float *q, 
             }
         };
         read(a, 0);
-        for (; t + 64 <= n; t += 64) {
-            read(b, t + 32);
+        for (; t + 8 * B <= n; t += 8 * B) {
+            read(b, t + 4 * B);
             __builtin_amdgcn_sched_barrier(0);
             add(a);
-            read(a, t + 64);
+            read(a, t + 8 * B);
             __builtin_amdgcn_sched_barrier(0);
             add(b);
         }
