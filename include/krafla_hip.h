@@ -292,7 +292,10 @@ void krh_heads_norm_rope(float *q, float *k, const float *q_norm, const float *k
  * (the reference's projections write them in place, model/transformer.c:263-264) */
 void krh_store_rows_f32(float *kc, float *vc, const float *k, const float *v, int kv_dim, const int *pos);
 /* ops/ops.c:141: score rows (token t, head h) of att ([ntok][n_heads][max_seq])
- * become cap * tanhf(score / cap) over the positions attended from *pos + t */
+ * become cap * tanhf(score / cap), as many as position *pos + t attends, from the
+ * row's start: a windowed row holds its scores packed, the first attended
+ * position's at 0. (The attention calls soft-cap their own scratch, whose
+ * batched rows start at that position's index.) */
 void krh_softcap_att(float *att, int n_heads, int max_seq, int window, const int *pos, int ntok, float cap);
 /* krh_attention_kv with soft-capped scores (cap > 0, ops/ops.c:141): Gemma 2 */
 void krh_attention_kv_softcap(float *ao, float *att, const float *q, const ml_kv_layer *kv, int n_heads,

@@ -261,3 +261,21 @@ def ref_ml_run(model, tokens, steps, threads=1, dump=None, isa="scalar", timeout
         raise RuntimeError("ml_run failed (%d): %s" % (r.returncode, r.stderr))
     ids = np.array([int(v) for v in r.stdout.split()], dtype=np.int32)
     return ids, r.stderr
+
+
+def want_ml_run(model, tokens, steps, dump=None, extra=()):
+    """what ref_ml_run (ISA scalar) gives: the reference's own ml_run where its
+    build is there, else the oracle's C restatement, which test_oracle.py holds
+    to it bit for bit where both are"""
+    if os.path.exists(os.path.join(REF_DIR, "scalar", "ml_run")):
+        return ref_ml_run(model, tokens, steps, dump=dump, extra=extra)
+    extra = list(extra)
+    assert not extra or (len(extra) == 2 and extra[0] == "--kv"), extra
+    om = OracleModel(model, {"f16": K.ML_F16, "q8": K.ML_Q8_0, "f32": K.ML_F32}[extra[1] if extra else "f32"])
+    try:
+        if dump:
+            om.prefill(tokens, 0, logits=True).tofile(dump)
+            return None, ""
+        return om.generate(tokens, steps), ""
+    finally:
+        om.close()

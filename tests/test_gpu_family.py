@@ -1,7 +1,8 @@
 """The families' layer path on the device: q/k RMSNorm per head (Qwen3) and
 post-norms (Gemma 3), model/transformer.c:240-248. The heads' norm and RoPE
 kernel against the oracle's kernels; whole-model logits and greedy ids
-against the reference's ml_run, with each KV cache type."""
+against the reference's ml_run (without its build, the oracle), with each KV
+cache type."""
 import ctypes as C
 import os
 
@@ -143,6 +144,23 @@ def test_gelu_softcap_ops(n):
         b.free()
 
 
+@pytest.mark.parametrize("pos,ntok,window", [(0, 1, 0), (40, 3, 0), (300, 2, 17), (10, 4, 12)])
+def test_softcap_att(pos, ntok, window):
+    """krh_softcap_att: the attended scores of every row, packed at its start; the rest stay"""
+    nh, max_seq, cap = 3, 320, 2.5
+    a = np.random.default_rng(31).normal(0, 4, (ntok, nh, max_seq)).astype(np.float32)
+    att, posb = K.DevBuf.of(a), K.DevBuf.of(np.array([pos], np.int32))
+    K.hip.krh_softcap_att(att.ptr, nh, max_seq, window, posb.ptr, ntok, cap)
+    assert K.hip.krh_sync() == 0
+    for t in range(ntok):
+        n = min(pos + t + 1, window) if window else pos + t + 1
+        for h in range(nh):
+            oracle.kro_softcap_rows(a[t, h].ctypes.data, max_seq, 1, n, cap)
+    assert np.array_equal(bits(att.get(np.float32, a.size)), bits(a.reshape(-1)))
+    for b in (att, posb):
+        b.free()
+
+
 def test_store_rows_f32():
     n, rows, pos = 640, 9, 7
     k = np.arange(n, dtype=np.float32)
@@ -174,7 +192,7 @@ def test_family_model_matches_reference(name, kv, workdir):
     toks = [int(t) for t in np.random.default_rng(5).integers(1, V, 12)]
     dump = path + "." + kv + ".logits"
     print("family", name, kv, flush=True)
-    O.ref_ml_run(path, toks, len(toks), dump=dump, extra=("--kv", kv))
+    O.want_ml_run(path, toks, len(toks), dump=dump, extra=("--kv", kv))
     want = np.fromfile(dump, dtype=np.float32).reshape(len(toks), V)
     got = np.empty((len(toks), V), dtype=np.float32)
     s.prefill(toks, 0, logits=got)
@@ -182,7 +200,7 @@ def test_family_model_matches_reference(name, kv, workdir):
     s.close()
     s = K.State(m, KV[kv])
     steps = min(m.cfg.max_seq, 8 + 80)
-    want_ids, _ = O.ref_ml_run(path, toks[:8], steps, extra=("--kv", kv))
+    want_ids, _ = O.want_ml_run(path, toks[:8], steps, extra=("--kv", kv))
     got_ids, _, _ = s.generate(toks[:8], steps)
     assert np.array_equal(got_ids, want_ids)
     s.close()
@@ -207,7 +225,7 @@ def test_family_batched_prefill(name, kv, workdir):
     toks = [int(t) for t in np.random.default_rng(9).integers(1, V, n)]
     dump = path + "." + kv + ".long.logits"
     print("family batched", name, kv, n, flush=True)
-    O.ref_ml_run(path, toks, n, dump=dump, extra=("--kv", kv))
+    O.want_ml_run(path, toks, n, dump=dump, extra=("--kv", kv))
     want = np.fromfile(dump, dtype=np.float32).reshape(n, V)
     for batch in (0, 7, 1):
         s = K.State(m, KV[kv])

@@ -310,9 +310,16 @@ def test_matvec_float_input(dev, typ, d16, rows, cols):
                                                   # the softmax inside the mix launch (rows of at most 4096
                                                   # scores, groups of 1 to 4): at the limit, groups 1 and 2
                                                   (32, 8, 128, 4095, 0), (8, 8, 64, 1000, 0), (8, 4, 64, 3000, 0),
-                                                  (6, 3, 64, 4095, 100)])
-def test_attention(dev, nh, nkv, hd, pos, window):
+                                                  (6, 3, 64, 4095, 100), (8, 2, 64, 1500, 600)])
+@pytest.mark.parametrize("long_cache", [False, True])
+def test_attention(dev, nh, nkv, hd, pos, window, long_cache):
+    """long_cache: rows too long for the one-launch attention, so that short
+    positions run the three launches (a window within its limit still runs it)"""
     max_seq = max(256, pos + 1)
+    if long_cache:
+        if max_seq > K.hip.krh_attention_short(hd, K.ML_F32):
+            pytest.skip("three launches already")
+        max_seq = K.hip.krh_attention_short(hd, K.ML_F32) + pos + 8
     kvd, qd = nkv * hd, nh * hd
     q = f32(RNG.normal(0, 1, qd))
     kc = f32(RNG.normal(0, 1, max_seq * kvd))

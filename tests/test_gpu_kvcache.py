@@ -125,9 +125,17 @@ def views(dev, kv_type, k, v, kd, vd, window):
 @pytest.mark.parametrize("nh,nkv,hd,pos,window", [(6, 6, 48, 0, 0), (14, 2, 64, 511, 0), (32, 8, 128, 2175, 0),
                                                   (32, 8, 128, 2303, 0), (8, 2, 64, 100, 7), (16, 1, 64, 63, 0),
                                                   (12, 4, 96, 130, 0), (4, 2, 32, 9000, 0), (8, 4, 256, 300, 0),
-                                                  (4, 1, 256, 200, 64), (32, 8, 128, 4095, 0), (8, 8, 64, 1000, 0)])
-def test_attention_kv(dev, kv_type, nh, nkv, hd, pos, window):
+                                                  (4, 1, 256, 200, 64), (32, 8, 128, 4095, 0), (8, 8, 64, 1000, 0),
+                                                  (8, 2, 64, 1500, 600), (16, 1, 64, 700, 650)])
+@pytest.mark.parametrize("long_cache", [False, True])
+def test_attention_kv(dev, kv_type, nh, nkv, hd, pos, window, long_cache):
+    """long_cache: a last position too far for the one-launch attention, so
+    that short positions run the three launches over halves too"""
     max_seq = max(256, pos + 1)
+    if long_cache:
+        if max_seq > K.hip.krh_attention_short(hd, kv_type):
+            pytest.skip("three launches already")
+        max_seq = K.hip.krh_attention_short(hd, kv_type) + pos + 8
     kvd, qd = nkv * hd, nh * hd
     q = f32(RNG.normal(0, 1, qd))
     q[:hd] = 0.0   # a zero query head: Q8 scale 0
@@ -336,7 +344,7 @@ def test_logits_match_reference_kv(name, kv, batch, workdir):
     toks = [int(t) for t in np.random.default_rng(6).integers(1, V, 12)]
     dump = path + "." + kv + ".logits"
     if not os.path.exists(dump):
-        O.ref_ml_run(path, toks, len(toks), dump=dump, extra=("--kv", kv))
+        O.want_ml_run(path, toks, len(toks), dump=dump, extra=("--kv", kv))
     want = np.fromfile(dump, dtype=np.float32).reshape(len(toks), V)
     got = np.empty((len(toks), V), dtype=np.float32)
     s.prefill(toks, 0, logits=got)
@@ -355,7 +363,7 @@ def test_greedy_ids_match_reference_kv(name, kv, workdir):
     s = K.State(m, KV[kv])
     toks = [int(t) for t in np.random.default_rng(6).integers(1, m.cfg.vocab, 5)]
     steps = min(m.cfg.max_seq, 60)
-    ids_ref, _ = O.ref_ml_run(path, toks, steps, extra=("--kv", kv))
+    ids_ref, _ = O.want_ml_run(path, toks, steps, extra=("--kv", kv))
     ids, _, _ = s.generate(toks, steps)
     assert np.array_equal(ids, ids_ref)
     s.close()

@@ -41,7 +41,7 @@ def test_logits_match_reference(name, workdir):
     V = m.cfg.vocab
     toks = [int(t) for t in np.random.default_rng(5).integers(1, V, 12)]
     dump = path + ".logits"
-    O.ref_ml_run(path, toks, len(toks), dump=dump)
+    O.want_ml_run(path, toks, len(toks), dump=dump)
     want = np.fromfile(dump, dtype=np.float32).reshape(len(toks), V)
     got = np.empty((len(toks), V), dtype=np.float32)
     s.prefill(toks, 0, logits=got)
@@ -64,7 +64,7 @@ def test_prefill_paths_match_reference(name, batch, workdir):
     V = m.cfg.vocab
     toks = [int(t) for t in np.random.default_rng(5).integers(1, V, 12)]
     dump = path + ".logits"
-    O.ref_ml_run(path, toks, len(toks), dump=dump)
+    O.want_ml_run(path, toks, len(toks), dump=dump)
     want = np.fromfile(dump, dtype=np.float32).reshape(len(toks), V)
     got = np.empty((len(toks), V), dtype=np.float32)
     s.prefill(toks, 0, logits=got)
@@ -82,7 +82,7 @@ def test_greedy_ids_match_reference(name, workdir):
     s = K.State(m)
     prompt = [int(t) for t in np.random.default_rng(6).integers(1, m.cfg.vocab, 8)]
     steps = min(m.cfg.max_seq, 8 + 128)
-    want, _ = O.ref_ml_run(path, prompt, steps)
+    want, _ = O.want_ml_run(path, prompt, steps)
     got, _, _ = s.generate(prompt, steps)
     assert np.array_equal(got, want)
     s.close()
@@ -96,7 +96,7 @@ def test_stories15m_shape_128_greedy(workdir):
     m = K.Model(path)
     s = K.State(m)
     prompt = [int(t) for t in np.random.default_rng(1).integers(1, 32000, 8)]
-    want, _ = O.ref_ml_run(path, prompt, 135)
+    want, _ = O.want_ml_run(path, prompt, 135)
     got, _, _ = s.generate(prompt, 135)
     assert len(got) == 135 and np.array_equal(got, want)
     # decoding again from a fresh prefill gives the same ids (state reuse)

@@ -1,14 +1,15 @@
 """krh_attention_noalloc, the decode attention that allocates nothing (its
 score rows live in a static device array), against krh_attention with a
-caller-allocated workspace: bit for bit, on two calls in a row (the second
-smaller, over the array's stale contents), and the size limit. Needs a
-gfx950 device."""
+caller-allocated workspace and the oracle: bit for bit, on calls in a row (the
+later ones smaller, over the array's stale contents), and the size limit. Needs
+a gfx950 device."""
 import ctypes as C
 
 import numpy as np
 import pytest
 
 import krafla as K
+import oracle_lib as O
 
 pytestmark = pytest.mark.gpu
 RNG = np.random.default_rng(7)
@@ -27,11 +28,11 @@ def bits(a):
 
 
 def both(nh, nkv, hd, max_seq, pos, window):
-    """ao of krh_attention_noalloc and of krh_attention on the same inputs"""
+    """ao of krh_attention_noalloc, of krh_attention and of the oracle on the same inputs"""
     kvd, qd = nkv * hd, nh * hd
-    q = K.DevBuf.of(RNG.normal(0, 1, qd).astype(np.float32))
-    kc = K.DevBuf.of(RNG.normal(0, 1, max_seq * kvd).astype(np.float32))
-    vc = K.DevBuf.of(RNG.normal(0, 1, max_seq * kvd).astype(np.float32))
+    qh = RNG.normal(0, 1, qd).astype(np.float32)
+    kh, vh = (RNG.normal(0, 1, max_seq * kvd).astype(np.float32) for _ in range(2))
+    q, kc, vc = K.DevBuf.of(qh), K.DevBuf.of(kh), K.DevBuf.of(vh)
     posb = K.DevBuf.of(np.array([pos], np.int32))
     scale = C.c_float(float(np.float32(1.0) / np.sqrt(np.float32(hd))))
     ao_n, ao_w, att = K.DevBuf(4 * qd), K.DevBuf(4 * qd), K.DevBuf(4 * nh * max_seq)
@@ -40,18 +41,28 @@ def both(nh, nkv, hd, max_seq, pos, window):
                         posb.ptr)
     st = K.hip.krh_sync()
     assert st == 0, K.hip.krh_last_error().decode()
-    out = ao_n.get(np.float32, qd), ao_w.get(np.float32, qd)
+    cfg = K.MlConfig(n_heads=nh, n_kv_heads=nkv, head_dim=hd, kv_dim=kvd, q_dim=qd, max_seq=max_seq,
+                     attn_scale=scale.value)
+    kvl = O.KvLayer(kh.ctypes.data, vh.ctypes.data, None, None, None, None, window, None, None)
+    ref, scratch = np.zeros(qd, np.float32), np.zeros(max_seq, np.float32)
+    O.oracle.kro_attention(ref.ctypes.data, qh.ctypes.data, C.byref(kvl), scratch.ctypes.data, C.byref(cfg), pos)
+    out = ao_n.get(np.float32, qd), ao_w.get(np.float32, qd), ref
     for b in (q, kc, vc, posb, ao_n, ao_w, att):
         b.free()
     return out
 
 
 def test_noalloc_matches_workspace_entry_twice():
-    # the 8B shape at a long position, then a smaller call (fewer heads, a
-    # shorter cache and a window) over what the first left in the array
-    for nh, nkv, hd, max_seq, pos, window in [(32, 8, 128, 4096, 3000, 0), (14, 2, 64, 1024, 500, 100)]:
-        got, want = both(nh, nkv, hd, max_seq, pos, window)
+    # the 8B shape at a long position, then smaller calls (fewer heads, a shorter
+    # cache) over what the first left in the array: three launches, which write
+    # and read score rows there, without and with a window, and one that does not
+    for nh, nkv, hd, max_seq, pos, window in [(32, 8, 128, 4096, 3000, 0), (14, 2, 64, 1024, 500, 0),
+                                              (14, 2, 64, 1024, 900, 600), (14, 2, 64, 1024, 500, 100)]:
+        rows = window if window and pos >= window else max_seq
+        assert (rows <= K.hip.krh_attention_short(hd, K.ML_F32)) == (window == 100)
+        got, want, oracle = both(nh, nkv, hd, max_seq, pos, window)
         assert np.array_equal(bits(got), bits(want)), (nh, max_seq, pos)
+        assert np.array_equal(bits(got), bits(oracle)), (nh, max_seq, pos)
 
 
 def test_noalloc_rejects_beyond_the_array():
