@@ -274,8 +274,9 @@ def prefill_roofline(K, model, ntok, prefill_s, reps=2):
     quantized activation batch; int8 ops = 2 * rows * cols * ntok per launch,
     against the 5.0 POP/s dense int8 peak and against the exact-order VALU
     bound (3 VALU operations -- fma, mul, add -- per output and 32-block of
-    f16-scaled weights, at 64 lanes x CUs x 2.4 GHz); plus the whole prefill's int8 ops
-    over its wall time (attention, norms and launches included)"""
+    f16-scaled weights, 4 -- cvt, mul, mul, add -- of f32-scaled ones, at 64 lanes
+    x CUs x 2.4 GHz); plus the whole prefill's int8 ops over its wall time
+    (attention, norms and launches included)"""
     cfg = model.cfg
     T = ntok
     ldx = (T + 127) // 128 * 128
@@ -303,7 +304,8 @@ def prefill_roofline(K, model, ntok, prefill_s, reps=2):
     mfma = mfma_int8_rate(K)
     ops = 2.0 * rows * cols * T
     tops = ops / (us * 1e-6) / 1e12
-    valu_tops = 64 * K.hip.krh_device_cus() * 2.4e9 * (2 * 32 / 3) / 1e12   # int8 ops per exact-order VALU lane-op: 64 / 3
+    valu_ops = 3 if w1[0].contents.d16 else 4
+    valu_tops = 64 * K.hip.krh_device_cus() * 2.4e9 * (2 * 32 / valu_ops) / 1e12   # 64 int8 ops an output and block
     layer_ops = 0
     for l in range(cfg.n_layers):
         for wn in (b"wq", b"wk", b"wv", b"wo", b"w1", b"w2", b"w3"):
