@@ -472,7 +472,11 @@ __global__ void __launch_bounds__(64) k_store_kv(const KvOut o, const float *k, 
 }
 
 // The decode kernels first and together in the code object: a token's three
-// attention launches then run from one stretch of it.
+// attention launches then run from one stretch of it. (A token's launches hold
+// more code than the instruction cache, and where a process's objects and
+// buffers lie moves the 8B shape's attention block between 41.0 and 41.9 us
+// with the same binary: orders that measured better on one run did not on the
+// next.)
 template __global__ void k_attn_scores<AT_TD, false>(float *, const float *, const float *, int, int, int, int, int, float,
                                                      const int *);
 template __global__ void k_attn_softmax<SMX_THREADS, AT_CHUNK, false, false>(float *, int, int, const int *);

@@ -525,9 +525,10 @@ __device__ __forceinline__ float kr_spec_sum(float *t, int n, unsigned char *lds
 
 // The ordered sum by the workgroup's first wave alone, as kr_spec_sum
 // otherwise: the same terms, calling rules and bits (+0 start). Kernels take
-// it for n <= SC_SHORT. The line: 288 terms (a 15M model's norms) one by one
-// take the FFN of a token from 10.8 to 9.45 us; 896 terms (the 0.5B shape's)
-// were slower that way (its prompt and 32 decoded tokens 41.2 ms against 40.7).
+// it for n <= SC_SHORT. The line: one by one, the FFN of a token over 288 terms
+// (a 15M model's norms) takes 9.3 us against 10.7, over 480 10.3 and 11.2, 640
+// 10.7 and 11.2; 896 terms (the 0.5B shape's) were slower that way (its prompt
+// and 32 decoded tokens 41.2 ms against 40.7).
 constexpr int SC_SHORT = 640;
 __device__ __forceinline__ float kr_short_sum(const float *t, int n, unsigned char *lds) {
     float *res = (float *)lds;
