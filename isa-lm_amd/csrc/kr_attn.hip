@@ -471,12 +471,17 @@ __global__ void __launch_bounds__(64) k_store_kv(const KvOut o, const float *k, 
     if (lane == 0) (which ? o.vd : o.kd)[(size_t)(*pos0 + t) * o.n_kv + h] = zero ? 0.0f : kr_fdiv(m, 127.0f);
 }
 
-// The decode kernels first and together in the code object: a token's three
-// attention launches then run from one stretch of it. (A token's launches hold
-// more code than the instruction cache, and where a process's objects and
-// buffers lie moves the 8B shape's attention block between 41.0 and 41.9 us
-// with the same binary: orders that measured better on one run did not on the
-// next.)
+// The one-launch kernels, then a token's three launches, first and together in
+// the code object. A token's launches hold more code than the instruction cache, so
+// where this code and a process's buffers lie moves the 8B shape's attention
+// block by up to 0.9 us: over the performance cases in one process this order
+// took 41.1 us (the block's projections in another object, 47.6 the 1B shape's
+// Q8 block), the three launches first 42.0 (47.9); alone in a process 41.0 to
+// 41.4 and 41.4 to 41.9.
+template __global__ void k_attn_short<KV_F32>(float *, const float *, const KvView, int, int, int, int, float, const int *,
+                                              int);
+template __global__ void k_attn_short<KV_F16>(float *, const float *, const KvView, int, int, int, int, float, const int *,
+                                              int);
 template __global__ void k_attn_scores<AT_TD, false>(float *, const float *, const float *, int, int, int, int, int, float,
                                                      const int *);
 template __global__ void k_attn_softmax<SMX_THREADS, AT_CHUNK, false, false>(float *, int, int, const int *);
