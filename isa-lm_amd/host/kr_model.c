@@ -623,7 +623,7 @@ static ml_status batch_buffers(kr_state *s, int with_logits) {
 /* whether a prompt step of T tokens takes the FFN as one launch
  * (krh_matmul_swiglu: 64-row tiles of w1 and w3 together): from 3/4 of a
  * tile per compute unit, where the single launch fills the device; shorter
- * steps keep the separate products, whose 32-row tiles do. */
+ * steps keep the separate products, which take smaller tiles. */
 static int swiglu_fused(const kr_state *s, const struct kr_dev_layer *D, int T) {
     const ml_config *c = &s->m->cfg;
     if (D->w1.type != D->w3.type || D->w1.d16 != D->w3.d16 || c->hidden_dim % 32) return 0;
